@@ -94,6 +94,7 @@ hipError_t launch_tick(const TickShape &sh, const u8 *src, u8 *dst, int nx, int 
 hipError_t launch_tick_chunked(int seg, const u8 *src, u8 *dst, int nx, int ny, int nz, u64 t, const u64 *tick_dev,
                                u32 k_off, const u64 *rule, u64 *hash_parts, hipStream_t s);
 hipError_t launch_fill_u64(u64 *p, size_t n, u64 v, hipStream_t s);
+hipError_t launch_fill_u32(u32 *p, size_t n, u32 v, hipStream_t s);
 // Work-list entry of the listed skipping tick: active lanes of one row quad and
 // its position (zq << 32 | yq).  On odd ticks of the packed schedule, edge bit s
 // is set unless the block straddling x = s * seg is known not to change: it did
@@ -202,7 +203,15 @@ struct fs3d_world {
   fs3d::u32 *d_ctl = nullptr;         // list counts, one per tick mod 3
   fs3d::u32 list_waves = 0;           // persistent waves of the listed tick
   fs3d::u32 pack_waves = 0;           // persistent waves of the packed tick
-  // cached graphs keyed by (nticks, hash_every, cur)
+  // the grid as bit planes (two buffers, allocated on first use): planes[pcur]
+  // holds the current state while planes_valid; buf[cur] always does between calls
+  void *planes[2] = {nullptr, nullptr};
+  int pcur = 0;
+  bool planes_valid = false, planes_off = false;
+  fs3d::u32 *d_reserved = nullptr;  // a byte >= 4 has been packed or set
+  bool masks_stale = false;         // plane ticks have run since the change masks were last exact
+  bool fuse_set = false;            // set_fuse has been called
+  // cached graphs keyed by (nticks, hash_every, buffers and path)
   std::map<std::tuple<int, int, int>, hipGraphExec_t> graphs;
 };
 

@@ -705,6 +705,11 @@ __global__ __launch_bounds__(256) void fill_u64_kernel(u64 *p, size_t n, u64 v) 
     p[i] = v;
 }
 
+__global__ __launch_bounds__(256) void fill_u32_kernel(u32 *p, size_t n, u32 v) {
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
+    p[i] = v;
+}
+
 __global__ void mark_cells_kernel(u64 *m0, u64 *m1, long long i0, long long i1, u64 bits, size_t edge_off) {
   if (threadIdx.x == 0) {
     m0[i0] |= bits;
@@ -927,6 +932,12 @@ hipError_t launch_fill_u64(u64 *p, size_t n, u64 v, hipStream_t s) {
   if (blocks > 4096) blocks = 4096;
   if (blocks == 0) blocks = 1;
   hipLaunchKernelGGL(fill_u64_kernel, dim3((unsigned)blocks), dim3(256), 0, s, p, n, v);
+  return hipGetLastError();
+}
+
+hipError_t launch_fill_u32(u32 *p, size_t n, u32 v, hipStream_t s) {
+  const size_t blocks = std::min<size_t>(std::max<size_t>((n + 255) / 256, 1), 4096);
+  hipLaunchKernelGGL(fill_u32_kernel, dim3((unsigned)blocks), dim3(256), 0, s, p, n, v);
   return hipGetLastError();
 }
 
