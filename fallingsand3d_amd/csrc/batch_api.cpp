@@ -21,10 +21,14 @@ struct fs3d_batch {
   std::vector<size_t> off, cells;
   std::vector<TickShape> plain_shape;  // single-world launch shape per world (plain loop)
   u8 *arena = nullptr;
-  size_t arena_bytes = 0;
+  size_t arena_bytes = 0;  // of the grids
+  void *planes = nullptr;  // plane scratch of the worlds too large for LDS, behind them
   BWorld *d_worlds = nullptr;
-  int *d_order = nullptr;
+  int *d_order = nullptr;                  // world indices by plane words, largest first
+  std::vector<u32> sorted_words;           // their plane words
   u32 *d_queue = nullptr;
+  std::vector<size_t> poff;                // word offsets of the plane scratch, behind the grids in the arena
+  bool planes_off = false;                 // no plane scratch: persistent runs take the wide kernel
   u64 *d_hashes = nullptr;
   long long *d_prefix = nullptr;  // wide mode: workgroup prefix per parity, 2 x (n + 1)
   int *d_blk2ent[2] = {nullptr, nullptr};  // wide mode: workgroup -> world, per parity
@@ -38,8 +42,8 @@ struct fs3d_batch {
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   double last_ms = 0.0;
-  // (mode, nticks, hash, tick parity, seg, threads, groups)
-  std::map<std::tuple<int, int, int, int, int, int, int>, hipGraphExec_t> graphs;
+  // (mode, nticks, hash, tick parity, seg, threads)
+  std::map<std::tuple<int, int, int, int, int, int>, hipGraphExec_t> graphs;
 };
 
 namespace {
@@ -71,6 +75,7 @@ int sync_table(fs3d_batch *b, int nt = 0) {
     w.nt = nt;
     w.slot = i;
     w.fin = 1;  // a batch run's last tick is the one hashed
+    w.poff = b->poff[i];
     w.tick = b->tick;
   }
   FS3D_HIP(hipMemcpyAsync(b->d_worlds, b->h_worlds.data(), sizeof(BWorld) * b->n, hipMemcpyHostToDevice, b->stream));
@@ -98,6 +103,10 @@ int sync_table(fs3d_batch *b, int nt = 0) {
   return FS3D_OK;
 }
 
+u32 plane_words_of(const fs3d_batch *b, int i) {
+  return (u32)((b->nx[i] + 63) / 64) * (u32)b->ny[i] * (u32)b->nz[i];
+}
+
 int apply_config(fs3d_batch *b, int seg, int threads, int groups) {
   if (!batch_config_ok(seg, threads, groups))
     return set_error(FS3D_ERR_INVALID, "batch config (seg %d, threads %d, groups %d) unsupported", seg, threads,
@@ -106,7 +115,7 @@ int apply_config(fs3d_batch *b, int seg, int threads, int groups) {
     return set_error(FS3D_ERR_INVALID, "segment %d too narrow for nx=%d", seg, max_nx(b));
   hipDeviceProp_t prop;
   FS3D_HIP(hipGetDeviceProperties(&prop, b->dev));
-  const int occ = batch_occupancy(seg, threads, groups);
+  const int occ = batch_occupancy(threads);
   b->seg = seg;
   b->threads = threads;
   b->groups = groups;
@@ -135,13 +144,18 @@ void release(fs3d_batch *b) {
 
 int run_persistent(fs3d_batch *b, int nticks, int want_hash) {
   const int flags = (want_hash ? kBatchHash : 0) | (b->settle ? kBatchSettle : 0);
-  const auto key = std::make_tuple((int)FS3D_BATCH_PERSISTENT, nticks, flags, 0, b->seg, b->threads, b->groups);
+  const auto key = std::make_tuple((int)FS3D_BATCH_PERSISTENT, nticks, flags, 0, 0, b->threads);
   auto it = b->graphs.find(key);
   if (it == b->graphs.end()) {
     hipGraph_t graph = nullptr;
+    // worlds of fewer words than a wave's share of the LDS go to waves
+    const u32 wave_words = batch_wave_words(batch_lds_words(b->threads), b->threads / 64);
+    const int n_wide = (int)(std::partition_point(b->sorted_words.begin(), b->sorted_words.end(),
+                                                  [&](u32 w) { return w >= wave_words; }) -
+                             b->sorted_words.begin());
     FS3D_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-    hipError_t e = launch_batch(b->seg, b->threads, b->groups, b->d_worlds, b->d_order, b->n, nticks, b->d_queue,
-                                device_rule_table(b->dev), b->d_hashes, flags, b->grid, b->stream);
+    hipError_t e = launch_batch(b->threads, b->d_worlds, b->d_order, n_wide, b->n, nticks, b->d_queue,
+                                b->planes, b->d_hashes, flags, b->grid, b->stream);
     hipError_t e2 = hipStreamEndCapture(b->stream, &graph);
     if (e != hipSuccess || e2 != hipSuccess) {
       if (graph) (void)hipGraphDestroy(graph);
@@ -165,7 +179,7 @@ int run_wide(fs3d_batch *b, int nticks, int want_hash) {
   if (b->table_nt != nticks)
     if (int rc = sync_table(b, nticks)) return rc;
   const int par = (int)(b->tick & 1u);
-  const auto key = std::make_tuple((int)FS3D_BATCH_WIDE, nticks, want_hash, par, b->seg, 0, 0);
+  const auto key = std::make_tuple((int)FS3D_BATCH_WIDE, nticks, want_hash, par, b->seg, 0);
   auto it = b->graphs.find(key);
   if (it == b->graphs.end()) {
     hipGraph_t graph = nullptr;
@@ -246,7 +260,25 @@ int fs3d_batch_create(int32_t n, const int32_t *dims, fs3d_batch **out) {
   b->arena_bytes = total;
   b->h_worlds.resize(n);
   hipError_t e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
-  if (e == hipSuccess) e = hipMalloc(&b->arena, total);
+  // Plane scratch for the worlds whose planes exceed the smallest workgroup's LDS
+  // share.  Without room for it (or with a world of 4 GiB of planes) persistent
+  // runs take the wide kernel, which needs none.
+  size_t scratch = 0;
+  for (int i = 0; i < n; i++) {
+    const size_t words = (size_t)((b->nx[i] + 63) / 64) * (size_t)b->ny[i] * (size_t)b->nz[i];
+    b->planes_off = b->planes_off || words >= (1ull << 28);
+    b->poff.push_back(scratch);
+    if (words > batch_lds_words(256)) scratch += (words + 15) & ~(size_t)15;
+  }
+  if (e == hipSuccess && !b->planes_off) {
+    if (hipMalloc(&b->arena, total + scratch * 16) == hipSuccess) {
+      b->planes = b->arena + total;
+    } else {
+      (void)hipGetLastError();
+      b->planes_off = true;
+    }
+  }
+  if (e == hipSuccess && b->planes_off) e = hipMalloc(&b->arena, total);
   if (e == hipSuccess) e = hipMalloc(&b->d_worlds, sizeof(BWorld) * n);
   if (e == hipSuccess) e = hipMalloc(&b->d_order, sizeof(int) * n);
   if (e == hipSuccess) e = hipMalloc(&b->d_queue, 256);
@@ -265,7 +297,9 @@ int fs3d_batch_create(int32_t n, const int32_t *dims, fs3d_batch **out) {
   // largest worlds first: they start early and the short ones fill the tail
   std::vector<int> order(n);
   std::iota(order.begin(), order.end(), 0);
-  std::stable_sort(order.begin(), order.end(), [&](int a, int c) { return b->cells[a] > b->cells[c]; });
+  std::stable_sort(order.begin(), order.end(),
+                   [&](int a, int c) { return plane_words_of(b, a) > plane_words_of(b, c); });
+  for (int i : order) b->sorted_words.push_back(plane_words_of(b, i));
   e = hipMemcpyAsync(b->d_order, order.data(), sizeof(int) * n, hipMemcpyHostToDevice, b->stream);
   if (e != hipSuccess) {
     release(b);
@@ -395,6 +429,7 @@ int fs3d_batch_run(fs3d_batch *b, int32_t nticks, int32_t mode, uint64_t *hashes
     b->last_ms = 0.0;
     return clear_error();
   }
+  if (mode == FS3D_BATCH_PERSISTENT && b->planes_off) mode = FS3D_BATCH_WIDE;
   int rc = mode == FS3D_BATCH_PERSISTENT ? run_persistent(b, nticks, want_hash)
            : mode == FS3D_BATCH_WIDE     ? run_wide(b, nticks, want_hash)
                                          : run_plain(b, nticks, want_hash);
@@ -421,8 +456,9 @@ int fs3d_batch_last_run_ms(const fs3d_batch *b, double *ms) {
   return clear_error();
 }
 
-// Times every supported persistent-kernel shape on a scratch copy of the arena
-// (the batch's own state is not advanced) and keeps the fastest.
+// Times the persistent kernel's workgroup sizes and the wide mode's segments on a
+// scratch copy of the arena (the batch's own state is not advanced) and keeps the
+// fastest.
 int fs3d_batch_autotune(fs3d_batch *b, int32_t trial_ticks, int32_t *seg_out, int32_t *threads_out,
                         int32_t *groups_out, int32_t *mode_out, double *best_ms) {
   if (int rc = check_batch(b)) return rc;
@@ -436,35 +472,38 @@ int fs3d_batch_autotune(fs3d_batch *b, int32_t trial_ticks, int32_t *seg_out, in
   double best = 1e30;
   int bseg = seg0, bthr = thr0, bgrp = grp0, bmode = FS3D_BATCH_PERSISTENT;
   int rc = FS3D_OK;
-  const int segs[3] = {8, 16, 32}, thrs[3] = {256, 512, 1024}, grps[3] = {1, 2, 4};
-  // trial index 27 + si: the wide mode at segment segs[si]
-  for (int si = 0; si < 3 && !rc; si++)
-    for (int ti = 0; ti < 4 && !rc; ti++)
-      for (int gi = 0; gi < 3 && !rc; gi++) {
-        const bool wide = ti == 3;
-        if (wide && gi > 0) continue;
-        if (!wide && !batch_config_ok(segs[si], thrs[ti], grps[gi])) continue;
-        if ((max_nx(b) + segs[si] - 1) / segs[si] > 64) continue;
-        hipError_t e = hipMemcpyAsync(scratch, real, b->arena_bytes, hipMemcpyDeviceToDevice, b->stream);
-        if (e != hipSuccess) {
-          rc = set_error(FS3D_ERR_HIP, "autotune copy failed: %s", hipGetErrorString(e));
-          break;
-        }
-        b->arena = scratch;
-        rc = wide ? apply_config(b, segs[si], 256, 1) : apply_config(b, segs[si], thrs[ti], grps[gi]);
-        if (!rc) rc = wide ? run_wide(b, trial_ticks, 0) : run_persistent(b, trial_ticks, 0);
-        if (!rc && hipStreamSynchronize(b->stream) != hipSuccess) rc = set_error(FS3D_ERR_HIP, "autotune sync failed");
-        float ms = 0.f;
-        if (!rc) (void)hipEventElapsedTime(&ms, b->ev0, b->ev1);
-        b->arena = real;
-        if (!rc && ms < best) {
-          best = ms;
-          bseg = segs[si];
-          bthr = wide ? 256 : thrs[ti];  // persistent shape unused by the wide mode
-          bgrp = wide ? 1 : grps[gi];
-          bmode = wide ? FS3D_BATCH_WIDE : FS3D_BATCH_PERSISTENT;
-        }
-      }
+  struct Trial {
+    int seg, threads, mode;
+  };
+  const int pseg = max_nx(b) <= 512 ? 8 : (max_nx(b) <= 1024 ? 16 : 32);  // persistent runs do not depend on it
+  std::vector<Trial> trials;
+  for (int thr : {256, 512, 1024})
+    if (!b->planes_off && batch_config_ok(pseg, thr, 1)) trials.push_back({pseg, thr, FS3D_BATCH_PERSISTENT});
+  for (int seg : {8, 16, 32})
+    if ((max_nx(b) + seg - 1) / seg <= 64) trials.push_back({seg, 256, FS3D_BATCH_WIDE});
+  for (const Trial &t : trials) {
+    if (rc) break;
+    const bool wide = t.mode == FS3D_BATCH_WIDE;
+    hipError_t e = hipMemcpyAsync(scratch, real, b->arena_bytes, hipMemcpyDeviceToDevice, b->stream);
+    if (e != hipSuccess) {
+      rc = set_error(FS3D_ERR_HIP, "autotune copy failed: %s", hipGetErrorString(e));
+      break;
+    }
+    b->arena = scratch;
+    rc = apply_config(b, t.seg, t.threads, 1);
+    if (!rc) rc = wide ? run_wide(b, trial_ticks, 0) : run_persistent(b, trial_ticks, 0);
+    if (!rc && hipStreamSynchronize(b->stream) != hipSuccess) rc = set_error(FS3D_ERR_HIP, "autotune sync failed");
+    float ms = 0.f;
+    if (!rc) (void)hipEventElapsedTime(&ms, b->ev0, b->ev1);
+    b->arena = real;
+    if (!rc && ms < best) {
+      best = ms;
+      bseg = t.seg;
+      bthr = t.threads;  // workgroup size unused by the wide mode
+      bgrp = 1;
+      bmode = t.mode;
+    }
+  }
   b->arena = real;
   drop_graphs(b);
   (void)hipStreamSynchronize(b->stream);

@@ -14,6 +14,7 @@ struct BWorld {
   int slot;      // wide launches: index of the entry's hash slot
   int fin;       // wide launches: 1 when the round's last tick is the entry's final one (hash it)
   u64 tick;      // tick counter before the next run (round)
+  u64 poff;      // batches: word offset of the world's planes in the plane scratch
 };
 
 // The grid of a world-table entry as a global-memory pointer.  A pointer read
@@ -25,13 +26,20 @@ __device__ __forceinline__ u8 *grid_of(const BWorld &w) {
 }
 
 bool batch_config_ok(int seg, int threads, int groups);
-int batch_occupancy(int seg, int threads, int groups);
-// flags of the persistent batch launch: hash every world's final tick; stop
+// Workgroups of the persistent kernel that share a CU, the plane words one of
+// them holds in LDS, and each of its nw waves for the worlds that waves take.
+int batch_occupancy(int threads);
+u32 batch_lds_words(int threads);
+__host__ __device__ inline u32 batch_wave_words(u32 lds_words, int nw) { return (lds_words + 1u) / (u32)nw; }
+// flags of the persistent batch launch: hash every world's final state; stop
 // ticking a world after two ticks in which nothing changed (its state is then a
-// fixed point of both parities) and run only its final tick.
+// fixed point of both parities).
 constexpr int kBatchHash = 1, kBatchSettle = 2;
-hipError_t launch_batch(int seg, int threads, int groups, BWorld *worlds, const int *order, int n, int nticks,
-                        u32 *queue, const u64 *rule, u64 *hashes, int flags, int grid, hipStream_t s);
+// order: world indices by plane words, largest first, the first n_wide for
+// workgroups and the rest (at most batch_wave_words - 1 words each) for waves;
+// planes: plane scratch of the worlds over batch_lds_words.
+hipError_t launch_batch(int threads, BWorld *worlds, const int *order, int n_wide, int n, int nticks, u32 *queue,
+                        void *planes, u64 *hashes, int flags, int grid, hipStream_t s);
 hipError_t launch_batch_hash(const BWorld *worlds, int n, u64 *hashes, hipStream_t s);
 hipError_t launch_batch_fill_rain(const BWorld *worlds, int n, const u64 *seeds, const u64 *thr, size_t max_cells,
                                   hipStream_t s);

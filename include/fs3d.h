@@ -198,10 +198,11 @@ int fs3d_batch_download(fs3d_batch *b, int32_t i, uint8_t *host, size_t nbytes);
 int fs3d_batch_fill_rain(fs3d_batch *b, const uint64_t *seeds, const uint64_t *thr);
 int fs3d_batch_get_tick(const fs3d_batch *b, uint64_t *tick);
 int fs3d_batch_set_tick(fs3d_batch *b, uint64_t tick);
-/* Persistent-kernel shape: bytes per lane (8 or 16; 32 with 256 threads and 1
- * group), workgroup size (256, 512, 1024) and row-quad groups each wave loads
- * before updating (1, 2, 4: memory-level parallelism).  *grid receives the
- * number of resident workgroups. */
+/* Launch shape: workgroup size of the persistent kernel (256, 512 or 1024: the
+ * larger, the more LDS a world may take) and bytes per lane of the wide one (8 or
+ * 16; 32 with 256 threads and 1 group).  groups (1, 2, 4) is checked and kept,
+ * and has no effect on either kernel.  *grid receives the number of resident
+ * workgroups. */
 int fs3d_batch_set_config(fs3d_batch *b, int32_t seg, int32_t threads, int32_t groups);
 int fs3d_batch_get_config(const fs3d_batch *b, int32_t *seg, int32_t *threads, int32_t *groups, int32_t *grid);
 /* Settled worlds (on by default): in FS3D_BATCH_PERSISTENT runs a world in which
@@ -215,8 +216,8 @@ int fs3d_batch_get_skip(const fs3d_batch *b, int32_t *on);
 int fs3d_batch_run(fs3d_batch *b, int32_t nticks, int32_t mode, uint64_t *hashes);
 /* Device time (ms, HIP events) of the last fs3d_batch_run. */
 int fs3d_batch_last_run_ms(const fs3d_batch *b, double *ms);
-/* Times every persistent-kernel shape and the wide mode at each segment width
- * on a scratch copy of the arena for trial_ticks ticks (the batch itself does
+/* Times the persistent kernel's workgroup sizes and the wide mode at each segment
+ * width on a scratch copy of the arena for trial_ticks ticks (the batch itself does
  * not advance), keeps the fastest and makes its mode the FS3D_BATCH_TUNED one. */
 int fs3d_batch_autotune(fs3d_batch *b, int32_t trial_ticks, int32_t *seg, int32_t *threads, int32_t *groups,
                         int32_t *mode, double *best_ms);
