@@ -189,8 +189,8 @@ int run_wide(fs3d_batch *b, int nticks, int want_hash) {
     const u64 *rule = device_rule_table(b->dev);
     for (int k = 0; k < nticks && e == hipSuccess; k++) {
       const int p = (par + k) & 1;
-      e = launch_wide(b->seg, b->d_worlds, b->d_prefix + (size_t)p * (b->n + 1), b->d_blk2ent[p], b->total_blocks[p],
-                      k, rule, want_hash ? b->d_hashes : nullptr, b->stream);
+      e = launch_wide(b->seg, b->d_worlds, b->d_prefix + (size_t)p * (b->n + 1), b->d_blk2ent[p], 0,
+                      b->total_blocks[p], k, rule, want_hash ? b->d_hashes : nullptr, b->stream);
     }
     hipError_t e2 = hipStreamEndCapture(b->stream, &graph);
     if (e != hipSuccess || e2 != hipSuccess) {

@@ -51,10 +51,24 @@ __host__ __device__ inline long long world_waves_dev(int ny, int nz, int rqpw, i
 }
 
 // Wide launch k of a round: entry i owns workgroups [bpre[i], bpre[i+1]) (4 waves
-// each; none when it sits the launch out); blk2ent maps workgroup -> entry.
+// each; none when it sits the launch out); blk2ent maps workgroup -> entry; the
+// launch covers workgroups [blk0, blk0 + blocks).
 // chg (optional): settled-world flags, four u32 per hash slot (see wide.hip).
-hipError_t launch_wide(int seg, const BWorld *ents, const long long *bpre, const int *blk2ent, long long blocks, int k,
-                       const u64 *rule, u64 *hashes, hipStream_t s, u32 *chg = nullptr);
+hipError_t launch_wide(int seg, const BWorld *ents, const long long *bpre, const int *blk2ent, long long blk0,
+                       long long blocks, int k, const u64 *rule, u64 *hashes, hipStream_t s, u32 *chg = nullptr);
+// The same on grids kept as bit planes.
+hipError_t launch_wide_planes(const BWorld *ents, const long long *bpre, const int *blk2ent, long long blk0,
+                              long long blocks, int k, u64 *hashes, hipStream_t s, u32 *chg);
+// Rain fills of worlds kept as bit planes, 256 plane words per workgroup.
+struct FillEntry {
+  u8 *g;
+  int nx, ny, nz;
+  int slot;
+  u64 seed, thr;
+  unsigned first;  // first workgroup of the entry
+};
+hipError_t launch_wide_fill(const FillEntry *ents, int n, unsigned blocks, u64 *hashes, u32 *chg, hipStream_t s);
+hipError_t launch_gather_hashes(const u64 *hashes, const int *slots, int n, u64 *out, hipStream_t s);
 hipError_t launch_expand(const long long *bpre, int n, int *blk2ent, hipStream_t s);
 // Tables of K launches in one pass (bpre: K prefixes of n+1; koff: K+1 launch
 // offsets into blk2ent; total = koff[K]).

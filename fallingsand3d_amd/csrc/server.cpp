@@ -52,7 +52,7 @@ struct Request {
 };
 
 struct Round {
-  u8 *h_buf = nullptr;  // pinned: entries | bpre (K x (n+1)) | launch offsets (K+1)
+  u8 *h_buf = nullptr;  // pinned: entries | bpre (K x (n+1)) | launch offsets (K+1) | finishing slots
   u8 *d_buf = nullptr;  // device copy of the same
   size_t cap = 0;
   int *d_blk = nullptr;  // device: blk2ent for all launches
@@ -65,6 +65,21 @@ struct Round {
   int nlaunch = 0;
   bool inflight = false;
 };
+
+// Table of the plane fills of one admission pass; free again once `done` has passed.
+struct FillTable {
+  FillEntry *h = nullptr, *d = nullptr;  // pinned, device
+  int cap = 0;
+  hipEvent_t done = nullptr;
+  bool used = false;
+};
+
+// Grids are kept as bit planes where those fit the bytes the budget counts
+// (16 bytes per 64 cells of a row, so rows of at least 16 cells) and a buffer
+// (4 GiB).
+bool planes_fit(const Request &r) {
+  return r.nx >= 16 && (size_t)((r.nx + 63) / 64) * (size_t)r.ny * (size_t)r.nz < (1ull << 28);
+}
 
 double now_s() {
   using namespace std::chrono;
@@ -113,6 +128,7 @@ struct fs3d_server {
   std::deque<long long> queue;
   std::vector<long long> pending, active;
   Round rounds[2];
+  FillTable fills[4];
   int next_round = 0;
   std::deque<int> inflight;  // round indices in launch order
   // stats
@@ -196,13 +212,47 @@ int reap(fs3d_server *s) {
   return FS3D_OK;
 }
 
+// A fill table that no fill in flight reads, with room for n entries; nullptr when
+// all are in use.
+int free_fill_table(fs3d_server *s, int n, FillTable **out) {
+  *out = nullptr;
+  for (FillTable &f : s->fills) {
+    if (f.used) {
+      const hipError_t q = hipEventQuery(f.done);
+      if (q == hipErrorNotReady) continue;
+      if (q != hipSuccess) return set_error(FS3D_ERR_HIP, "fill failed: %s", hipGetErrorString(q));
+      f.used = false;
+    }
+    if (!f.done) FS3D_HIP(hipEventCreateWithFlags(&f.done, hipEventDisableTiming));
+    if (n > f.cap) {
+      if (f.h) FS3D_HIP(hipHostFree(f.h));
+      if (f.d) FS3D_HIP(hipFree(f.d));
+      f.h = f.d = nullptr;
+      f.cap = std::max(n, 64) * 2;
+      FS3D_HIP(hipHostMalloc(&f.h, sizeof(FillEntry) * (size_t)f.cap, hipHostMallocDefault));
+      FS3D_HIP(hipMalloc(&f.d, sizeof(FillEntry) * (size_t)f.cap));
+    }
+    *out = &f;
+    return FS3D_OK;
+  }
+  return FS3D_OK;
+}
+
 // Admits queued requests in arrival order while a hash slot is free and the
 // arena can place their grids within the budget; stops at the first that does
 // not fit (it waits for finished grids to come back).  A request larger than
 // the whole budget, or whose chunk allocation fails while no other request
-// holds memory that could come back, is rejected.
+// holds memory that could come back, is rejected.  The admitted grids are filled
+// by one launch (three calls per request took 12 us of host time each before).
 int admit(fs3d_server *s) {
+  if (s->queue.empty()) return FS3D_OK;
+  FillTable *ft = nullptr;
+  const int most = (int)std::min(s->queue.size(), s->free_slots.size());
+  if (int rc = free_fill_table(s, most, &ft)) return rc;
+  if (!ft) return FS3D_OK;  // the next poll admits
   bool any = false;
+  int nfill = 0;
+  size_t blocks = 0;
   while (!s->queue.empty()) {
     Request &r = s->reqs[s->queue.front()];
     const size_t need = grid_bytes(r);
@@ -213,6 +263,9 @@ int admit(fs3d_server *s) {
       continue;
     }
     if (s->free_slots.empty()) break;
+    const size_t fill_blocks =
+        planes_fit(r) ? ((size_t)((r.nx + 63) / 64) * (size_t)r.ny * (size_t)r.nz + 255) / 256 : 0;
+    if (blocks + fill_blocks > 0x7FFFFFFFu) break;  // the next pass admits
     u8 *g = nullptr;
     const GridArena::Result res = s->arena.alloc(need, &g);
     if (res != GridArena::kOk) {
@@ -229,10 +282,15 @@ int admit(fs3d_server *s) {
     r.bytes = need;
     r.slot = s->free_slots.back();
     s->free_slots.pop_back();
-    FS3D_HIP(launch_fill_rain(r.g, r.nx, r.ny, r.nz, r.seed, r.thr, s->s_fill));
-    FS3D_HIP(hipMemsetAsync(s->d_hashes + r.slot, 0, sizeof(u64), s->s_fill));
-    // all four change flags set: the first ticks of a new world always run
-    FS3D_HIP(hipMemsetAsync(s->d_chg + (size_t)r.slot * 4, 1, 4 * sizeof(u32), s->s_fill));
+    if (planes_fit(r)) {
+      ft->h[nfill++] = FillEntry{r.g, r.nx, r.ny, r.nz, r.slot, r.seed, r.thr, (unsigned)blocks};
+      blocks += fill_blocks;
+    } else {
+      FS3D_HIP(launch_fill_rain(r.g, r.nx, r.ny, r.nz, r.seed, r.thr, s->s_fill));
+      FS3D_HIP(hipMemsetAsync(s->d_hashes + r.slot, 0, sizeof(u64), s->s_fill));
+      // all four change flags set: the first ticks of a new world always run
+      FS3D_HIP(hipMemsetAsync(s->d_chg + (size_t)r.slot * 4, 1, 4 * sizeof(u32), s->s_fill));
+    }
     r.status = kStatusActive;
     r.t_admit = now_s() - s->t0;
     r.remaining = r.ticks;
@@ -240,6 +298,12 @@ int admit(fs3d_server *s) {
     s->pending.push_back(s->queue.front());
     s->queue.pop_front();
     any = true;
+  }
+  if (nfill) {
+    FS3D_HIP(hipMemcpyAsync(ft->d, ft->h, sizeof(FillEntry) * (size_t)nfill, hipMemcpyHostToDevice, s->s_fill));
+    FS3D_HIP(launch_wide_fill(ft->d, nfill, (unsigned)blocks, s->d_hashes, s->d_chg, s->s_fill));
+    FS3D_HIP(hipEventRecord(ft->done, s->s_fill));
+    ft->used = true;
   }
   if (any) FS3D_HIP(hipEventRecord(s->fill_ev, s->s_fill));
   return FS3D_OK;
@@ -254,6 +318,10 @@ int launch_round(fs3d_server *s) {
     for (long long id : s->pending) s->active.push_back(id);
     s->pending.clear();
   }
+  // plane grids first: each launch covers them and the byte grids by two kernels
+  const int n_planes = (int)(std::stable_partition(s->active.begin(), s->active.end(),
+                                                   [&](long long id) { return planes_fit(s->reqs[id]); }) -
+                             s->active.begin());
   const int n = (int)s->active.size();
   int K = 0;
   for (long long id : s->active) K = std::max(K, std::min(s->cfg.round_ticks, s->reqs[id].remaining));
@@ -270,7 +338,7 @@ int launch_round(fs3d_server *s) {
     w.nx = r.nx;
     w.ny = r.ny;
     w.nz = r.nz;
-    w.lr = (r.nx + s->seg - 1) / s->seg;
+    w.lr = i < n_planes ? (r.nx + 63) / 64 : (r.nx + s->seg - 1) / s->seg;
     w.rqpw = 64 / w.lr;
     w.nt = std::min(s->cfg.round_ticks, r.remaining);
     w.slot = r.slot;
@@ -293,14 +361,17 @@ int launch_round(fs3d_server *s) {
   std::vector<long long> fin;
   for (int i = 0; i < n; i++)
     if (s->reqs[s->active[i]].remaining == ents[i].nt) fin.push_back(s->active[i]);
-  const size_t koff_bytes = sizeof(long long) * (size_t)(K + 1);
-  if (int rc = ensure_round_cap(rd, ent_bytes + pre_bytes + koff_bytes, blks, (int)fin.size(), K + 1)) return rc;
+  const size_t koff_bytes = sizeof(long long) * (size_t)(K + 1), fin_bytes = sizeof(int) * fin.size();
+  const size_t table_bytes = ent_bytes + pre_bytes + koff_bytes + fin_bytes;
+  if (int rc = ensure_round_cap(rd, table_bytes, blks, (int)fin.size(), K + 1)) return rc;
   std::copy(ents.begin(), ents.end(), (BWorld *)rd.h_buf);
   std::copy(pre.begin(), pre.end(), (long long *)(rd.h_buf + ent_bytes));
   long long *koff = (long long *)(rd.h_buf + ent_bytes + pre_bytes);
   koff[0] = 0;
   for (int k = 0; k < K; k++) koff[k + 1] = koff[k] + tot[k];
-  FS3D_HIP(hipMemcpyAsync(rd.d_buf, rd.h_buf, ent_bytes + pre_bytes + koff_bytes, hipMemcpyHostToDevice, s->s_tick));
+  int *fin_slots = (int *)(rd.h_buf + ent_bytes + pre_bytes + koff_bytes);
+  for (size_t i = 0; i < fin.size(); i++) fin_slots[i] = s->reqs[fin[i]].slot;
+  FS3D_HIP(hipMemcpyAsync(rd.d_buf, rd.h_buf, table_bytes, hipMemcpyHostToDevice, s->s_tick));
   const BWorld *d_ents = (const BWorld *)rd.d_buf;
   const long long *d_pre = (const long long *)(rd.d_buf + ent_bytes);
   // one pass fills the workgroup -> entry tables of all K launches
@@ -310,14 +381,16 @@ int launch_round(fs3d_server *s) {
   size_t boff = 0;
   FS3D_HIP(hipEventRecord(rd.ev[0], s->s_tick));
   for (int k = 0; k < K; k++) {
-    FS3D_HIP(launch_wide(s->seg, d_ents, d_pre + (size_t)k * (n + 1), rd.d_blk + boff, tot[k], k, rule, s->d_hashes,
-                         s->s_tick, s->d_chg));
+    const long long *pk = d_pre + (size_t)k * (n + 1);
+    const long long bp = pre[(size_t)k * (n + 1) + n_planes];  // workgroups of the plane grids
+    FS3D_HIP(launch_wide_planes(d_ents, pk, rd.d_blk + boff, 0, bp, k, s->d_hashes, s->s_tick, s->d_chg));
+    FS3D_HIP(launch_wide(s->seg, d_ents, pk, rd.d_blk + boff, bp, tot[k] - bp, k, rule, s->d_hashes, s->s_tick,
+                         s->d_chg));
     FS3D_HIP(hipEventRecord(rd.ev[k + 1], s->s_tick));
     boff += (size_t)tot[k];
   }
-  for (size_t i = 0; i < fin.size(); i++)
-    FS3D_HIP(hipMemcpyAsync(rd.h_hash + i, s->d_hashes + s->reqs[fin[i]].slot, sizeof(u64), hipMemcpyDeviceToHost,
-                            s->s_tick));
+  FS3D_HIP(launch_gather_hashes(s->d_hashes, (const int *)(rd.d_buf + ent_bytes + pre_bytes + koff_bytes),
+                                (int)fin.size(), rd.h_hash, s->s_tick));
   FS3D_HIP(hipEventRecord(rd.done, s->s_tick));
   rd.finishing = fin;
   rd.nlaunch = K;
@@ -397,6 +470,11 @@ int fs3d_server_destroy(fs3d_server *s) {
     if (rd.h_hash) (void)hipHostFree(rd.h_hash);
     for (hipEvent_t e : rd.ev) (void)hipEventDestroy(e);
     if (rd.done) (void)hipEventDestroy(rd.done);
+  }
+  for (FillTable &f : s->fills) {
+    if (f.h) (void)hipHostFree(f.h);
+    if (f.d) (void)hipFree(f.d);
+    if (f.done) (void)hipEventDestroy(f.done);
   }
   s->arena.clear();
   if (s->d_hashes) (void)hipFree(s->d_hashes);
