@@ -111,6 +111,11 @@ void release(fs3d_world *w) {
   for (int i = 0; i < 2; i++)
     if (w->planes[i]) (void)hipFree(w->planes[i]);
   if (w->d_reserved) (void)hipFree(w->d_reserved);
+  for (int i = 0; i < 2; i++)
+    if (w->pflags[i]) (void)hipFree(w->pflags[i]);
+  if (w->d_since) (void)hipFree(w->d_since);
+  if (w->d_items) (void)hipFree(w->d_items);
+  if (w->d_nitems) (void)hipFree(w->d_nitems);
   if (w->d_parts) (void)hipFree(w->d_parts);
   if (w->d_rgb) (void)hipFree(w->d_rgb);
   if (w->d_hit) (void)hipFree(w->d_hit);
@@ -258,80 +263,101 @@ constexpr int kPlaneMinTicks = 3;
 bool plane_path(const fs3d_world *w, int nticks) {
   if (w->planes_off || w->seg_req != 0 || w->d_stats || nticks < 1) return false;
   if (w->skip != FS3D_SKIP_OFF && w->skip != FS3D_SKIP_AUTO) return false;
-  // large grids of which little moves: the packed schedule ticks only that (2048^3
-  // pillar scene 0.36 ms per tick, dense plane pairs 0.42)
-  if (w->skip && skip_schedule(w) == FS3D_SKIP_SEGS) return false;
   if (!w->skip && w->fuse_set && !w->fuse) return false;
   if (w->nx < 16 || plane_words(plane_shape(w->nx, w->ny, w->nz)) >= (1ull << 28)) return false;
   return w->planes_valid || nticks >= kPlaneMinTicks;
 }
 
-// Plane buffers on first use; false (and the byte kernels from then on) when the
-// device has no room for them.
+// Whether the plane ticks of a skipping world visit only its active items.  Below
+// this size a pass over everything is as fast as listing what moves.
+constexpr u64 kItemsMinVoxels = 1ull << 29;
+bool item_ticks(const fs3d_world *w) { return w->skip && (u64)w->n > kItemsMinVoxels; }
+
+// Plane buffers (and the item lists) on first use; false (and the byte kernels from
+// then on) when the device has no room for them.
 bool ensure_planes(fs3d_world *w) {
-  if (w->planes[0]) return true;
-  const size_t bytes = plane_words(plane_shape(w->nx, w->ny, w->nz)) * 16;
-  hipError_t e = hipMalloc((void **)&w->d_reserved, sizeof(u32));
-  for (int i = 0; i < 2 && e == hipSuccess; i++) e = hipMalloc(&w->planes[i], bytes);
+  const PlaneShape ps = plane_shape(w->nx, w->ny, w->nz);
+  hipError_t e = hipSuccess;
+  if (!w->planes[0]) {
+    e = hipMalloc((void **)&w->d_reserved, sizeof(u32));
+    for (int i = 0; i < 2 && e == hipSuccess; i++) e = hipMalloc(&w->planes[i], plane_words(ps) * 16);
+    for (int i = 0; i < 2 && e == hipSuccess; i++) e = launch_plane_pad(ps, w->planes[i], w->stream);
+  }
+  if (item_ticks(w) && !w->d_items && e == hipSuccess) {
+    const PlaneCells c = plane_cells(ps);
+    int cus = 0;
+    e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, w->dev);
+    w->item_waves = (u32)(std::max(cus, 1) * plane_list_blocks_per_cu() * 4);
+    for (int i = 0; i < 2 && e == hipSuccess; i++) e = hipMalloc(&w->pflags[i], c.flag_words * sizeof(u64));
+    if (e == hipSuccess) e = hipMalloc(&w->d_since, c.since_words * sizeof(u64));
+    if (e == hipSuccess) e = hipMalloc(&w->d_nitems, sizeof(u32));
+    if (e == hipSuccess) e = hipMalloc(&w->d_items, c.list_words * sizeof(u32));
+  }
   if (e == hipSuccess) return true;
   (void)hipGetLastError();
-  for (void *&p : w->planes) {
+  auto drop = [](auto *&p) {
     if (p) (void)hipFree(p);
     p = nullptr;
+  };
+  for (int i = 0; i < 2; i++) {
+    if (w->planes[i]) (void)hipFree(w->planes[i]);
+    w->planes[i] = nullptr;
+    drop(w->pflags[i]);
   }
-  if (w->d_reserved) (void)hipFree(w->d_reserved);
-  w->d_reserved = nullptr;
+  drop(w->d_reserved);
+  drop(w->d_since);
+  drop(w->d_nitems);
+  drop(w->d_items);
+  w->planes_valid = false;
   w->planes_off = true;
   return false;
 }
 
-// The launch shape of a pair: row quads along y and z per lane.  Longer sweeps
-// evaluate fewer halo quads, shorter ones keep more waves in flight (us per tick
-// at (k, zlen): 512^3 9.3 at (1, 4), 10.7 at (2, 4); 1000x701x603 22.4 at (2, 8),
-// 24.4 at (2, 4), 31.1 at (2, 16); 1024^3 55.5 at (2, 16), 57.6 at (2, 8); 2048^3
-// 416 at (2, 16), 424 at (2, 8)).
-void pair_shape(const PlaneShape &ps, int *k, int *zlen) {
-  const int upw = 64 / ps.lr, nyq = (ps.ny + 1) >> 1, nzq = (ps.nz + 1) >> 1;
-  const int opts[][2] = {{2, 16}, {2, 8}, {1, 4}, {1, 2}, {1, 1}};
-  for (const auto &o : opts) {
-    *k = o[0];
-    *zlen = o[1];
-    const long long strips = (nyq + o[0] - 1) / o[0];
-    const long long waves = ((strips + upw - 1) / upw) * ((nzq + o[1] - 1) / o[1]);
-    if (waves >= 2048) break;
-  }
-}
-
 // Enqueues nticks ticks of the planes (packing them first when they are not the
-// current state) and the unpacking into buf[cur]; *pfinal: the plane buffer
-// holding the result.
+// current state) and the unpacking into buf[cur].  *pfinal: the index of the plane
+// buffer holding the result, + 2 * that of the last pass's change flags.
 int enqueue_planes(fs3d_world *w, int nticks, int hash_every, const u64 *tick_dev, int *pfinal, bool launch = true) {
   const PlaneShape ps = plane_shape(w->nx, w->ny, w->nz);
-  int src = w->planes_valid ? w->pcur : 0, k2 = 1, zlen = 1;
-  pair_shape(ps, &k2, &zlen);
+  const bool items = item_ticks(w);
+  int src = w->planes_valid ? w->pcur : 0, f = w->fcur;
+  bool fresh = !w->planes_valid || !w->pflags_valid;
   if (launch && !w->planes_valid) {
     FS3D_HIP(launch_fill_u32(w->d_reserved, 1, 0, w->stream));
     FS3D_HIP(launch_plane_pack(ps, w->buf[w->cur], w->planes[src], w->d_reserved, w->stream));
   }
+  if (launch && items && fresh)
+    FS3D_HIP(launch_fill_u64(w->pflags[f], plane_cells(ps).flag_words, ~0ull, w->stream));
   auto hashed_after = [&](int k) { return hash_every > 0 && (k + 1) % hash_every == 0; };
   for (int k = 0; k < nticks;) {
     const u64 t = w->tick + (u64)k;
     const bool pair = (t & 1u) && k + 1 < nticks && !hashed_after(k);
     if (launch) {
-      if (pair)
-        FS3D_HIP(launch_plane_pair(ps, w->planes[src], w->planes[src ^ 1], t, tick_dev, (u32)k, k2, zlen, w->stream));
+      if (items)
+        FS3D_HIP(launch_plane_list(ps, w->planes[src], w->planes[src ^ 1], t, tick_dev, (u32)k, pair, fresh,
+                                   w->pflags[f], w->pflags[f ^ 1], w->d_since, w->d_items, w->d_nitems,
+                                   w->item_waves, w->stream));
+      else if (pair)
+        FS3D_HIP(launch_plane_pair(ps, w->planes[src], w->planes[src ^ 1], t, tick_dev, (u32)k, w->stream));
       else
         FS3D_HIP(launch_plane_tick(ps, w->planes[src], w->planes[src ^ 1], t, tick_dev, (u32)k, w->stream));
     }
     src ^= 1;
+    f ^= 1;
+    fresh = false;
     k += pair ? 2 : 1;
     if (launch && hashed_after(k - 1)) {
       FS3D_HIP(launch_plane_hash(ps, w->planes[src], w->buf[w->cur], w->d_reserved, w->d_parts, w->stream));
       FS3D_HIP(launch_hash_finalize(w->d_parts, w->d_small + k / hash_every, w->stream));
     }
   }
-  if (launch) FS3D_HIP(launch_plane_unpack(ps, w->planes[src], w->buf[w->cur], w->d_reserved, w->stream));
-  if (pfinal) *pfinal = src;
+  if (launch) {
+    if (items)
+      FS3D_HIP(launch_plane_unpack_cells(ps, w->planes[src], w->buf[w->cur], w->pflags[f], w->d_since, w->d_reserved,
+                                         w->stream));
+    else
+      FS3D_HIP(launch_plane_unpack(ps, w->planes[src], w->buf[w->cur], w->d_reserved, w->stream));
+  }
+  if (pfinal) *pfinal = src | f << 1;
   return FS3D_OK;
 }
 
@@ -347,8 +373,10 @@ int choose_path(fs3d_world *w, int nticks, bool *planes) {
 // The world's bookkeeping after nticks ticks on either path.
 void ticked(fs3d_world *w, int nticks, bool planes, int fin) {
   if (planes) {
-    w->pcur = fin;
+    w->pcur = fin & 1;
+    w->fcur = fin >> 1;
     w->planes_valid = true;
+    w->pflags_valid = item_ticks(w);
     w->masks_stale = true;
     w->occ_valid = false;
   } else {
@@ -426,7 +454,8 @@ namespace {
 int world_graph(fs3d_world *w, int nticks, int hash_every, bool planes, hipGraphExec_t *out) {
   // a plane graph pairs its ticks by the start tick's parity
   const int state = !planes ? w->cur
-                            : 16 | w->cur | (w->planes_valid ? 8 | w->pcur << 1 : 0) | (int)(w->tick & 1u) << 2;
+                            : 64 | w->cur | (w->planes_valid ? 8 | w->pcur << 1 : 0) | (int)(w->tick & 1u) << 2 |
+                                  (item_ticks(w) ? w->fcur << 4 | (w->pflags_valid ? 32 : 0) : 0);
   const auto key = std::make_tuple(nticks, hash_every, state);
   auto it = w->graphs.find(key);
   if (it == w->graphs.end()) {
@@ -576,7 +605,7 @@ int fs3d_world_set_voxel(fs3d_world *w, int32_t x, int32_t y, int32_t z, uint8_t
   FS3D_HIP(hipMemcpyAsync(w->buf[w->cur] + off, &v, 1, hipMemcpyHostToDevice, w->stream));
   if (w->planes_valid)
     FS3D_HIP(launch_plane_set(plane_shape(w->nx, w->ny, w->nz), w->planes[w->pcur], x, y, z, v, w->d_reserved,
-                              w->stream));
+                              w->pflags_valid ? w->pflags[w->fcur] : nullptr, w->stream));
   if (int rc = mark_cell(w, x, y, z)) return rc;
   FS3D_HIP(hipStreamSynchronize(w->stream));
   return clear_error();

@@ -209,6 +209,14 @@ struct fs3d_world {
   int pcur = 0;
   bool planes_valid = false, planes_off = false;
   fs3d::u32 *d_reserved = nullptr;  // a byte >= 4 has been packed or set
+  // ticks of the active items only: change flags of the last pass (pflags[fcur],
+  // exact or too many while pflags_valid), items changed since the bytes were
+  // written, work list and its count
+  fs3d::u64 *pflags[2] = {nullptr, nullptr}, *d_since = nullptr;
+  fs3d::u32 *d_items = nullptr, *d_nitems = nullptr;
+  int fcur = 0;
+  bool pflags_valid = false;
+  fs3d::u32 item_waves = 0;
   bool masks_stale = false;         // plane ticks have run since the change masks were last exact
   bool fuse_set = false;            // set_fuse has been called
   // cached graphs keyed by (nticks, hash_every, buffers and path)

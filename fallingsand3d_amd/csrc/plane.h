@@ -14,8 +14,10 @@ struct PlaneShape {
   int lr = 0;  // 64-cell words per row
 };
 inline PlaneShape plane_shape(int nx, int ny, int nz) { return PlaneShape{nx, ny, nz, (nx + 63) / 64}; }
-// 16-byte words of a plane grid.
-inline size_t plane_words(const PlaneShape &p) { return (size_t)p.lr * (size_t)p.ny * (size_t)p.nz; }
+// 16-byte words of a plane grid with the zero rows around it.
+inline size_t plane_words(const PlaneShape &p) {
+  return (size_t)p.lr * ((size_t)(p.ny + 1) * (size_t)(p.nz + 2) + 1);
+}
 
 struct PlaneArgs {
   const plane_u32x4 *src;
@@ -33,9 +35,11 @@ struct PlaneArgs {
 // One tick, any parity.
 hipError_t launch_plane_tick(const PlaneShape &ps, const void *src, void *dst, u64 t, const u64 *tick_dev, u32 k_off,
                              hipStream_t s);
-// Ticks t and t + 1, t odd: k even-parity row quads along y and zlen along z per lane.
+// Ticks t and t + 1, t odd.
 hipError_t launch_plane_pair(const PlaneShape &ps, const void *src, void *dst, u64 t, const u64 *tick_dev, u32 k_off,
-                             int k, int zlen, hipStream_t s);
+                             hipStream_t s);
+// Zeroes the rows around the grid (once per buffer: no kernel writes them).
+hipError_t launch_plane_pad(const PlaneShape &ps, void *planes, hipStream_t s);
 // Bytes (values >= 4 as STATIC, *reserved set) to planes and back (with *reserved,
 // bytes >= 4 already in g stay).
 hipError_t launch_plane_pack(const PlaneShape &ps, const u8 *g, void *planes, u32 *reserved, hipStream_t s);
@@ -44,7 +48,29 @@ hipError_t launch_plane_unpack(const PlaneShape &ps, const void *planes, u8 *g, 
 // State hash of the grid into the partial sums; g holds the bytes of reserved cells.
 hipError_t launch_plane_hash(const PlaneShape &ps, const void *planes, const u8 *g, const u32 *reserved, u64 *parts,
                              hipStream_t s);
-hipError_t launch_plane_set(const PlaneShape &ps, void *planes, int x, int y, int z, u8 v, u32 *reserved,
+// One cell of planes, and of its item's change flags when given.
+hipError_t launch_plane_set(const PlaneShape &ps, void *planes, int x, int y, int z, u8 v, u32 *reserved, u64 *flags,
                             hipStream_t s);
+
+// ---- ticks of the active items only (plane.hip has the rule) ----
+constexpr int kItemQuads = 1;   // even-parity row quads of an item along y
+constexpr int kItemLayers = 8;  // and along z
+struct PlaneCells {
+  int strips = 0, zcells = 0;  // the strip grid: items of one word per cell and word
+  int virt = 0;                // 1: a virtual word behind each row
+  size_t flag_words = 0, since_words = 0, list_words = 0;  // u64, u64, u32
+};
+PlaneCells plane_cells(const PlaneShape &ps);
+int plane_list_blocks_per_cu();
+// A pass over the active items: ticks t and t + 1 (pair, t odd) or tick t (of
+// either parity; *tick_dev + k_off has t's).  flags_in: the pass before; flags_out:
+// this one's; since: items changed since the bytes were written; fresh: the first
+// pass after packing (every flag set).
+hipError_t launch_plane_list(const PlaneShape &ps, const void *src, void *dst, u64 t, const u64 *tick_dev, u32 k_off,
+                             bool pair, bool fresh, const u64 *flags_in, u64 *flags_out, u64 *since, u32 *list,
+                             u32 *count, u32 nwaves, hipStream_t s);
+// Writes the bytes of the items in since or flags (the last pass's) and clears since.
+hipError_t launch_plane_unpack_cells(const PlaneShape &ps, const void *planes, u8 *g, const u64 *flags, u64 *since,
+                                     const u32 *reserved, hipStream_t s);
 
 }  // namespace fs3d

@@ -1,8 +1,11 @@
 // Bit-plane kernels: packing, unpacking, single ticks, pairs of ticks and the
 // state hash on two bits per cell (plane_core.h has the layout and the rule).
 //
-// A plane grid is rows of lr = ceil(nx / 64) words of 16 bytes, v[z][y][word].
-// One lane holds one word of each of a row quad's four rows.
+// A plane grid is rows of lr = ceil(nx / 64) words of 16 bytes, v[z][y][word], with
+// a row of zeros (STATIC) before every layer's first row and a layer of them at
+// either end: the rows around the grid that its border blocks read are memory like
+// any other, and a quad's four loads differ by uniform offsets.  One lane holds one
+// word of each of a row quad's four rows.
 //
 // What this replaces: the byte kernels move 2 bytes per voxel-update and gather
 // one 8-byte table entry per block (510 vector instructions per 1024 blocks and
@@ -61,23 +64,24 @@ __global__ __launch_bounds__(256) void plane_tick_kernel(PlaneArgs a) {
   if (__builtin_amdgcn_readfirstlane(first) >= nyq || zq >= nzq) return;
   const Lane L = lane_of(a, first, lane);
   const Planes src(a.src, a.bytes), dst(a.dst, a.bytes);
+  const u32 row = (u32)a.lr * 16u, layer = row * (u32)(a.ny + 1);
   const int y0 = 2 * L.unit - p, z0 = 2 * zq - p;
+  const bool in = L.in && L.unit < nyq;
+  const u32 off = in ? (u32)(z0 + 1) * layer + (u32)(y0 + 1) * row + (u32)L.seg * 16u : kOutside;
   u32x4 r[4];
-  u32 off[4];
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int y = y0 + (i & 1), z = z0 + (i >> 1);
-    const bool ok = L.in && (unsigned)y < (unsigned)a.ny && (unsigned)z < (unsigned)a.nz;
-    off[i] = ok ? ((u32)(z * a.ny + y) * (u32)a.lr + (u32)L.seg) * 16u : kOutside;
-    r[i] = src.load(off[i]);
-  }
+  for (int i = 0; i < 4; i++) r[i] = src.load(off, (i & 1 ? row : 0u) + (i >> 1 ? layer : 0u));
   const u32 base = variant_base((u32)L.unit, (u32)zq, t);
   if (p)
     quad_odd<WALL>(r, (u32)L.seg, base, L.prev, L.next, L.wall);
   else
     quad_even(r, (u32)L.seg, base);
 #pragma unroll
-  for (int i = 0; i < 4; i++) dst.store(off[i], r[i]);
+  for (int l = 0; l < 2; l++)
+    if ((unsigned)(z0 + l) < (unsigned)a.nz) {
+      dst.store(in && y0 >= 0, off + (l ? layer : 0u), r[2 * l]);
+      dst.store(in && y0 + 1 < a.ny, off + row + (l ? layer : 0u), r[2 * l + 1]);
+    }
 }
 
 // ---- a pair of ticks --------------------------------------------------------------
@@ -87,7 +91,12 @@ __global__ __launch_bounds__(256) void plane_tick_kernel(PlaneArgs a) {
 // row quad (Y0 + j, b) takes its four rows from odd quads j and j + 1 of s = b
 // (their upper layers) and s = b + 1 (their lower ones).  Everything stays in
 // registers: the upper layers of the previous s (top), and the quad before.
-template <bool WALL, int K>
+//
+// A strip's odd quad K is the next strip's quad 0.  With SHARE, it is evaluated by
+// the next strip alone, lr lanes on, and its two rows come from there; the wave's
+// last strip then only serves the one before (K odd evaluations per K quads and
+// layer pair instead of K + 1, on all strips but one).
+template <bool WALL, int K, bool SHARE>
 __global__ __launch_bounds__(256) void plane_pair_kernel(PlaneArgs a) {
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -100,109 +109,455 @@ __global__ __launch_bounds__(256) void plane_pair_kernel(PlaneArgs a) {
   const int nzq = (a.nz + 1) >> 1;
   const int Z0 = zr * a.zlen, Z1 = min(Z0 + a.zlen, nzq);
   if (Z0 >= nzq) return;
-  const Lane L = lane_of(a, yt * a.upw, lane);
+  const Lane L = lane_of(a, yt * (SHARE ? a.upw - 1 : a.upw), lane);
   const int Y0 = L.unit * K;
   const u32 seg = (u32)L.seg;
   const Planes src(a.src, a.bytes), dst(a.dst, a.bytes);
-  const u32 row_bytes = (u32)a.lr * 16u, layer_bytes = row_bytes * (u32)a.ny;
-  const u32 lane_off = (u32)(2 * Y0) * row_bytes + seg * 16u;  // row 2 Y0 of a layer
-  auto offset = [&](int dy, int z) {
-    const bool ok = L.in && (unsigned)(2 * Y0 + dy) < (unsigned)a.ny && (unsigned)z < (unsigned)a.nz;
-    return ok ? lane_off + (u32)dy * row_bytes + (u32)z * layer_bytes : kOutside;
-  };
+  const u32 row = (u32)a.lr * 16u, layer = row * (u32)(a.ny + 1);
+  // row 2 Y0 - 1 of layer 2 Z0 - 1; strips past the last row are bounded by the buffer
+  const u32 off = L.in ? (u32)(2 * Z0) * layer + (u32)(2 * Y0) * row + seg * 16u : kOutside;
+  const bool owns = L.in && (!SHARE || L.unit < yt * (a.upw - 1) + a.upw - 1);
+  const int beyond = (lane + a.lr < 64 ? lane + a.lr : lane) * 4;  // the same word of the next strip
+  constexpr int NI = SHARE ? K : K + 1;  // odd quads evaluated per layer pair
   u32x4 top[2 * K];
   u32x4 nx[4];
 #pragma unroll
-  for (int r = 0; r < 4; r++) nx[r] = src.load(offset(-1 + (r & 1), 2 * Z0 - 1 + (r >> 1)));
-  for (int s = Z0; s <= Z1; s++) {
+  for (int r = 0; r < 4; r++) nx[r] = src.load(off, (r & 1 ? row : 0u) + (r >> 1 ? layer : 0u));
+  u32 base = 0;  // of odd layer 2 s - 1
+  for (int s = Z0; s <= Z1; s++, base += 2u * layer) {
+    // the even quad (Y0 + j, s - 1) from the rows of the odd quads around it
+    auto even = [&](int j, const u32x4 &low0, const u32x4 &low1) {
+      if (s == Z0) return;
+      u32x4 e[4] = {top[2 * j], top[2 * j + 1], low0, low1};
+      quad_even(e, seg, variant_base((u32)(Y0 + j), (u32)(s - 1), t + 1u));
+      const u32 b = base - layer;  // layer 2 s - 2
+      const bool on0 = owns && 2 * (Y0 + j) < a.ny, on1 = owns && 2 * (Y0 + j) + 1 < a.ny;
+      dst.store(on0, off + (b + (u32)(2 * j + 1) * row), e[0]);
+      dst.store(on1, off + (b + (u32)(2 * j + 2) * row), e[1]);
+      if (2 * s - 1 < a.nz) {
+        dst.store(on0, off + (base + (u32)(2 * j + 1) * row), e[2]);
+        dst.store(on1, off + (base + (u32)(2 * j + 2) * row), e[3]);
+      }
+    };
     u32x4 lowp, upp;  // upper row of the odd quad before: its lower and upper layer
+    u32x4 low0, up0;  // SHARE: lower row of quad 0
 #pragma unroll
-    for (int i = 0; i <= K; i++) {
+    for (int i = 0; i < NI; i++) {
       u32x4 q[4];
 #pragma unroll
       for (int r = 0; r < 4; r++) q[r] = nx[r];
-      const int in = i < K ? i + 1 : 0, sn = i < K ? s : s + 1;
+      const u32 at = i < NI - 1 ? base + (u32)(2 * i + 2) * row : base + 2u * layer;
 #pragma unroll
-      for (int r = 0; r < 4; r++) nx[r] = src.load(offset(2 * in - 1 + (r & 1), 2 * sn - 1 + (r >> 1)));
+      for (int r = 0; r < 4; r++) nx[r] = src.load(off, at + (r & 1 ? row : 0u) + (r >> 1 ? layer : 0u));
       // One quad at a time: left alone, the scheduler interleaves the evaluations
       // of several, for which there are no registers.
       __builtin_amdgcn_sched_barrier(0);
       quad_odd<WALL>(q, seg, variant_base((u32)(Y0 + i), (u32)s, t), L.prev, L.next, L.wall);
       __builtin_amdgcn_sched_barrier(0);
       if (i > 0) {
-        if (s > Z0) {
-          u32x4 e[4] = {top[2 * i - 2], top[2 * i - 1], lowp, q[0]};
-          quad_even(e, seg, variant_base((u32)(Y0 + i - 1), (u32)(s - 1), t + 1u));
-#pragma unroll
-          for (int r = 0; r < 4; r++) dst.store(offset(2 * i - 2 + (r & 1), 2 * (s - 1) + (r >> 1)), e[r]);
-        }
+        even(i - 1, lowp, q[0]);
         top[2 * i - 2] = upp;
         top[2 * i - 1] = q[2];
+      } else if (SHARE) {
+        low0 = q[0];
+        up0 = q[2];
       }
       lowp = q[1];
       upp = q[3];
+    }
+    if constexpr (SHARE) {
+      u32x4 l, u;
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        l[c] = from_lane(beyond, low0[c]);
+        u[c] = from_lane(beyond, up0[c]);
+      }
+      even(K - 1, lowp, l);
+      top[2 * K - 2] = upp;
+      top[2 * K - 1] = u;
+    }
+  }
+}
+
+// ---- ticks of the active items only ----------------------------------------------
+// An item is one word of a strip of K even-parity row quads over zlen z row-quads
+// (a cell of the strip grid).  A pass (a pair of ticks, or one tick at either end of
+// a run) leaves an item alone when nothing in it can change: no block of it changed
+// during the pass before (both parities, since a single tick's flags are ORed onto
+// the pass before it), and neither did a block that reaches over its faces from a
+// neighbour.  Whether a block is a fixed point does not depend on its variant, so a
+// block that did not change at its parity's last tick and whose cells did not change
+// since does not change.  The destination then already holds the item: it is the
+// state of two passes ago.
+//
+// Flags are u64 masks over the words of a strip (bit = word), kFlags per cell: any
+// change; a change of a block at the item's first or last word bit, row, layer; any
+// change in the last pass alone.  A flag may be set without need, never missing.
+//
+// Bound by the 128-byte lines around the 16-byte words it visits: sand columns over a
+// pool at 2048^3, where 12 % of the items have work, read 2.1 GB and write 0.5 GB per
+// pass (0.69 ms for two ticks, 0.13 ms of it instructions), against 4.3 GB (0.82 ms)
+// over everything; the byte kernels' packed schedule takes 2 x 0.36 ms.
+enum { kAny = 0, kXFirst, kXLast, kYFirst, kYLast, kZFirst, kZLast, kNow, kFlags };
+
+// One thread per cell: which items have work, appended to the list in word order;
+// clears the flags the pass will write (or, before a single tick, carries the old
+// ones over), and adds the changes of the pass before to the cells' `since` (fresh:
+// the first pass over a grid just packed, whose flags are all set).
+// A full last word (nx a multiple of 64) has a virtual neighbour, word lr, whose
+// lane evaluates the half blocks at the row's end.
+__global__ __launch_bounds__(256) void plane_plan_kernel(const u64 *__restrict__ in, u64 *__restrict__ out,
+                                                         u64 *__restrict__ since, int strips, int zcells, int lr,
+                                                         int virt, int carry, int fresh, u32 *list, u32 *count) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int ncell = strips * zcells;
+  const int c = (int)blockIdx.x * 256 + (int)threadIdx.x;
+  const u64 bits = lr == 64 ? ~0ull : (1ull << lr) - 1ull;
+  u64 act = 0;
+  int zr = 0, st = 0;
+  if (c < ncell) {
+    zr = c / strips;
+    st = c - zr * strips;
+#pragma unroll
+    for (int dz = -1; dz <= 1; dz++)
+#pragma unroll
+      for (int dy = -1; dy <= 1; dy++) {
+        const int y = st + dy, z = zr + dz;
+        if (y < 0 || y >= strips || z < 0 || z >= zcells) continue;
+        const u64 *f = in + (size_t)(z * strips + y) * kFlags;
+        u64 m = f[kAny];
+        if (dy) m &= f[dy > 0 ? kYFirst : kYLast];
+        if (dz) m &= f[dz > 0 ? kZFirst : kZLast];
+        act |= m | ((m & f[kXFirst]) >> 1) | ((m & f[kXLast]) << 1);
+      }
+    act &= bits;
+    const u64 *f = in + (size_t)c * kFlags;
+    since[c] = fresh ? 0ull : since[c] | f[kNow];
+#pragma unroll
+    for (int i = 0; i < kFlags; i++) out[(size_t)c * kFlags + i] = carry && i != kNow ? f[i] : 0ull;
+  }
+  const int n = __builtin_popcountll(act) + (virt && ((act >> (lr - 1)) & 1u) ? 1 : 0);
+  int incl = n;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int y = __shfl_up(incl, d, 64);
+    if (lane >= d) incl += y;
+  }
+  __shared__ u32 wsum[4], wbase;
+  if (lane == 63) wsum[wv] = (u32)incl;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const u32 tot = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+    wbase = tot ? atomicAdd(count, tot) : 0u;
+  }
+  __syncthreads();
+  u32 at = wbase + (u32)(incl - n);
+  for (int i = 0; i < wv; i++) at += wsum[i];
+  const u32 code = (u32)c * (u32)(lr + virt);
+  while (act) {
+    const int s = __builtin_ctzll(act);
+    act &= act - 1ull;
+    list[at++] = code + (u32)s;
+    if (virt && s == lr - 1) list[at++] = code + (u32)lr;
+  }
+}
+
+enum { kPair = 0, kOdd, kEven };
+
+// A lane per listed item, 62 per wave: lanes 0 and 63 repeat the items before and
+// after the wave's own, so that a word's neighbours are in the lanes beside it when
+// they have work.  A neighbour that has none is not looked at: the block across the
+// edge is a fixed point, so its cells in this item stay as they are, and it does not
+// move with STATIC in the neighbour's cells either (what blocks every move with
+// those cells there blocks the moves among the others).
+template <int MODE, int K>
+__global__ __launch_bounds__(256) void plane_list_kernel(PlaneArgs a, const u32 *__restrict__ list, const u32 *count,
+                                                         u64 *flags, int strips, int virt, u32 nwaves) {
+  const int lane = threadIdx.x & 63;
+  const u32 wave = blockIdx.x * 4 + (u32)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const u32 t = (u32)tick_of(a);
+  const u32 n = *count;
+  const Planes src(a.src, a.bytes), dst(a.dst, a.bytes);
+  const u32 row = (u32)a.lr * 16u, layer = row * (u32)(a.ny + 1);
+  const int m = a.zlen;
+  const int prev = (lane ? lane - 1 : 0) * 4, next = (lane < 63 ? lane + 1 : 63) * 4;
+  for (u32 w = wave; w * 62u < n; w += nwaves) {
+    const u32 e = w * 62u + (u32)lane - 1u;
+    const bool in = e < n;  // (entry -1 is none)
+    const u32 code = in ? list[e] : 0xFFFFFF00u;
+    const u32 per = (u32)(a.lr + virt), cell = code / per;
+    const int seg = (int)(code - cell * per);
+    const int zr = (int)(cell / (u32)strips), st = (int)(cell - (u32)zr * (u32)strips);
+    const int y0 = st * 2 * K, z0 = zr * 2 * m, by0 = st * K, bz0 = zr * m;
+    const u32 cp = from_lane(prev, code), cn = from_lane(next, code);
+    const bool has_prev = in && lane > 0 && seg > 0 && cp + 1u == code;
+    const bool has_next = in && lane < 63 && seg + 1 < (int)per && cn == code + 1u;
+    const bool word = in && seg < a.lr;  // not the virtual word
+    const bool mine = word && lane > 0 && lane < 63;
+    // row y0 - 1 of layer z0 - 1
+    const u32 off = word ? (u32)z0 * layer + (u32)y0 * row + (u32)seg * 16u : kOutside;
+    bool on[2 * K];
+#pragma unroll
+    for (int j = 0; j < 2 * K; j++) on[j] = mine && y0 + j < a.ny;
+    const int zleft = a.nz - z0;  // layers of the item inside the grid
+    u32 acc[kFlags] = {};
+    // odd quad (i, s) in place; returns its changed blocks, bit 31 also standing
+    // for the block at the word's right edge
+    auto odd = [&](u32x4(&q)[4], int i, int s) {
+      u32 lo[2][4], hi[2][4], v0, v1;
+      variant_planes((u32)seg, variant_base((u32)(by0 + i), (u32)(bz0 + s), t), v0, v1);
+      u32 last = 0;  // last odd cells, kept where no neighbour evaluates their block
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        u32 px = from_lane(prev, q[r].y), ph = from_lane(prev, q[r].w);
+        px = has_prev ? px : 0u;
+        ph = has_prev ? ph : 0u;
+        const int l = r >> 1, kl = (r & 1) ? 3 : 0, kr = (r & 1) ? 2 : 1;
+        lo[l][kl] = shift_in(q[r].y, px);
+        hi[l][kl] = shift_in(q[r].w, ph);
+        lo[l][kr] = q[r].x;
+        hi[l][kr] = q[r].z;
+        last |= (q[r].y >> 31) << r | (q[r].w >> 31) << (4 + r);
+      }
+      const u32 c = block_rule<false>(lo, hi, v0, v1, 0u);
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int l = r >> 1, kl = (r & 1) ? 3 : 0, kr = (r & 1) ? 2 : 1;
+        // (read by every lane: a lane left out is not readable by its neighbour)
+        u32 nx = from_lane(next, lo[l][kl]), nh = from_lane(next, hi[l][kl]);
+        nx = has_next ? nx : last >> r;
+        nh = has_next ? nh : last >> (4 + r);
+        q[r] = u32x4{lo[l][kr], shift_back(lo[l][kl], nx & 1u), hi[l][kr], shift_back(hi[l][kl], nh & 1u)};
+      }
+      const u32 cnext = from_lane(next, c);
+      return c | (has_next ? cnext << 31 : 0u);
+    };
+    // (i, s) in quads of the item's rows and layers; quads past the grid hold nothing
+    auto note = [&](u32 c, int y, int z, bool yf, bool yl, bool zf, bool zl) {
+      c = y0 + y < a.ny && z < zleft ? c : 0u;
+      acc[kAny] |= c;
+      if (yf) acc[kYFirst] |= c;
+      if (yl) acc[kYLast] |= c;
+      if (zf) acc[kZFirst] |= c;
+      if (zl) acc[kZLast] |= c;
+    };
+    if constexpr (MODE == kEven) {
+      u32 base = layer;  // layer 2 b
+#pragma unroll 1
+      for (int b = 0; b < m; b++, base += 2u * layer)
+#pragma unroll
+        for (int j = 0; j < K; j++) {
+          u32x4 q[4];
+#pragma unroll
+          for (int r = 0; r < 4; r++)
+            q[r] = src.load(off, base + (u32)(2 * j + 1 + (r & 1)) * row + (r >> 1 ? layer : 0u));
+          const u32 c = quad_even(q, (u32)seg, variant_base((u32)(by0 + j), (u32)(bz0 + b), t));
+          note(c, 2 * j, 2 * b, j == 0, j == K - 1, b == 0, b == m - 1);
+#pragma unroll
+          for (int r = 0; r < 4; r++)
+            dst.store(on[2 * j + (r & 1)] && 2 * b + (r >> 1) < zleft,
+                      off + (base + (u32)(2 * j + 1 + (r & 1)) * row + (r >> 1 ? layer : 0u)), q[r]);
+        }
+    } else {
+      u32x4 top[2 * K], nx[4];
+      u32 base = 0;  // layer 2 s - 1
+#pragma unroll
+      for (int r = 0; r < 4; r++) nx[r] = src.load(off, (r & 1 ? row : 0u) + (r >> 1 ? layer : 0u));
+#pragma unroll 1
+      for (int s = 0; s <= m; s++, base += 2u * layer) {
+        u32x4 lowp, upp;
+#pragma unroll
+        for (int i = 0; i <= K; i++) {
+          u32x4 q[4];
+#pragma unroll
+          for (int r = 0; r < 4; r++) q[r] = nx[r];
+          const u32 at = i < K ? base + (u32)(2 * i + 2) * row : base + 2u * layer;
+#pragma unroll
+          for (int r = 0; r < 4; r++) nx[r] = src.load(off, at + (r & 1 ? row : 0u) + (r >> 1 ? layer : 0u));
+          __builtin_amdgcn_sched_barrier(0);
+          const u32 c = odd(q, i, s);
+          note(c, 2 * i - 1, 2 * s - 1, i == 0, i == K, s == 0, s == m);
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (MODE == kOdd) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+              const int dy = 2 * i - 1 + (r & 1), dz = 2 * s - 1 + (r >> 1);
+              if (dy >= 0 && dy < 2 * K)
+                dst.store(on[dy] && (unsigned)dz < (unsigned)min(2 * m, zleft),
+                          off + (base + (u32)(dy + 1) * row + (r >> 1 ? layer : 0u)), q[r]);
+            }
+          } else {
+            if (i > 0) {
+              if (s > 0) {
+                u32x4 v[4] = {top[2 * i - 2], top[2 * i - 1], lowp, q[0]};
+                const u32 c2 = quad_even(v, (u32)seg, variant_base((u32)(by0 + i - 1), (u32)(bz0 + s - 1), t + 1u));
+                note(c2, 2 * i - 2, 2 * s - 2, i == 1, i == K, s == 1, s == m);
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                  dst.store(on[2 * i - 2 + (r & 1)] && 2 * s - 2 + (r >> 1) < zleft,
+                            off + (base - layer + (u32)(2 * i - 1 + (r & 1)) * row + (r >> 1 ? layer : 0u)), v[r]);
+              }
+              top[2 * i - 2] = upp;
+              top[2 * i - 1] = q[2];
+            }
+            lowp = q[1];
+            upp = q[3];
+          }
+        }
+      }
+    }
+    // the first lane of each run of neighbouring items ORs the run's flags
+    acc[kXFirst] = acc[kAny] & 1u;
+    acc[kXLast] = acc[kAny] >> 31;
+    acc[kNow] = acc[kAny];
+    const u64 starts = __ballot(!has_prev);
+    const u64 after = lane < 63 ? starts >> (lane + 1) : 0ull;
+    const int len = after ? __builtin_ctzll(after) + 1 : 64 - lane;
+    const u64 run = len >= 64 ? ~0ull : (1ull << len) - 1ull;
+#pragma unroll
+    for (int f = 0; f < kFlags; f++) {
+      const u64 b = __ballot(mine && acc[f] != 0u);
+      const u64 bits = ((b >> lane) & run) << (seg & 63);
+      if (!has_prev && in && bits)
+        atomicOr((unsigned long long *)(flags + (size_t)cell * kFlags + f), (unsigned long long)bits);
     }
   }
 }
 
 // ---- bytes <-> planes --------------------------------------------------------------
+// A layer's words are contiguous, so a lane's place in the planes is its index in the
+// layer; its row, and with it its place in the bytes, takes one multiplication
+// (magic = ceil(2^32 / d), exact while the layer's index times d stays below 2^32;
+// 0 asks for a division).
+__device__ __forceinline__ u32 div_by(u32 i, u32 d, u32 magic) { return magic ? __umulhi(i, magic) : i / d; }
+
+struct LayerArgs {
+  int nx, ny, nz, lr;
+  u32 magic;  // of lr (one lane per word) or 4 lr (per quarter)
+};
+
+// First word of a layer's first row.
+__device__ __forceinline__ size_t layer_word(const LayerArgs &a, int z) {
+  return ((size_t)(z + 1) * (u32)(a.ny + 1) + 1u) * (u32)a.lr;
+}
+
 // One lane per word: 64 bytes of a row.  *reserved is set when a byte >= 4 is seen
 // (the planes hold STATIC for it).
-__global__ __launch_bounds__(256) void plane_pack_kernel(const u8 *g, u32x4 *out, int nx, int lr, size_t words,
-                                                         u32 *reserved) {
+__global__ __launch_bounds__(256) void plane_pack_kernel(const u8 *g, u32x4 *out, LayerArgs a, u32 *reserved) {
   bool any = false;
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < words; i += (size_t)gridDim.x * 256) {
-    const size_t row = i / (u32)lr;
-    const int x0 = (int)(i - row * (u32)lr) * 64, m = min(64, nx - x0);
+  const u32 i = blockIdx.x * 256u + threadIdx.x;
+  const bool in = i < (u32)a.ny * (u32)a.lr;
+  const u32 y = in ? div_by(i, (u32)a.lr, a.magic) : 0u;
+  const int x0 = in ? (int)(i - y * (u32)a.lr) * 64 : 0;
+  for (int z = (int)blockIdx.y; z < a.nz; z += (int)gridDim.y) {
     // loads may run up to 63 bytes past the last row, into the guard bytes
-    out[i] = word_from_bytes(g + row * (size_t)nx + x0, m, &any);
+    const u32x4 v = word_from_bytes(g + ((size_t)z * (u32)a.ny + y) * (u32)a.nx + (u32)x0, min(64, a.nx - x0), &any);
+    if (in) out[layer_word(a, z) + i] = v;
   }
   if (__any(any) && (threadIdx.x & 63) == 0) *reserved = 1u;
 }
 
 // Planes to bytes, four lanes per word so that a wave stores 1 KiB in a row.
-__global__ __launch_bounds__(256) void plane_unpack_kernel(const u32x4 *in, u8 *g, int nx, int lr, size_t quarters,
-                                                           const u32 *reserved) {
+__global__ __launch_bounds__(256) void plane_unpack_kernel(const u32x4 *in, u8 *g, LayerArgs a, const u32 *reserved) {
   const bool keep = *reserved != 0;
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < quarters; i += (size_t)gridDim.x * 256) {
-    const u32 qpr = 4u * (u32)lr;
-    const size_t row = i / qpr;
-    const int c = (int)(i - row * qpr), m = min(16, nx - 16 * c);
-    if (m <= 0) continue;
-    u8 *p = g + row * (size_t)nx + 16 * c;
+  const u32 i = blockIdx.x * 256u + threadIdx.x, qpr = 4u * (u32)a.lr;
+  if (i >= (u32)a.ny * qpr) return;
+  const u32 y = div_by(i, qpr, a.magic);
+  const int c = (int)(i - y * qpr), m = min(16, a.nx - 16 * c);
+  if (m <= 0) return;
+  for (int z = (int)blockIdx.y; z < a.nz; z += (int)gridDim.y) {
     u32 d[4];
-    unpack_quarter(in[i >> 2], c & 3, d);
-    store_quarter(p, m, d, keep);  // reserved cells hold their bytes (they never move)
+    unpack_quarter(in[layer_word(a, z) + (i >> 2)], c & 3, d);
+    // reserved cells hold their bytes (they never move)
+    store_quarter(g + ((size_t)z * (u32)a.ny + y) * (u32)a.nx + (u32)(16 * c), m, d, keep);
   }
 }
 
 // State hash of a plane grid, four lanes per word: each lane mixes its quarter's
 // non-empty cells.  With *reserved, STATIC cells are read from the bytes.
-__global__ __launch_bounds__(256) void plane_hash_kernel(const u32x4 *in, const u8 *g, int nx, int lr, size_t quarters,
-                                                         const u32 *reserved, u64 *parts) {
+__global__ __launch_bounds__(256) void plane_hash_kernel(const u32x4 *in, const u8 *g, LayerArgs a, const u32 *reserved,
+                                                         u64 *parts) {
   const bool bytes = *reserved != 0;
   u64 acc = 0;
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < quarters; i += (size_t)gridDim.x * 256) {
-    const u32 qpr = 4u * (u32)lr;
-    const size_t row = i / qpr;
-    const int c = (int)(i - row * qpr), m = min(16, nx - 16 * c);
-    const u64 i0 = row * (u64)nx + (u64)(16 * c);
-    acc += hash_quarter(in[i >> 2], c & 3, m, i0, bytes ? g + i0 : nullptr);
-  }
+  const u32 i = blockIdx.x * 256u + threadIdx.x, qpr = 4u * (u32)a.lr;
+  const u32 y = div_by(i, qpr, a.magic);
+  const int c = (int)(i - y * qpr);
+  const int m = i < (u32)a.ny * qpr ? min(16, a.nx - 16 * c) : 0;
+  if (m > 0)
+    for (int z = (int)blockIdx.y; z < a.nz; z += (int)gridDim.y) {
+      const u64 i0 = ((u64)z * (u32)a.ny + y) * (u32)a.nx + (u32)(16 * c);
+      acc += hash_quarter(in[layer_word(a, z) + (i >> 2)], c & 3, m, i0, bytes ? g + i0 : nullptr);
+    }
   __shared__ u64 wsum[4];
   acc = wave_sum_u64(acc);
   if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = acc;
   __syncthreads();
   if (threadIdx.x == 0) {
     const u64 tot = wsum[0] + wsum[1] + wsum[2] + wsum[3];
-    if (tot) atomicAdd((unsigned long long *)(parts + (size_t)(blockIdx.x % kHashParts) * kHashStride),
-                       (unsigned long long)tot);
+    const u32 slot = (blockIdx.y * gridDim.x + blockIdx.x) % kHashParts;
+    if (tot) atomicAdd((unsigned long long *)(parts + (size_t)slot * kHashStride), (unsigned long long)tot);
   }
 }
 
-// One cell set by the host.
-__global__ void plane_set_kernel(u32 *planes, size_t word, int x, u32 v, u32 *reserved) {
+// The rows around the grid: the layers before the first and after the last, and the
+// row between every two layers.
+__global__ __launch_bounds__(256) void plane_pad_kernel(u32x4 *p, int ny, int nz, int lr) {
+  const size_t end = (size_t)(ny + 1) * (u32)lr, mid = (size_t)nz * (u32)lr, n = 2 * end + mid + (u32)lr;
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+    size_t w;
+    if (i < end) {
+      w = i;
+    } else if (i < end + mid) {
+      const size_t k = i - end, z = k / (u32)lr;
+      w = (z + 1) * end + (k - z * (u32)lr);
+    } else {
+      w = (size_t)(nz + 1) * end + (i - end - mid);
+    }
+    p[w] = u32x4{0u, 0u, 0u, 0u};
+  }
+}
+
+// Unpacks the items changed since the bytes were last written: a wave per cell of
+// the strip grid, 16 words of a row at a time.
+__global__ __launch_bounds__(256) void plane_unpack_cells_kernel(const u32x4 *in, u8 *g, int nx, int ny, int nz, int lr,
+                                                                 int strips, int ncell, int rows, int layers,
+                                                                 const u64 *flags, u64 *since, const u32 *reserved) {
+  const int lane = threadIdx.x & 63;
+  const int c = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  if (c >= ncell) return;
+  const u64 bits = since[c] | flags[(size_t)c * kFlags + kNow];
+  if (bits == 0) return;
+  const bool keep = *reserved != 0;
+  const int zr = c / strips, st = c - zr * strips;
+  const int q = lane & 3;
+  for (int s0 = 0; s0 < lr; s0 += 16) {
+    if (((bits >> s0) & 0xFFFFull) == 0) continue;
+    const int seg = s0 + (lane >> 2);
+    const int x0 = 64 * seg + 16 * q, m = min(16, nx - x0);
+    if (seg >= lr || !((bits >> seg) & 1ull) || m <= 0) continue;
+    for (int dz = 0; dz < layers; dz++) {
+      const int z = zr * layers + dz;
+      if (z >= nz) break;
+#pragma unroll 4
+      for (int dy = 0; dy < rows; dy++) {
+        const int y = st * rows + dy;
+        if (y < ny) {
+          u32 d[4];
+          unpack_quarter(in[((size_t)(z + 1) * (u32)(ny + 1) + (u32)(y + 1)) * (u32)lr + (u32)seg], q, d);
+          store_quarter(g + ((size_t)z * (u32)ny + (u32)y) * (u32)nx + (u32)x0, m, d, keep);
+        }
+      }
+    }
+  }
+  if (lane == 0) since[c] = 0;
+}
+
+// One cell set by the host; its item counts as changed throughout (flags: the
+// item's cell of the strip grid, or nullptr).
+__global__ void plane_set_kernel(u32 *planes, size_t word, int x, u32 v, u32 *reserved, u64 *flags) {
   if (threadIdx.x != 0) return;
+  if (flags)
+    for (int i = 0; i < kFlags; i++) flags[i] |= 1ull << (x >> 6);
   if (v >= 4u) *reserved = 1u;
   const u32 code = (v >= 4u ? (u32)FS3D_STATIC : v) ^ 1u;
   u32 *w = planes + 4 * word + (x & 1);
@@ -240,8 +595,43 @@ hipError_t launch_plane_tick(const PlaneShape &ps, const void *src, void *dst, u
   return hipGetLastError();
 }
 
+// The launch shape of a pair.  Per SIMD, w resident waves of e evaluations each take
+// about e * max(0.87, 0.6 w) us (one wave alone waits for its own loads), so the
+// shape that takes the fewest evaluations is not always the fastest: long sweeps
+// evaluate fewer halo quads and leave fewer waves.  K = 2 without sharing is the
+// shape of rows too long to share (us per tick at 512^3: K = 1 unshared, zlen 2 / 4 /
+// 8: 9.7 / 9.1 / 11.3; K = 2, zlen 2 / 4 / 8: 9.5 / 10.9 / 16.8; 2048^3: K = 1, zlen
+// 16 415, K = 2, zlen 8 / 16 409 / 416, all bound by memory).
+struct PairShape {
+  int k, zlen;
+  bool share;
+};
+static PairShape pair_shape(const PlaneShape &ps) {
+  const int upw = 64 / ps.lr, nyq = (ps.ny + 1) >> 1, nzq = (ps.nz + 1) >> 1;
+  PairShape best{1, 1, false};
+  double least = 1e300;
+  for (int v = 0; v < 3; v++) {
+    const int k = v == 2 ? 2 : 1;
+    const bool share = v == 0;
+    const int adv = share ? upw - 1 : upw;  // strips per wave
+    if (adv < 1) continue;
+    const int strips = (nyq + k - 1) / k, yt = (strips + adv - 1) / adv;
+    for (int z = 1; z <= 16; z++) {
+      const double waves = (double)yt * ((nzq + z - 1) / z), w = waves / 1024.0;
+      const double evals = (double)(share ? k : k + 1) * (z + 1) + (double)k * z;
+      const double whole = w > 8.0 ? w : (double)(long long)(w + 0.999);  // the last round of few is not full
+      const double t = evals * std::max(0.87, 0.6 * whole);
+      if (t < least * 0.999) {
+        least = t;
+        best = PairShape{k, z, share};
+      }
+    }
+  }
+  return best;
+}
+
 hipError_t launch_plane_pair(const PlaneShape &ps, const void *src, void *dst, u64 t, const u64 *tick_dev, u32 k_off,
-                             int k, int zlen, hipStream_t s) {
+                             hipStream_t s) {
   PlaneArgs a{};
   fill_args(a, ps);
   a.src = static_cast<const u32x4 *>(src);
@@ -249,59 +639,135 @@ hipError_t launch_plane_pair(const PlaneShape &ps, const void *src, void *dst, u
   a.t = t;
   a.tick_dev = tick_dev;
   a.k_off = k_off;
-  a.zlen = zlen;
+  const PairShape p = pair_shape(ps);
+  a.zlen = p.zlen;
   const int nyq = (ps.ny + 1) >> 1, nzq = (ps.nz + 1) >> 1;
-  const int strips = (nyq + k - 1) / k;
-  a.ytiles = (strips + a.upw - 1) / a.upw;
-  const long long waves = (long long)a.ytiles * ((nzq + zlen - 1) / zlen);
+  const int strips = (nyq + p.k - 1) / p.k, adv = p.share ? a.upw - 1 : a.upw;
+  a.ytiles = (strips + adv - 1) / adv;
+  const long long waves = (long long)a.ytiles * ((nzq + p.zlen - 1) / p.zlen);
   const dim3 grid((unsigned)((waves + 3) / 4));
   const bool wall = ps.nx % 64 == 0;
-  switch (k) {
-    case 1:
-      if (wall) hipLaunchKernelGGL((plane_pair_kernel<true, 1>), grid, dim3(256), 0, s, a);
-      else hipLaunchKernelGGL((plane_pair_kernel<false, 1>), grid, dim3(256), 0, s, a);
-      break;
-    case 2:
-      if (wall) hipLaunchKernelGGL((plane_pair_kernel<true, 2>), grid, dim3(256), 0, s, a);
-      else hipLaunchKernelGGL((plane_pair_kernel<false, 2>), grid, dim3(256), 0, s, a);
-      break;
-    default:
-      if (wall) hipLaunchKernelGGL((plane_pair_kernel<true, 4>), grid, dim3(256), 0, s, a);
-      else hipLaunchKernelGGL((plane_pair_kernel<false, 4>), grid, dim3(256), 0, s, a);
-      break;
+  if (p.share) {
+    if (wall) hipLaunchKernelGGL((plane_pair_kernel<true, 1, true>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((plane_pair_kernel<false, 1, true>), grid, dim3(256), 0, s, a);
+  } else if (p.k == 1) {
+    if (wall) hipLaunchKernelGGL((plane_pair_kernel<true, 1, false>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((plane_pair_kernel<false, 1, false>), grid, dim3(256), 0, s, a);
+  } else {
+    if (wall) hipLaunchKernelGGL((plane_pair_kernel<true, 2, false>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((plane_pair_kernel<false, 2, false>), grid, dim3(256), 0, s, a);
   }
   return hipGetLastError();
 }
 
+PlaneCells plane_cells(const PlaneShape &ps) {
+  PlaneCells c;
+  c.strips = (((ps.ny + 1) >> 1) + kItemQuads - 1) / kItemQuads;
+  c.zcells = (((ps.nz + 1) >> 1) + kItemLayers - 1) / kItemLayers;
+  c.virt = ps.nx % 64 == 0 ? 1 : 0;
+  const size_t n = (size_t)c.strips * (size_t)c.zcells;
+  c.flag_words = n * kFlags;
+  c.since_words = n;
+  c.list_words = n * (size_t)(ps.lr + c.virt);
+  return c;
+}
+
+int plane_list_blocks_per_cu() {
+  int n = 0;
+  const hipError_t e =
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, plane_list_kernel<kPair, kItemQuads>, 256, 0);
+  return e == hipSuccess && n > 0 ? n : 1;
+}
+
+hipError_t launch_plane_list(const PlaneShape &ps, const void *src, void *dst, u64 t, const u64 *tick_dev, u32 k_off,
+                             bool pair, bool fresh, const u64 *flags_in, u64 *flags_out, u64 *since, u32 *list,
+                             u32 *count, u32 nwaves, hipStream_t s) {
+  PlaneArgs a{};
+  fill_args(a, ps);
+  a.src = static_cast<const u32x4 *>(src);
+  a.dst = static_cast<u32x4 *>(dst);
+  a.t = t;
+  a.tick_dev = tick_dev;
+  a.k_off = k_off;
+  a.zlen = kItemLayers;
+  const PlaneCells c = plane_cells(ps);
+  const unsigned plan = (unsigned)((c.since_words + 255) / 256);
+  hipError_t e = launch_fill_u32(count, 1, 0, s);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(plane_plan_kernel, dim3(plan), dim3(256), 0, s, flags_in, flags_out, since, c.strips, c.zcells,
+                     ps.lr, c.virt, pair ? 0 : 1, fresh ? 1 : 0, list, count);
+  const dim3 grid(nwaves / 4);
+  // the caller's t has the tick's parity, on replays too
+  if (pair)
+    hipLaunchKernelGGL((plane_list_kernel<kPair, kItemQuads>), grid, dim3(256), 0, s, a, list, count, flags_out,
+                       c.strips, c.virt, nwaves);
+  else if (t & 1u)
+    hipLaunchKernelGGL((plane_list_kernel<kOdd, kItemQuads>), grid, dim3(256), 0, s, a, list, count, flags_out,
+                       c.strips, c.virt, nwaves);
+  else
+    hipLaunchKernelGGL((plane_list_kernel<kEven, kItemQuads>), grid, dim3(256), 0, s, a, list, count, flags_out,
+                       c.strips, c.virt, nwaves);
+  return hipGetLastError();
+}
+
+hipError_t launch_plane_unpack_cells(const PlaneShape &ps, const void *planes, u8 *g, const u64 *flags, u64 *since,
+                                     const u32 *reserved, hipStream_t s) {
+  const PlaneCells c = plane_cells(ps);
+  const int ncell = (int)c.since_words;
+  hipLaunchKernelGGL(plane_unpack_cells_kernel, dim3((unsigned)((ncell + 3) / 4)), dim3(256), 0, s,
+                     static_cast<const u32x4 *>(planes), g, ps.nx, ps.ny, ps.nz, ps.lr, c.strips, ncell,
+                     2 * kItemQuads, 2 * kItemLayers, flags, since, reserved);
+  return hipGetLastError();
+}
+
+// per: lanes per word.  Layers per lane: enough blocks for the chip, few enough that
+// the row's division and a hash's reduction are shared by several layers.
+static LayerArgs layer_args(const PlaneShape &ps, int per, dim3 *grid) {
+  const u64 d = (u64)per * (u64)ps.lr, n = d * (u64)ps.ny;
+  LayerArgs a{ps.nx, ps.ny, ps.nz, ps.lr, 0};
+  if (n * d < (1ull << 32) && d > 1) a.magic = (u32)(((1ull << 32) + d - 1) / d);
+  const unsigned gx = (unsigned)((n + 255) / 256);
+  const unsigned gy = (unsigned)std::min<u64>((u64)std::min(ps.nz, 65535), std::max<u64>(1, 16384 / std::max(gx, 1u)));
+  *grid = dim3(gx, gy);
+  return a;
+}
+
+hipError_t launch_plane_pad(const PlaneShape &ps, void *planes, hipStream_t s) {
+  const size_t n = ((size_t)2 * (u32)(ps.ny + 1) + (u32)ps.nz + 1) * (u32)ps.lr;
+  hipLaunchKernelGGL(plane_pad_kernel, dim3((unsigned)std::min<size_t>((n + 255) / 256, 4096)), dim3(256), 0, s,
+                     static_cast<u32x4 *>(planes), ps.ny, ps.nz, ps.lr);
+  return hipGetLastError();
+}
+
 hipError_t launch_plane_pack(const PlaneShape &ps, const u8 *g, void *planes, u32 *reserved, hipStream_t s) {
-  const size_t words = plane_words(ps);
-  const unsigned grid = (unsigned)std::min<size_t>((words + 255) / 256, 1u << 20);
-  hipLaunchKernelGGL(plane_pack_kernel, dim3(grid), dim3(256), 0, s, g, static_cast<u32x4 *>(planes), ps.nx, ps.lr,
-                     words, reserved);
+  dim3 grid;
+  const LayerArgs a = layer_args(ps, 1, &grid);
+  hipLaunchKernelGGL(plane_pack_kernel, grid, dim3(256), 0, s, g, static_cast<u32x4 *>(planes), a, reserved);
   return hipGetLastError();
 }
 
 hipError_t launch_plane_unpack(const PlaneShape &ps, const void *planes, u8 *g, const u32 *reserved, hipStream_t s) {
-  const size_t quarters = 4 * plane_words(ps);
-  const unsigned grid = (unsigned)std::min<size_t>((quarters + 255) / 256, 1u << 20);
-  hipLaunchKernelGGL(plane_unpack_kernel, dim3(grid), dim3(256), 0, s, static_cast<const u32x4 *>(planes), g, ps.nx,
-                     ps.lr, quarters, reserved);
+  dim3 grid;
+  const LayerArgs a = layer_args(ps, 4, &grid);
+  hipLaunchKernelGGL(plane_unpack_kernel, grid, dim3(256), 0, s, static_cast<const u32x4 *>(planes), g, a, reserved);
   return hipGetLastError();
 }
 
 hipError_t launch_plane_hash(const PlaneShape &ps, const void *planes, const u8 *g, const u32 *reserved, u64 *parts,
                              hipStream_t s) {
-  const size_t quarters = 4 * plane_words(ps);
-  const unsigned grid = (unsigned)std::min<size_t>((quarters + 255) / 256, 8192);
-  hipLaunchKernelGGL(plane_hash_kernel, dim3(grid), dim3(256), 0, s, static_cast<const u32x4 *>(planes), g, ps.nx,
-                     ps.lr, quarters, reserved, parts);
+  dim3 grid;
+  const LayerArgs a = layer_args(ps, 4, &grid);
+  hipLaunchKernelGGL(plane_hash_kernel, grid, dim3(256), 0, s, static_cast<const u32x4 *>(planes), g, a, reserved,
+                     parts);
   return hipGetLastError();
 }
 
-hipError_t launch_plane_set(const PlaneShape &ps, void *planes, int x, int y, int z, u8 v, u32 *reserved,
+hipError_t launch_plane_set(const PlaneShape &ps, void *planes, int x, int y, int z, u8 v, u32 *reserved, u64 *flags,
                             hipStream_t s) {
-  const size_t word = ((size_t)z * ps.ny + y) * ps.lr + (size_t)(x >> 6);
-  hipLaunchKernelGGL(plane_set_kernel, dim3(1), dim3(64), 0, s, static_cast<u32 *>(planes), word, x, (u32)v, reserved);
+  const size_t word = ((size_t)(z + 1) * (u32)(ps.ny + 1) + (u32)(y + 1)) * (u32)ps.lr + (u32)(x >> 6);
+  const size_t cell = (size_t)(z / (2 * kItemLayers)) * plane_cells(ps).strips + (size_t)(y / (2 * kItemQuads));
+  hipLaunchKernelGGL(plane_set_kernel, dim3(1), dim3(64), 0, s, static_cast<u32 *>(planes), word, x, (u32)v, reserved,
+                     flags ? flags + cell * kFlags : nullptr);
   return hipGetLastError();
 }
 

@@ -17,18 +17,27 @@ using tickcore::wave_sum_u64;
 
 // A plane grid as a buffer: loads out of range read 0 (STATIC), stores out of
 // range are dropped, so rows outside the grid need no branches.
+constexpr u32 kOutside = 0xFFFFFFF0u;  // an offset beyond every grid
+
 struct Planes {
   __amdgpu_buffer_rsrc_t rsrc;
+  u32 last;  // offset of the last word
   __device__ __forceinline__ Planes(const void *p, u32 bytes)
-      : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00020000)) {}
-  __device__ __forceinline__ u32x4 load(u32 off) const {
-    return __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off, 0, 0);
+      : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00020000)), last(bytes - 16u) {}
+  // A lane's offset plus a wave-uniform one; 0 beyond the buffer.  The range check
+  // compares `off` with the buffer's size minus the scalar offset, which must not
+  // exceed it (`last` is a word of zeros, like everything beyond).
+  __device__ __forceinline__ u32x4 load(u32 off, u32 uniform = 0) const {
+    return __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off, (int)(uniform < last ? uniform : last), 0);
   }
+  // Stored without a scalar offset: with one, a vector instruction that
+  // rewrites the data's registers right behind a 16-byte store has changed what was
+  // stored, and the compiler keeps the two apart only for stores that have none.
   __device__ __forceinline__ void store(u32 off, u32x4 v) const {
     __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, (int)off, 0, 0);
   }
+  __device__ __forceinline__ void store(bool on, u32 off, u32x4 v) const { store(on ? off : kOutside, v); }
 };
-constexpr u32 kOutside = 0xFFFFFFF0u;  // an offset beyond every grid
 
 __device__ __forceinline__ u32 from_lane(int addr, u32 v) { return (u32)__builtin_amdgcn_ds_bpermute(addr, (int)v); }
 
