@@ -328,10 +328,17 @@ int enqueue_planes(fs3d_world *w, int nticks, int hash_every, const u64 *tick_de
   if (launch && items && fresh)
     FS3D_HIP(launch_fill_u64(w->pflags[f], plane_cells(ps).flag_words, ~0ull, w->stream));
   auto hashed_after = [&](int k) { return hash_every > 0 && (k + 1) % hash_every == 0; };
+  const bool direct = plane_hash_direct(ps);
+  if (launch && direct && hash_every > 0 && nticks >= hash_every)
+    FS3D_HIP(launch_fill_u64(w->d_small + 1, (size_t)(nticks / hash_every), 0, w->stream));
+  PlaneHash hash{w->buf[w->cur], w->d_reserved, w->d_parts, nullptr};  // out: due for planes[src]
   for (int k = 0; k < nticks;) {
     const u64 t = w->tick + (u64)k;
     const bool pair = (t & 1u) && k + 1 < nticks && !hashed_after(k);
     if (launch) {
+      // a single tick hashes the state that it reads
+      const bool with = hash.out && !items && !pair;
+      if (hash.out && !with) FS3D_HIP(launch_plane_hash(ps, w->planes[src], hash, w->stream));
       if (items)
         FS3D_HIP(launch_plane_list(ps, w->planes[src], w->planes[src ^ 1], t, tick_dev, (u32)k, pair, fresh,
                                    w->pflags[f], w->pflags[f ^ 1], w->d_since, w->d_items, w->d_nitems,
@@ -339,16 +346,19 @@ int enqueue_planes(fs3d_world *w, int nticks, int hash_every, const u64 *tick_de
       else if (pair)
         FS3D_HIP(launch_plane_pair(ps, w->planes[src], w->planes[src ^ 1], t, tick_dev, (u32)k, w->stream));
       else
-        FS3D_HIP(launch_plane_tick(ps, w->planes[src], w->planes[src ^ 1], t, tick_dev, (u32)k, w->stream));
+        FS3D_HIP(launch_plane_tick(ps, w->planes[src], w->planes[src ^ 1], t, tick_dev, (u32)k,
+                                   with ? &hash : nullptr, w->stream));
+      if (hash.out && !direct) FS3D_HIP(launch_hash_finalize(w->d_parts, hash.out, w->stream));
     }
     src ^= 1;
     f ^= 1;
     fresh = false;
     k += pair ? 2 : 1;
-    if (launch && hashed_after(k - 1)) {
-      FS3D_HIP(launch_plane_hash(ps, w->planes[src], w->buf[w->cur], w->d_reserved, w->d_parts, w->stream));
-      FS3D_HIP(launch_hash_finalize(w->d_parts, w->d_small + k / hash_every, w->stream));
-    }
+    hash.out = hashed_after(k - 1) ? w->d_small + k / hash_every : nullptr;
+  }
+  if (launch && hash.out) {
+    FS3D_HIP(launch_plane_hash(ps, w->planes[src], hash, w->stream));
+    if (!direct) FS3D_HIP(launch_hash_finalize(w->d_parts, hash.out, w->stream));
   }
   if (launch) {
     if (items)

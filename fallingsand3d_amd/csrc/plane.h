@@ -32,9 +32,19 @@ struct PlaneArgs {
   int zlen, ytiles;  // pairs: z row-quads per wave, waves along y
 };
 
-// One tick, any parity.
+// State hash of a grid; g holds the bytes of reserved cells.  With plane_hash_direct
+// it is added to *out, otherwise to the partial sums, which launch_hash_finalize adds
+// up.
+struct PlaneHash {
+  const u8 *g;
+  const u32 *reserved;
+  u64 *parts, *out;
+};
+bool plane_hash_direct(const PlaneShape &ps);
+hipError_t launch_plane_hash(const PlaneShape &ps, const void *planes, const PlaneHash &hash, hipStream_t s);
+// One tick, any parity, and the hash of src when asked for.
 hipError_t launch_plane_tick(const PlaneShape &ps, const void *src, void *dst, u64 t, const u64 *tick_dev, u32 k_off,
-                             hipStream_t s);
+                             const PlaneHash *hash, hipStream_t s);
 // Ticks t and t + 1, t odd.
 hipError_t launch_plane_pair(const PlaneShape &ps, const void *src, void *dst, u64 t, const u64 *tick_dev, u32 k_off,
                              hipStream_t s);
@@ -45,9 +55,6 @@ hipError_t launch_plane_pad(const PlaneShape &ps, void *planes, hipStream_t s);
 hipError_t launch_plane_pack(const PlaneShape &ps, const u8 *g, void *planes, u32 *reserved, hipStream_t s);
 hipError_t launch_plane_unpack(const PlaneShape &ps, const void *planes, u8 *g, const u32 *reserved, hipStream_t s);
 
-// State hash of the grid into the partial sums; g holds the bytes of reserved cells.
-hipError_t launch_plane_hash(const PlaneShape &ps, const void *planes, const u8 *g, const u32 *reserved, u64 *parts,
-                             hipStream_t s);
 // One cell of planes, and of its item's change flags when given.
 hipError_t launch_plane_set(const PlaneShape &ps, void *planes, int x, int y, int z, u8 v, u32 *reserved, u64 *flags,
                             hipStream_t s);

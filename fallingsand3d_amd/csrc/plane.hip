@@ -51,16 +51,88 @@ __device__ __forceinline__ Lane lane_of(const PlaneArgs &a, int first_unit, int 
   return L;
 }
 
+// A layer's words are contiguous, so a lane's place in the planes is its index in the
+// layer; its row, and with it its place in the bytes, takes one multiplication
+// (magic = ceil(2^32 / d), exact while the layer's index times d stays below 2^32;
+// 0 asks for a division).
+__device__ __forceinline__ u32 div_by(u32 i, u32 d, u32 magic) { return magic ? __umulhi(i, magic) : i / d; }
+
+struct LayerArgs {
+  int nx, ny, nz, lr;
+  u32 magic;  // of lr (one lane per word) or 4 lr (per quarter)
+};
+
+// First word of a layer's first row.
+__device__ __forceinline__ size_t layer_word(const LayerArgs &a, int z) {
+  return ((size_t)(z + 1) * (u32)(a.ny + 1) + 1u) * (u32)a.lr;
+}
+
+// ---- state hash --------------------------------------------------------------------
+// Four lanes per word, each mixing its quarter's non-empty cells, or 16 lanes in a
+// small grid.  With *reserved, STATIC cells are read from the bytes.  Workgroup
+// `block` of gx * gy adds its sum to one of the slots, which start at 0.
+//
+// Bound by the mixing, about 190 cycles per 64 cells (two 64-bit products at a quarter
+// of the rate): 117 us at 512^3 with 35 % of the cells not empty.  In a small grid a
+// lane's chain of mixes is what takes the time: a hashed tick of 64^3 takes 4.6 us
+// with four lanes per word and 3.6 with 16; of 256 x 120 x 60, where there are waves
+// enough, 5.2 and 7.7.
+constexpr size_t kSplitHashWords = 1u << 13;  // with 16 lanes per word up to here
+struct HashArgs {
+  LayerArgs l;
+  const u32x4 *in;
+  const u8 *g;
+  const u32 *reserved;
+  u64 *out;  // slots sums, kHashStride apart
+  u32 gx, gy, slots;
+  int split;  // lanes per quarter (1 or 4)
+};
+
+__device__ __forceinline__ void hash_block(const HashArgs &h, u32 block) {
+  const LayerArgs &a = h.l;
+  const bool bytes = *h.reserved != 0;
+  const u32 by = block / h.gx, bx = block - by * h.gx;
+  u64 acc = 0;
+  const u32 lane = bx * 256u + threadIdx.x, qpr = 4u * (u32)a.lr;
+  const u32 i = h.split == 4 ? lane >> 2 : lane, cells = h.split == 4 ? 0xFu << 4 * (lane & 3u) : 0xFFFFu;
+  const u32 y = div_by(i, qpr, a.magic);
+  const int c = (int)(i - y * qpr);
+  const int m = i < (u32)a.ny * qpr ? min(16, a.nx - 16 * c) : 0;
+  if (m > 0)
+    for (int z = (int)by; z < a.nz; z += (int)h.gy) {
+      const u64 i0 = ((u64)z * (u32)a.ny + y) * (u32)a.nx + (u32)(16 * c);
+      acc += hash_quarter(h.in[layer_word(a, z) + (i >> 2)], c & 3, m, i0, bytes ? h.g + i0 : nullptr, cells);
+    }
+  __shared__ u64 wsum[4];
+  acc = wave_sum_u64(acc);
+  if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const u64 tot = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+    if (tot)
+      atomicAdd((unsigned long long *)(h.out + (size_t)(block % h.slots) * kHashStride), (unsigned long long)tot);
+  }
+}
+
+__global__ __launch_bounds__(256) void plane_hash_kernel(HashArgs h) { hash_block(h, blockIdx.x); }
+
 // ---- single tick ----------------------------------------------------------------
+// The first hash_blocks workgroups hash the state that the tick reads: a run that is
+// hashed after every tick takes one launch per tick instead of three (tick, partial
+// sums, their sum): 3.6 us per tick instead of 9.1 at 64^3.
 template <bool WALL>
-__global__ __launch_bounds__(256) void plane_tick_kernel(PlaneArgs a) {
+__global__ __launch_bounds__(256) void plane_tick_kernel(PlaneArgs a, HashArgs h, u32 hash_blocks, u32 tx) {
+  if (blockIdx.x < hash_blocks) {
+    hash_block(h, blockIdx.x);
+    return;
+  }
+  const u32 block = blockIdx.x - hash_blocks, bz = block / tx, bx = block - bz * tx;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const u64 t64 = tick_of(a);
   const u32 t = (u32)t64;
   const int p = (int)(t & 1u);
   const int nyq = (a.ny + p + 1) >> 1, nzq = (a.nz + p + 1) >> 1;
-  const int first = ((int)blockIdx.x * 4 + wv) * a.upw;
-  const int zq = (int)blockIdx.z * 65535 + (int)blockIdx.y;
+  const int first = ((int)bx * 4 + wv) * a.upw, zq = (int)bz;
   if (__builtin_amdgcn_readfirstlane(first) >= nyq || zq >= nzq) return;
   const Lane L = lane_of(a, first, lane);
   const Planes src(a.src, a.bytes), dst(a.dst, a.bytes);
@@ -425,22 +497,6 @@ __global__ __launch_bounds__(256) void plane_list_kernel(PlaneArgs a, const u32 
 }
 
 // ---- bytes <-> planes --------------------------------------------------------------
-// A layer's words are contiguous, so a lane's place in the planes is its index in the
-// layer; its row, and with it its place in the bytes, takes one multiplication
-// (magic = ceil(2^32 / d), exact while the layer's index times d stays below 2^32;
-// 0 asks for a division).
-__device__ __forceinline__ u32 div_by(u32 i, u32 d, u32 magic) { return magic ? __umulhi(i, magic) : i / d; }
-
-struct LayerArgs {
-  int nx, ny, nz, lr;
-  u32 magic;  // of lr (one lane per word) or 4 lr (per quarter)
-};
-
-// First word of a layer's first row.
-__device__ __forceinline__ size_t layer_word(const LayerArgs &a, int z) {
-  return ((size_t)(z + 1) * (u32)(a.ny + 1) + 1u) * (u32)a.lr;
-}
-
 // One lane per word: 64 bytes of a row.  *reserved is set when a byte >= 4 is seen
 // (the planes hold STATIC for it).
 __global__ __launch_bounds__(256) void plane_pack_kernel(const u8 *g, u32x4 *out, LayerArgs a, u32 *reserved) {
@@ -470,32 +526,6 @@ __global__ __launch_bounds__(256) void plane_unpack_kernel(const u32x4 *in, u8 *
     unpack_quarter(in[layer_word(a, z) + (i >> 2)], c & 3, d);
     // reserved cells hold their bytes (they never move)
     store_quarter(g + ((size_t)z * (u32)a.ny + y) * (u32)a.nx + (u32)(16 * c), m, d, keep);
-  }
-}
-
-// State hash of a plane grid, four lanes per word: each lane mixes its quarter's
-// non-empty cells.  With *reserved, STATIC cells are read from the bytes.
-__global__ __launch_bounds__(256) void plane_hash_kernel(const u32x4 *in, const u8 *g, LayerArgs a, const u32 *reserved,
-                                                         u64 *parts) {
-  const bool bytes = *reserved != 0;
-  u64 acc = 0;
-  const u32 i = blockIdx.x * 256u + threadIdx.x, qpr = 4u * (u32)a.lr;
-  const u32 y = div_by(i, qpr, a.magic);
-  const int c = (int)(i - y * qpr);
-  const int m = i < (u32)a.ny * qpr ? min(16, a.nx - 16 * c) : 0;
-  if (m > 0)
-    for (int z = (int)blockIdx.y; z < a.nz; z += (int)gridDim.y) {
-      const u64 i0 = ((u64)z * (u32)a.ny + y) * (u32)a.nx + (u32)(16 * c);
-      acc += hash_quarter(in[layer_word(a, z) + (i >> 2)], c & 3, m, i0, bytes ? g + i0 : nullptr);
-    }
-  __shared__ u64 wsum[4];
-  acc = wave_sum_u64(acc);
-  if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = acc;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const u64 tot = wsum[0] + wsum[1] + wsum[2] + wsum[3];
-    const u32 slot = (blockIdx.y * gridDim.x + blockIdx.x) % kHashParts;
-    if (tot) atomicAdd((unsigned long long *)(parts + (size_t)slot * kHashStride), (unsigned long long)tot);
   }
 }
 
@@ -577,8 +607,37 @@ static void fill_args(PlaneArgs &a, const PlaneShape &ps) {
   a.lr_magic = (65536u + (u32)ps.lr - 1u) / (u32)ps.lr;
 }
 
+// per: lanes per word.  Layers per lane: enough blocks for the chip, few enough that
+// the row's division and a hash's reduction are shared by several layers.
+static LayerArgs layer_args(const PlaneShape &ps, int per, dim3 *grid) {
+  const u64 d = (u64)per * (u64)ps.lr, n = d * (u64)ps.ny;
+  LayerArgs a{ps.nx, ps.ny, ps.nz, ps.lr, 0};
+  if (n * d < (1ull << 32) && d > 1) a.magic = (u32)(((1ull << 32) + d - 1) / d);
+  const unsigned gx = (unsigned)((n + 255) / 256);
+  const unsigned gy = (unsigned)std::min<u64>((u64)std::min(ps.nz, 65535), std::max<u64>(1, 16384 / std::max(gx, 1u)));
+  *grid = dim3(gx, gy);
+  return a;
+}
+
+static HashArgs hash_args(const PlaneShape &ps, const PlaneHash &ph, const void *planes) {
+  dim3 grid;
+  HashArgs h{};
+  h.l = layer_args(ps, 4, &grid);
+  h.in = static_cast<const u32x4 *>(planes);
+  h.g = ph.g;
+  h.reserved = ph.reserved;
+  h.gx = grid.x;
+  h.gy = grid.y;
+  const bool direct = plane_hash_direct(ps);
+  h.split = plane_words(ps) <= kSplitHashWords ? 4 : 1;
+  if (h.split == 4) h.gx = (unsigned)(((size_t)16 * (u32)ps.lr * (u32)ps.ny + 255) / 256);
+  h.out = direct ? ph.out : ph.parts;
+  h.slots = direct ? 1 : kHashParts;
+  return h;
+}
+
 hipError_t launch_plane_tick(const PlaneShape &ps, const void *src, void *dst, u64 t, const u64 *tick_dev, u32 k_off,
-                             hipStream_t s) {
+                             const PlaneHash *hash, hipStream_t s) {
   PlaneArgs a{};
   fill_args(a, ps);
   a.src = static_cast<const u32x4 *>(src);
@@ -587,11 +646,18 @@ hipError_t launch_plane_tick(const PlaneShape &ps, const void *src, void *dst, u
   a.tick_dev = tick_dev;
   a.k_off = k_off;
   const int nyq = (ps.ny + 2) >> 1, nzq = (ps.nz + 2) >> 1, per = 4 * a.upw;
-  const dim3 grid((unsigned)((nyq + per - 1) / per), (unsigned)std::min(nzq, 65535), (unsigned)((nzq + 65534) / 65535));
+  const u32 tx = (u32)((nyq + per - 1) / per);
+  HashArgs h{};
+  u32 hb = 0;
+  if (hash) {
+    h = hash_args(ps, *hash, src);
+    hb = h.gx * h.gy;
+  }
+  const dim3 grid(hb + tx * (u32)nzq);
   if (ps.nx % 64 == 0)
-    hipLaunchKernelGGL(plane_tick_kernel<true>, grid, dim3(256), 0, s, a);
+    hipLaunchKernelGGL(plane_tick_kernel<true>, grid, dim3(256), 0, s, a, h, hb, tx);
   else
-    hipLaunchKernelGGL(plane_tick_kernel<false>, grid, dim3(256), 0, s, a);
+    hipLaunchKernelGGL(plane_tick_kernel<false>, grid, dim3(256), 0, s, a, h, hb, tx);
   return hipGetLastError();
 }
 
@@ -660,6 +726,10 @@ hipError_t launch_plane_pair(const PlaneShape &ps, const void *src, void *dst, u
   return hipGetLastError();
 }
 
+// 512 workgroups at most add to one word; each addition takes it 13 ns (16384 at 512^3
+// made the hash 210 us instead of 117).
+bool plane_hash_direct(const PlaneShape &ps) { return plane_words(ps) <= (1u << 15); }
+
 PlaneCells plane_cells(const PlaneShape &ps) {
   PlaneCells c;
   c.strips = (((ps.ny + 1) >> 1) + kItemQuads - 1) / kItemQuads;
@@ -720,18 +790,6 @@ hipError_t launch_plane_unpack_cells(const PlaneShape &ps, const void *planes, u
   return hipGetLastError();
 }
 
-// per: lanes per word.  Layers per lane: enough blocks for the chip, few enough that
-// the row's division and a hash's reduction are shared by several layers.
-static LayerArgs layer_args(const PlaneShape &ps, int per, dim3 *grid) {
-  const u64 d = (u64)per * (u64)ps.lr, n = d * (u64)ps.ny;
-  LayerArgs a{ps.nx, ps.ny, ps.nz, ps.lr, 0};
-  if (n * d < (1ull << 32) && d > 1) a.magic = (u32)(((1ull << 32) + d - 1) / d);
-  const unsigned gx = (unsigned)((n + 255) / 256);
-  const unsigned gy = (unsigned)std::min<u64>((u64)std::min(ps.nz, 65535), std::max<u64>(1, 16384 / std::max(gx, 1u)));
-  *grid = dim3(gx, gy);
-  return a;
-}
-
 hipError_t launch_plane_pad(const PlaneShape &ps, void *planes, hipStream_t s) {
   const size_t n = ((size_t)2 * (u32)(ps.ny + 1) + (u32)ps.nz + 1) * (u32)ps.lr;
   hipLaunchKernelGGL(plane_pad_kernel, dim3((unsigned)std::min<size_t>((n + 255) / 256, 4096)), dim3(256), 0, s,
@@ -753,12 +811,9 @@ hipError_t launch_plane_unpack(const PlaneShape &ps, const void *planes, u8 *g, 
   return hipGetLastError();
 }
 
-hipError_t launch_plane_hash(const PlaneShape &ps, const void *planes, const u8 *g, const u32 *reserved, u64 *parts,
-                             hipStream_t s) {
-  dim3 grid;
-  const LayerArgs a = layer_args(ps, 4, &grid);
-  hipLaunchKernelGGL(plane_hash_kernel, grid, dim3(256), 0, s, static_cast<const u32x4 *>(planes), g, a, reserved,
-                     parts);
+hipError_t launch_plane_hash(const PlaneShape &ps, const void *planes, const PlaneHash &hash, hipStream_t s) {
+  const HashArgs h = hash_args(ps, hash, planes);
+  hipLaunchKernelGGL(plane_hash_kernel, dim3(h.gx * h.gy), dim3(256), 0, s, h);
   return hipGetLastError();
 }
 

@@ -161,12 +161,14 @@ __device__ __forceinline__ void store_quarter(u8 *p, int m, u32 (&d)[4], bool ke
 // A quarter's share of the state hash: its first m cells, the first of them cell
 // i0 of the grid; with `bytes`, STATIC cells are read from there (the quarter's
 // bytes), where reserved ones keep their values.
-__device__ __forceinline__ u64 hash_quarter(const u32x4 &v, int q, int m, u64 i0, const u8 *bytes) {
+// (`cells`: the ones to mix, a bit each.)
+__device__ __forceinline__ u64 hash_quarter(const u32x4 &v, int q, int m, u64 i0, const u8 *bytes,
+                                            u32 cells = 0xFFFFu) {
   // pairs 8q .. 8q + 7 sit 2 bits apart: even cells in place, odd ones beside them
   const int sh = 16 * (q & 1) + (q >> 1);
   const u32 x = ((v.x >> sh) & 0x5555u) | (((v.y >> sh) & 0x5555u) << 1);
   const u32 h = ((v.z >> sh) & 0x5555u) | (((v.w >> sh) & 0x5555u) << 1);
-  u32 ne = (~x | h) & (m >= 16 ? 0xFFFFu : m > 0 ? (1u << m) - 1u : 0u);
+  u32 ne = (~x | h) & cells & (m >= 16 ? 0xFFFFu : m > 0 ? (1u << m) - 1u : 0u);
   u64 acc = 0;
   while (ne) {
     const int k = __builtin_ctz(ne);
