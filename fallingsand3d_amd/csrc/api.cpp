@@ -11,6 +11,7 @@
 
 #include "fs3d_internal.h"
 #include "fs3d_render.h"
+#include "hostcopy.h"
 #include "plane.h"
 
 namespace fs3d {
@@ -132,6 +133,7 @@ void release(fs3d_world *w) {
   if (w->ev0) (void)hipEventDestroy(w->ev0);
   if (w->ev1) (void)hipEventDestroy(w->ev1);
   if (w->stream) (void)hipStreamDestroy(w->stream);
+  hostcopy_world(-1);
   delete w;
 }
 
@@ -536,6 +538,7 @@ int fs3d_world_create(const int32_t dims[3], uint32_t flags, fs3d_world **out) {
   int rc = ensure_device(dev);
   if (rc) return rc;
   fs3d_world *w = new fs3d_world();
+  hostcopy_world(1);
   w->dev = dev;
   w->nx = dims[0];
   w->ny = dims[1];
@@ -647,8 +650,7 @@ int fs3d_world_download(fs3d_world *w, uint8_t *host, size_t nbytes) {
   if (int rc = check_world(w)) return rc;
   if (!host || nbytes != w->n) return set_error(FS3D_ERR_INVALID, "download needs %zu bytes (got %zu)", w->n, nbytes);
   FS3D_HIP(hipSetDevice(w->dev));
-  FS3D_HIP(hipMemcpyAsync(host, w->buf[w->cur], w->n, hipMemcpyDeviceToHost, w->stream));
-  FS3D_HIP(hipStreamSynchronize(w->stream));
+  FS3D_HIP(copy_to_host({{host, w->buf[w->cur], w->n}}, w->dev, w->stream));
   return clear_error();
 }
 

@@ -2,6 +2,7 @@
 #pragma once
 
 #include "fs3d_internal.h"
+#include "hostcopy.h"
 
 namespace fs3d {
 
@@ -15,7 +16,9 @@ struct RenderCam {
   float aspect;
 };
 
-hipError_t launch_sdf(const float cam_pos[3], float aspect, int W, int H, float *d_rgba, hipStream_t s);
+// Pixels first, first + 1, ... of the W x H image to pinned memory.
+hipError_t launch_sdf(const float cam_pos[3], float aspect, int W, int H, size_t first, const PieceOut &out,
+                      hipStream_t s);
 // u64 words of a grid's occupancy maps: the coarse map (one bit per 8x8x8
 // brick, 64 bricks per word along x) followed by the fine map (one word per
 // brick, one bit per 2x2x2 sub-brick).

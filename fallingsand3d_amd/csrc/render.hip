@@ -33,6 +33,7 @@ __constant__ u32 kPaletteBits[1024] = {
 };
 
 typedef u32 u32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef u32x2 __attribute__((aligned(1))) u32x2_u;  // rows start at any byte
 
 struct F3 {
@@ -58,11 +59,7 @@ __device__ __forceinline__ F3 pixel_dir(int px, int py, int W, int H, float aspe
 
 __device__ __forceinline__ float sdf_map(float x, float y, float z) { return sqrtf((x * x + y * y) + z * z) - 0.5f; }
 
-__global__ __launch_bounds__(256) void sdf_kernel(float ox, float oy, float oz, float aspect, int W, int H,
-                                                  float *rgba) {
-  const int px = blockIdx.x * 16 + (threadIdx.x & 15), py = blockIdx.y * 16 + (threadIdx.x >> 4);
-  if (px >= W || py >= H) return;
-  const F3 d = pixel_dir(px, py, W, H, aspect);
+__device__ __forceinline__ f32x4 sdf_pixel(float ox, float oy, float oz, F3 d) {
   float r = 0.0f, gg = 0.0f, b = 0.0f;
   float t = 0.0f;
   for (int i = 0; i < 64; i++) {
@@ -85,11 +82,20 @@ __global__ __launch_bounds__(256) void sdf_kernel(float ox, float oy, float oz, 
     }
     t = t + dist;
   }
-  float *out = rgba + ((size_t)py * W + px) * 4;
-  out[0] = r;
-  out[1] = gg;
-  out[2] = b;
-  out[3] = 1.0f;
+  return f32x4{r, gg, b, 1.0f};
+}
+
+// A lane per pixel: a workgroup marches kBlockBytes of the image.
+__global__ __launch_bounds__(1024) void sdf_kernel(float ox, float oy, float oz, float aspect, int W, int H, u64 first,
+                                                  PieceOut o) {
+  const PinnedOut out(o.buf, o.n);
+  const u32 off = blockIdx.x * kBlockBytes + 16u * threadIdx.x;
+  if (off < o.n) {
+    const u64 pixel = first + off / 16u;
+    const int py = (int)(pixel / (u32)W), px = (int)(pixel - (u64)py * (u32)W);
+    out.store16(off, sdf_pixel(ox, oy, oz, pixel_dir(px, py, W, H, aspect)));
+  }
+  piece_done(o);
 }
 
 // shaders/raymarch_sphere.frag:9-53 -- the scene's active marcher: per fragment,
@@ -664,9 +670,10 @@ __global__ __launch_bounds__(256) void dda_kernel(const u8 *__restrict__ g, int 
 
 }  // namespace
 
-hipError_t launch_sdf(const float cam_pos[3], float aspect, int W, int H, float *d_rgba, hipStream_t s) {
-  const dim3 grid((W + 15) / 16, (H + 15) / 16);
-  hipLaunchKernelGGL(sdf_kernel, grid, dim3(256), 0, s, cam_pos[0], cam_pos[1], cam_pos[2], aspect, W, H, d_rgba);
+hipError_t launch_sdf(const float cam_pos[3], float aspect, int W, int H, size_t first, const PieceOut &out,
+                      hipStream_t s) {
+  hipLaunchKernelGGL(sdf_kernel, dim3(piece_blocks(out)), dim3(kBlockBytes / 16), 0, s, cam_pos[0], cam_pos[1], cam_pos[2], aspect,
+                     W, H, (u64)first, out);
   return hipGetLastError();
 }
 

@@ -19,6 +19,7 @@
 #include <cstring>
 
 #include "fs3d_render.h"
+#include "hostcopy.h"
 
 using namespace fs3d;
 
@@ -256,11 +257,10 @@ int fs3d_render_sdf(const float cam_pos[3], float aspect, int32_t W, int32_t H, 
   (void)hipGetDevice(&dev);
   if (int rc = ensure_device(dev)) return rc;
   const size_t bytes = (size_t)W * H * 4 * sizeof(float);
-  float *d = nullptr;
-  FS3D_HIP(hipMalloc(&d, bytes));
-  hipError_t e = launch_sdf(cam_pos, aspect, W, H, d, nullptr);
-  if (e == hipSuccess) e = hipMemcpy(rgba, d, bytes, hipMemcpyDeviceToHost);
-  (void)hipFree(d);
+  // rendered into pinned memory, a piece at a time: no image on the device
+  const hipError_t e = make_on_host(rgba, bytes, dev, [&](size_t off, const PieceOut &out, hipStream_t s) {
+    return launch_sdf(cam_pos, aspect, W, H, off / 16, out, s);
+  });
   if (e != hipSuccess) return set_error(FS3D_ERR_HIP, "render_sdf failed: %s", hipGetErrorString(e));
   return clear_error();
 }
@@ -337,10 +337,8 @@ int fs3d_world_render(fs3d_world *w, const fs3d_camera *cam, int32_t W, int32_t 
                       w->d_dirty, w->occ_valid, w->stream));
   w->occ_valid = true;
   FS3D_HIP(hipEventRecord(w->ev1, w->stream));
-  FS3D_HIP(hipMemcpyAsync(rgb, w->d_rgb, px * 3 * sizeof(float), hipMemcpyDeviceToHost, w->stream));
-  FS3D_HIP(hipMemcpyAsync(hit, w->d_hit, px * sizeof(u64), hipMemcpyDeviceToHost, w->stream));
-  FS3D_HIP(hipMemcpyAsync(face, w->d_face, px, hipMemcpyDeviceToHost, w->stream));
-  FS3D_HIP(hipStreamSynchronize(w->stream));
+  FS3D_HIP(copy_to_host({{rgb, w->d_rgb, px * 3 * sizeof(float)}, {hit, w->d_hit, px * sizeof(u64)}, {face, w->d_face, px}},
+                        w->dev, w->stream));
   float ms = 0.f;
   FS3D_HIP(hipEventElapsedTime(&ms, w->ev0, w->ev1));
   w->last_render_ms = ms;

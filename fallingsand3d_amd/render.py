@@ -23,7 +23,7 @@ def palette():
 
 def render_sdf(cam_pos=(0.0, 0.0, -5.0), aspect=1700.0 / 900.0, W=850, H=450):
     cp = np.ascontiguousarray(cam_pos, np.float32)
-    out = np.zeros((H, W, 4), np.float32)
+    out = np.empty((H, W, 4), np.float32)
     check(lib().fs3d_render_sdf(ptr(cp, c_float), aspect, W, H, ptr(out, c_float)))
     return out
 
@@ -75,9 +75,9 @@ def camera(origin, basis, light, aspect):
 
 def render(world, cam, W, H):
     """(rgb (H,W,3) float32, hit (H,W) uint64, face (H,W) uint8) of the world's grid."""
-    rgb = np.zeros((H, W, 3), np.float32)
-    hit = np.zeros((H, W), np.uint64)
-    face = np.zeros((H, W), np.uint8)
+    rgb = np.empty((H, W, 3), np.float32)
+    hit = np.empty((H, W), np.uint64)
+    face = np.empty((H, W), np.uint8)
     check(lib().fs3d_world_render(world.handle, ctypes.byref(cam), W, H, ptr(rgb, c_float), ptr(hit, c_u64),
                                   ptr(face, c_u8)))
     return rgb, hit, face
