@@ -96,8 +96,10 @@ int ensure_small(fs3d_world *w, int slots) {
   if (w->h_pinned_cap < cap + 1) {
     if (w->h_pinned) FS3D_HIP(hipHostFree(w->h_pinned));
     w->h_pinned = nullptr;
-    FS3D_HIP(hipHostMalloc(&w->h_pinned, (size_t)(cap + 1) * sizeof(u64), hipHostMallocDefault));
+    FS3D_HIP(hipHostMalloc(&w->h_pinned, (size_t)(cap + 3) * sizeof(u64), hipHostMallocDefault));
     w->h_pinned_cap = cap + 1;
+    w->h_pinned[w->h_pinned_cap + 1] = 0;  // no note
+    w->note_seq = 0;
   }
   return FS3D_OK;
 }
@@ -150,20 +152,18 @@ int mark_all(fs3d_world *w) {
   return FS3D_OK;
 }
 
-// Sets the change bits of every lane segment whose blocks contain cell (x,y,z),
-// at both parities (segments x/S - 1 .. x/S + 1 of the row quads holding it).
-int mark_cell(fs3d_world *w, int x, int y, int z) {
-  w->occ_valid = false;
-  long long idx[2];
-  for (int q = 0; q < 2; q++) {
-    const long long nyq = (w->ny + q + 1) >> 1;
-    idx[q] = (long long)((z + q) >> 1) * nyq + ((y + q) >> 1);
-  }
-  const int s = x / w->shape.seg, lr = w->shape.lanes_per_row;
-  u64 bits = 1ull << s;  // s <= 63
-  if (s > 0) bits |= 1ull << (s - 1);
-  if (s + 1 < lr) bits |= 1ull << (s + 1);
-  FS3D_HIP(launch_mark_cells(w->d_masks[0], w->d_masks[1], idx[0], idx[1], bits, w->mask_words, w->stream));
+// The note that the next launch is to write.
+Note next_note(fs3d_world *w) { return Note{w->h_pinned + w->h_pinned_cap, ++w->note_seq}; }
+
+// Waits for the last note and reads it: by looking for it, and after some 100 us, which
+// is more than a small world's work takes, by waiting for the stream.
+int read_note(fs3d_world *w, u64 *value) {
+  const u64 *at = w->h_pinned + w->h_pinned_cap;
+  auto here = [&] { return __atomic_load_n(at + 1, __ATOMIC_ACQUIRE) == w->note_seq; };
+  for (int i = 0; i < 4000 && !here(); i++) __builtin_ia32_pause();
+  if (!here()) FS3D_HIP(hipStreamSynchronize(w->stream));
+  if (!here()) return set_error(FS3D_ERR_HIP, "the stream ended without its result");
+  if (value) *value = at[0];
   return FS3D_OK;
 }
 
@@ -615,12 +615,31 @@ int fs3d_world_set_voxel(fs3d_world *w, int32_t x, int32_t y, int32_t z, uint8_t
   size_t off;
   if (int rc = voxel_offset(w, x, y, z, &off)) return rc;
   FS3D_HIP(hipSetDevice(w->dev));
-  FS3D_HIP(hipMemcpyAsync(w->buf[w->cur] + off, &v, 1, hipMemcpyHostToDevice, w->stream));
-  if (w->planes_valid)
-    FS3D_HIP(launch_plane_set(plane_shape(w->nx, w->ny, w->nz), w->planes[w->pcur], x, y, z, v, w->d_reserved,
-                              w->pflags_valid ? w->pflags[w->fcur] : nullptr, w->stream));
-  if (int rc = mark_cell(w, x, y, z)) return rc;
-  FS3D_HIP(hipStreamSynchronize(w->stream));
+  CellEdit e{};
+  e.cell = w->buf[w->cur] + off;
+  e.value = v;
+  // every lane segment whose blocks contain the cell, at both parities (segments
+  // x/S - 1 .. x/S + 1 of the row quads holding it)
+  for (int q = 0; q < 2; q++) {
+    e.masks[q] = w->d_masks[q];
+    e.idx[q] = (long long)((z + q) >> 1) * ((w->ny + q + 1) >> 1) + ((y + q) >> 1);
+  }
+  const int seg = x / w->shape.seg, lr = w->shape.lanes_per_row;
+  e.bits = 1ull << seg;  // seg <= 63
+  if (seg > 0) e.bits |= 1ull << (seg - 1);
+  if (seg + 1 < lr) e.bits |= 1ull << (seg + 1);
+  e.edge_off = w->mask_words;
+  if (w->planes_valid) {
+    const PlaneShape ps = plane_shape(w->nx, w->ny, w->nz);
+    e.planes = static_cast<u32 *>(w->planes[w->pcur]);
+    e.reserved = w->d_reserved;
+    e.word = plane_word(ps, x, y, z);
+    e.x = x;
+    if (w->pflags_valid) e.flags = w->pflags[w->fcur] + plane_cell_flags(ps, y, z, &e.nflags);
+  }
+  w->occ_valid = false;
+  FS3D_HIP(launch_set_cell(e, next_note(w), w->stream));
+  if (int rc = read_note(w, nullptr)) return rc;
   return clear_error();
 }
 
@@ -630,8 +649,10 @@ int fs3d_world_get_voxel(fs3d_world *w, int32_t x, int32_t y, int32_t z, uint8_t
   size_t off;
   if (int rc = voxel_offset(w, x, y, z, &off)) return rc;
   FS3D_HIP(hipSetDevice(w->dev));
-  FS3D_HIP(hipMemcpyAsync(v, w->buf[w->cur] + off, 1, hipMemcpyDeviceToHost, w->stream));
-  FS3D_HIP(hipStreamSynchronize(w->stream));
+  FS3D_HIP(launch_post_byte(w->buf[w->cur] + off, next_note(w), w->stream));
+  u64 got = 0;
+  if (int rc = read_note(w, &got)) return rc;
+  *v = (uint8_t)got;
   return clear_error();
 }
 
@@ -785,11 +806,17 @@ int fs3d_world_tick(fs3d_world *w, uint64_t *hash) {
   bool planes = false;
   if (int rc = choose_path(w, 1, &planes)) return rc;
   int fin = w->cur;
-  if (int rc = planes ? enqueue_planes(w, 1, 1, nullptr, &fin) : enqueue_ticks(w, 1, 1, nullptr, &fin)) return rc;
-  FS3D_HIP(hipMemcpyAsync(w->h_pinned, w->d_small + 1, sizeof(u64), hipMemcpyDeviceToHost, w->stream));
-  FS3D_HIP(hipStreamSynchronize(w->stream));
+  if (w->n <= kHashPostMax && !w->d_stats) {
+    if (int rc = planes ? enqueue_planes(w, 1, 0, nullptr, &fin) : enqueue_ticks(w, 1, 0, nullptr, &fin)) return rc;
+    FS3D_HIP(launch_hash_post(w->buf[planes ? w->cur : fin], w->n, w->d_parts, next_note(w), w->stream));
+  } else {
+    if (int rc = planes ? enqueue_planes(w, 1, 1, nullptr, &fin) : enqueue_ticks(w, 1, 1, nullptr, &fin)) return rc;
+    FS3D_HIP(launch_post(w->d_small + 1, next_note(w), w->stream));
+  }
+  u64 got = 0;
+  if (int rc = read_note(w, &got)) return rc;
   ticked(w, 1, planes, fin);
-  *hash = w->h_pinned[0];
+  *hash = got;
   return clear_error();
 }
 
@@ -797,11 +824,16 @@ int fs3d_world_hash(fs3d_world *w, uint64_t *hash) {
   if (int rc = check_world(w)) return rc;
   if (!hash) return set_error(FS3D_ERR_INVALID, "hash is NULL");
   FS3D_HIP(hipSetDevice(w->dev));
-  FS3D_HIP(launch_hash(w->buf[w->cur], w->n, w->d_parts, w->stream));
-  FS3D_HIP(launch_hash_finalize(w->d_parts, w->d_small + 1, w->stream));
-  FS3D_HIP(hipMemcpyAsync(w->h_pinned, w->d_small + 1, sizeof(u64), hipMemcpyDeviceToHost, w->stream));
-  FS3D_HIP(hipStreamSynchronize(w->stream));
-  *hash = w->h_pinned[0];
+  if (w->n <= kHashPostMax) {
+    FS3D_HIP(launch_hash_post(w->buf[w->cur], w->n, w->d_parts, next_note(w), w->stream));
+  } else {
+    FS3D_HIP(launch_hash(w->buf[w->cur], w->n, w->d_parts, w->stream));
+    FS3D_HIP(launch_hash_finalize(w->d_parts, w->d_small + 1, w->stream));
+    FS3D_HIP(launch_post(w->d_small + 1, next_note(w), w->stream));
+  }
+  u64 got = 0;
+  if (int rc = read_note(w, &got)) return rc;
+  *hash = got;
   return clear_error();
 }
 

@@ -132,9 +132,36 @@ hipError_t launch_tick_packed(const TickShape &sh, const u8 *src, u8 *dst, int n
                               u64 *stats, TickEntry *list, u32 *ctl, size_t mask_words, u32 pack_waves,
                               int chunk);
 int pack_blocks_per_cu(int seg);
-// Sets change bits `bits` of row quad i0 (parity 0) and i1 (parity 1), and the
-// edge bits next to them (edge words at offset edge_off).
-hipError_t launch_mark_cells(u64 *m0, u64 *m1, long long i0, long long i1, u64 bits, size_t edge_off, hipStream_t s);
+// A value for the host: at[0] = the value, then at[1] = seq, in pinned memory.
+struct Note {
+  u64 *at;
+  u64 seq;
+};
+__device__ __forceinline__ void post_note(const Note &n, u64 value) {
+  __hip_atomic_store(n.at, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(n.at + 1, n.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// State hash of up to kHashPostMax cells (g readable up to 3 bytes past them), posted.
+constexpr size_t kHashPostMax = 1u << 18;
+hipError_t launch_hash_post(const u8 *g, size_t n, u64 *hash_parts, const Note &note, hipStream_t s);
+// One cell set by the host: its byte, change bits `bits` of row quad idx[p] at either
+// parity and the edge bits next to them (edge words at offset edge_off), and, with
+// planes, its bits there and the nflags change flags of its item.
+struct CellEdit {
+  u8 *cell;
+  u32 value;
+  u64 *masks[2];
+  long long idx[2];
+  u64 bits;
+  size_t edge_off;
+  u32 *planes, *reserved;
+  u64 *flags;
+  size_t word;
+  int x, nflags;
+};
+hipError_t launch_set_cell(const CellEdit &e, const Note &n, hipStream_t s);
+hipError_t launch_post_byte(const u8 *p, const Note &n, hipStream_t s);
+hipError_t launch_post(const u64 *p, const Note &n, hipStream_t s);
 // Two dense ticks (t and t + 1) in one pass: src -> dst holds the state after
 // both.  Supported for one row quad per wave and LDS tiles within 64 KiB.
 bool tick2_supported(const TickShape &sh, int nx, size_t *lds_bytes);
@@ -176,6 +203,7 @@ struct fs3d_world {
   int small_cap = 0;             // number of hash output slots
   fs3d::u64 *h_pinned = nullptr; // pinned staging for small read-backs
   int h_pinned_cap = 0;
+  fs3d::u64 note_seq = 0;        // of the last note (h_pinned[h_pinned_cap ..])
   fs3d::TickShape shape{};
   fs3d::TickShape shape2{};  // the fused two-tick pass: smallest segment with whole rows per wave
   int seg_req = 0;

@@ -55,9 +55,8 @@ hipError_t launch_plane_pad(const PlaneShape &ps, void *planes, hipStream_t s);
 hipError_t launch_plane_pack(const PlaneShape &ps, const u8 *g, void *planes, u32 *reserved, hipStream_t s);
 hipError_t launch_plane_unpack(const PlaneShape &ps, const void *planes, u8 *g, const u32 *reserved, hipStream_t s);
 
-// One cell of planes, and of its item's change flags when given.
-hipError_t launch_plane_set(const PlaneShape &ps, void *planes, int x, int y, int z, u8 v, u32 *reserved, u64 *flags,
-                            hipStream_t s);
+// The word that holds a cell.
+size_t plane_word(const PlaneShape &ps, int x, int y, int z);
 
 // ---- ticks of the active items only (plane.hip has the rule) ----
 constexpr int kItemQuads = 1;   // even-parity row quads of an item along y
@@ -68,6 +67,8 @@ struct PlaneCells {
   size_t flag_words = 0, since_words = 0, list_words = 0;  // u64, u64, u32
 };
 PlaneCells plane_cells(const PlaneShape &ps);
+// Where the change flags of a cell's item begin (*n of them, bit = word).
+size_t plane_cell_flags(const PlaneShape &ps, int y, int z, int *n);
 int plane_list_blocks_per_cu();
 // A pass over the active items: ticks t and t + 1 (pair, t odd) or tick t (of
 // either parity; *tick_dev + k_off has t's).  flags_in: the pass before; flags_out:

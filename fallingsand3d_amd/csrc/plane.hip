@@ -582,20 +582,6 @@ __global__ __launch_bounds__(256) void plane_unpack_cells_kernel(const u32x4 *in
   if (lane == 0) since[c] = 0;
 }
 
-// One cell set by the host; its item counts as changed throughout (flags: the
-// item's cell of the strip grid, or nullptr).
-__global__ void plane_set_kernel(u32 *planes, size_t word, int x, u32 v, u32 *reserved, u64 *flags) {
-  if (threadIdx.x != 0) return;
-  if (flags)
-    for (int i = 0; i < kFlags; i++) flags[i] |= 1ull << (x >> 6);
-  if (v >= 4u) *reserved = 1u;
-  const u32 code = (v >= 4u ? (u32)FS3D_STATIC : v) ^ 1u;
-  u32 *w = planes + 4 * word + (x & 1);
-  const u32 m = 1u << pair_bit((x & 63) >> 1);
-  w[0] = (code & 1u) ? w[0] | m : w[0] & ~m;
-  w[2] = (code & 2u) ? w[2] | m : w[2] & ~m;
-}
-
 }  // namespace
 
 static void fill_args(PlaneArgs &a, const PlaneShape &ps) {
@@ -817,13 +803,13 @@ hipError_t launch_plane_hash(const PlaneShape &ps, const void *planes, const Pla
   return hipGetLastError();
 }
 
-hipError_t launch_plane_set(const PlaneShape &ps, void *planes, int x, int y, int z, u8 v, u32 *reserved, u64 *flags,
-                            hipStream_t s) {
-  const size_t word = ((size_t)(z + 1) * (u32)(ps.ny + 1) + (u32)(y + 1)) * (u32)ps.lr + (u32)(x >> 6);
-  const size_t cell = (size_t)(z / (2 * kItemLayers)) * plane_cells(ps).strips + (size_t)(y / (2 * kItemQuads));
-  hipLaunchKernelGGL(plane_set_kernel, dim3(1), dim3(64), 0, s, static_cast<u32 *>(planes), word, x, (u32)v, reserved,
-                     flags ? flags + cell * kFlags : nullptr);
-  return hipGetLastError();
+size_t plane_word(const PlaneShape &ps, int x, int y, int z) {
+  return ((size_t)(z + 1) * (u32)(ps.ny + 1) + (u32)(y + 1)) * (u32)ps.lr + (u32)(x >> 6);
+}
+
+size_t plane_cell_flags(const PlaneShape &ps, int y, int z, int *n) {
+  *n = kFlags;
+  return ((size_t)(z / (2 * kItemLayers)) * plane_cells(ps).strips + (size_t)(y / (2 * kItemQuads))) * kFlags;
 }
 
 }  // namespace fs3d

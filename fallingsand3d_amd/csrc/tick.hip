@@ -710,15 +710,6 @@ __global__ __launch_bounds__(256) void fill_u32_kernel(u32 *p, size_t n, u32 v) 
     p[i] = v;
 }
 
-__global__ void mark_cells_kernel(u64 *m0, u64 *m1, long long i0, long long i1, u64 bits, size_t edge_off) {
-  if (threadIdx.x == 0) {
-    m0[i0] |= bits;
-    m1[i1] |= bits;
-    m0[edge_off + i0] |= bits | (bits << 1);
-    m1[edge_off + i1] |= bits | (bits << 1);
-  }
-}
-
 }  // namespace
 
 int plan_tick(int nx, int ny, int nz, int seg_req, TickShape *out) {
@@ -938,11 +929,6 @@ hipError_t launch_fill_u64(u64 *p, size_t n, u64 v, hipStream_t s) {
 hipError_t launch_fill_u32(u32 *p, size_t n, u32 v, hipStream_t s) {
   const size_t blocks = std::min<size_t>(std::max<size_t>((n + 255) / 256, 1), 4096);
   hipLaunchKernelGGL(fill_u32_kernel, dim3((unsigned)blocks), dim3(256), 0, s, p, n, v);
-  return hipGetLastError();
-}
-
-hipError_t launch_mark_cells(u64 *m0, u64 *m1, long long i0, long long i1, u64 bits, size_t edge_off, hipStream_t s) {
-  hipLaunchKernelGGL(mark_cells_kernel, dim3(1), dim3(64), 0, s, m0, m1, i0, i1, bits, edge_off);
   return hipGetLastError();
 }
 
