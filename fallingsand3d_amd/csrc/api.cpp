@@ -365,7 +365,7 @@ int enqueue_planes(fs3d_world *w, int nticks, int hash_every, const u64 *tick_de
   if (launch) {
     if (items)
       FS3D_HIP(launch_plane_unpack_cells(ps, w->planes[src], w->buf[w->cur], w->pflags[f], w->d_since, w->d_reserved,
-                                         w->stream));
+                                         w->occ_track ? w->d_dirty : nullptr, w->stream));
     else
       FS3D_HIP(launch_plane_unpack(ps, w->planes[src], w->buf[w->cur], w->d_reserved, w->stream));
   }
@@ -390,7 +390,8 @@ void ticked(fs3d_world *w, int nticks, bool planes, int fin) {
     w->planes_valid = true;
     w->pflags_valid = item_ticks(w);
     w->masks_stale = true;
-    w->occ_valid = false;
+    // the items' unpacking has marked the bricks it wrote
+    w->occ_valid = w->occ_valid && w->pflags_valid && w->occ_track;
   } else {
     w->cur = fin;
     if (nticks > 0) w->planes_valid = false;

@@ -264,10 +264,13 @@ hipError_t make_on_host(void *host, size_t n, int dev,
   if (!g) return hipErrorOutOfMemory;
   hipError_t e = hipErrorOutOfMemory;
   try {
+    std::vector<u8> between;  // the threads write ordinary memory only
+    if (!pageable(host)) between.resize(n);
     std::vector<Piece> pieces;
-    split(&pieces, host, n, 0, piece_of(n));
+    split(&pieces, between.empty() ? host : between.data(), n, 0, piece_of(n));
     e = run(g, pieces, piece_of(n), n, g->stream,
             [&](size_t, size_t off, const PieceOut &out, hipStream_t st) { return make(off, out, st); });
+    if (e == hipSuccess && !between.empty()) e = hipMemcpy(host, between.data(), n, hipMemcpyDefault);
   } catch (...) {
   }
   give_back(g);

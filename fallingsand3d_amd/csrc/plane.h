@@ -77,8 +77,9 @@ int plane_list_blocks_per_cu();
 hipError_t launch_plane_list(const PlaneShape &ps, const void *src, void *dst, u64 t, const u64 *tick_dev, u32 k_off,
                              bool pair, bool fresh, const u64 *flags_in, u64 *flags_out, u64 *since, u32 *list,
                              u32 *count, u32 nwaves, hipStream_t s);
-// Writes the bytes of the items in since or flags (the last pass's) and clears since.
+// Writes the bytes of the items in since or flags (the last pass's) and clears since;
+// dirty (or nullptr): a bit per 8^3 brick, set for those that hold a written item.
 hipError_t launch_plane_unpack_cells(const PlaneShape &ps, const void *planes, u8 *g, const u64 *flags, u64 *since,
-                                     const u32 *reserved, hipStream_t s);
+                                     const u32 *reserved, u64 *dirty, hipStream_t s);
 
 }  // namespace fs3d

@@ -35,3 +35,18 @@ def test_items_match_byte_kernels(gpu, shape):
                     b.set_voxel(x, y, z, v)
                 a.skip = gpu.SKIP_OFF if k == 5 else gpu.SKIP_AUTO
             assert np.array_equal(a.download(), b.download())
+
+
+def test_items_mark_the_renderers_bricks(gpu):
+    from fallingsand3d_amd import render as R
+    from test_render_incremental_gpu import expected_maps
+    shape = (1000, 1031, 525)
+    announce(f"frames between item ticks {shape}")
+    cam = R.orbit_camera(shape, 0.4, 1.6, 0.4, 1.5)
+    with gpu.World(shape) as w:
+        w.fill_pillars(4, (40, 2, 9, 65, 459, 125, 333, 130, 340, 3, 30))
+        for n in (4, 1, 3, 12):  # the first frame reads every brick, the later ones what moved
+            w.run(n, 0)
+            R.render(w, cam, 60, 40)
+            maps, want = R.render_maps(w), expected_maps(w.download())
+            assert all((a == b).all() for a, b in zip(maps, want)), n
