@@ -251,6 +251,19 @@ int dense_chunk_seg(const fs3d_world *w) { return w->seg_req == 0 && w->nx > 102
 // the destination already holding its bytes.
 constexpr size_t kInPlaceMaxBytes = size_t(1) << 27;
 
+// Whether the plane ticks of a skipping world visit only its active items.  Below
+// this size a pass over everything is as fast as listing what moves.  (Thin grids'
+// tiles would outgrow the addressing.)
+constexpr u64 kItemsMinVoxels = 1ull << 29;
+constexpr size_t kMaxPlaneWords = (1ull << 28) - 1;
+bool may_list(const fs3d_world *w) {
+  return (u64)w->n > kItemsMinVoxels && plane_words(plane_shape(w->nx, w->ny, w->nz, true)) <= kMaxPlaneWords;
+}
+bool item_ticks(const fs3d_world *w) { return w->skip && may_list(w); }
+
+// The planes' shape for what the world does now.
+PlaneShape shape_of(const fs3d_world *w) { return plane_shape(w->nx, w->ny, w->nz, item_ticks(w)); }
+
 // ---- bit-plane ticks ----------------------------------------------------------
 // Runs of ticks go through the bit planes: packed once, ticked in pairs at a
 // quarter of the bytes and without table lookups, unpacked once.  The byte
@@ -266,23 +279,26 @@ bool plane_path(const fs3d_world *w, int nticks) {
   if (w->planes_off || w->seg_req != 0 || w->d_stats || nticks < 1) return false;
   if (w->skip != FS3D_SKIP_OFF && w->skip != FS3D_SKIP_AUTO) return false;
   if (!w->skip && w->fuse_set && !w->fuse) return false;
-  if (w->nx < 16 || plane_words(plane_shape(w->nx, w->ny, w->nz)) >= (1ull << 28)) return false;
+  if (w->nx < 16 || plane_words(shape_of(w)) > kMaxPlaneWords) return false;
   return w->planes_valid || nticks >= kPlaneMinTicks;
 }
-
-// Whether the plane ticks of a skipping world visit only its active items.  Below
-// this size a pass over everything is as fast as listing what moves.
-constexpr u64 kItemsMinVoxels = 1ull << 29;
-bool item_ticks(const fs3d_world *w) { return w->skip && (u64)w->n > kItemsMinVoxels; }
 
 // Plane buffers (and the item lists) on first use; false (and the byte kernels from
 // then on) when the device has no room for them.
 bool ensure_planes(fs3d_world *w) {
-  const PlaneShape ps = plane_shape(w->nx, w->ny, w->nz);
+  const PlaneShape ps = shape_of(w);
   hipError_t e = hipSuccess;
-  if (!w->planes[0]) {
+  const bool created = !w->planes[0];
+  if (created) {
     e = hipMalloc((void **)&w->d_reserved, sizeof(u32));
-    for (int i = 0; i < 2 && e == hipSuccess; i++) e = hipMalloc(&w->planes[i], plane_words(ps) * 16);
+    // room for either layout: the schedule may change
+    const size_t most = std::max(plane_words(plane_shape(w->nx, w->ny, w->nz)),
+                                 may_list(w) ? plane_words(plane_shape(w->nx, w->ny, w->nz, true)) : 0);
+    for (int i = 0; i < 2 && e == hipSuccess; i++) e = hipMalloc(&w->planes[i], most * 16);
+  }
+  if (created || w->planes_tiled != ps.tiled) {
+    w->planes_tiled = ps.tiled;
+    w->planes_valid = false;
     for (int i = 0; i < 2 && e == hipSuccess; i++) e = launch_plane_pad(ps, w->planes[i], w->stream);
   }
   if (item_ticks(w) && !w->d_items && e == hipSuccess) {
@@ -319,7 +335,7 @@ bool ensure_planes(fs3d_world *w) {
 // current state) and the unpacking into buf[cur].  *pfinal: the index of the plane
 // buffer holding the result, + 2 * that of the last pass's change flags.
 int enqueue_planes(fs3d_world *w, int nticks, int hash_every, const u64 *tick_dev, int *pfinal, bool launch = true) {
-  const PlaneShape ps = plane_shape(w->nx, w->ny, w->nz);
+  const PlaneShape ps = shape_of(w);
   const bool items = item_ticks(w);
   int src = w->planes_valid ? w->pcur : 0, f = w->fcur;
   bool fresh = !w->planes_valid || !w->pflags_valid;
@@ -631,7 +647,7 @@ int fs3d_world_set_voxel(fs3d_world *w, int32_t x, int32_t y, int32_t z, uint8_t
   if (seg + 1 < lr) e.bits |= 1ull << (seg + 1);
   e.edge_off = w->mask_words;
   if (w->planes_valid) {
-    const PlaneShape ps = plane_shape(w->nx, w->ny, w->nz);
+    const PlaneShape ps = plane_shape(w->nx, w->ny, w->nz, w->planes_tiled);
     e.planes = static_cast<u32 *>(w->planes[w->pcur]);
     e.reserved = w->d_reserved;
     e.word = plane_word(ps, x, y, z);

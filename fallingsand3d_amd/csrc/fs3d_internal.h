@@ -236,6 +236,7 @@ struct fs3d_world {
   void *planes[2] = {nullptr, nullptr};
   int pcur = 0;
   bool planes_valid = false, planes_off = false;
+  bool planes_tiled = false;  // the buffers' layout (its rows around the grid are zero)
   fs3d::u32 *d_reserved = nullptr;  // a byte >= 4 has been packed or set
   // ticks of the active items only: change flags of the last pass (pflags[fcur],
   // exact or too many while pflags_valid), items changed since the bytes were

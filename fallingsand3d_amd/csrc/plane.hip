@@ -59,13 +59,25 @@ __device__ __forceinline__ u32 div_by(u32 i, u32 d, u32 magic) { return magic ? 
 
 struct LayerArgs {
   int nx, ny, nz, lr;
-  u32 magic;  // of lr (one lane per word) or 4 lr (per quarter)
+  u32 magic;  // of the words of a row (or of a tile's eight), times the lanes per word
+  u32 words;  // of a layer
+  size_t first, stride;  // word 0 of layer 0, words from layer to layer
+  bool tiled;
 };
 
-// First word of a layer's first row.
-__device__ __forceinline__ size_t layer_word(const LayerArgs &a, int z) {
-  return ((size_t)(z + 1) * (u32)(a.ny + 1) + 1u) * (u32)a.lr;
+// Row and word of a lane's place i in a layer, `per` lanes to a word (sub: which of
+// them).  Rows outside the grid (tiles have some) are >= ny.
+__device__ __forceinline__ u32 place(const LayerArgs &a, u32 i, u32 per, u32 *seg, u32 *sub) {
+  const u32 d = per * (u32)a.lr * (a.tiled ? 8u : 1u);
+  const u32 q = div_by(i, d, a.magic), rest = i - q * d;
+  *sub = rest % per;
+  const u32 w = rest / per;
+  *seg = a.tiled ? w >> 3 : w;
+  return a.tiled ? 8u * q + (w & 7u) - 1u : q;
 }
+
+// First word of a layer.
+__device__ __forceinline__ size_t layer_word(const LayerArgs &a, int z) { return a.first + (size_t)z * a.stride; }
 
 // ---- state hash --------------------------------------------------------------------
 // Four lanes per word, each mixing its quarter's non-empty cells, or 16 lanes in a
@@ -93,11 +105,12 @@ __device__ __forceinline__ void hash_block(const HashArgs &h, u32 block) {
   const bool bytes = *h.reserved != 0;
   const u32 by = block / h.gx, bx = block - by * h.gx;
   u64 acc = 0;
-  const u32 lane = bx * 256u + threadIdx.x, qpr = 4u * (u32)a.lr;
+  const u32 lane = bx * 256u + threadIdx.x;
   const u32 i = h.split == 4 ? lane >> 2 : lane, cells = h.split == 4 ? 0xFu << 4 * (lane & 3u) : 0xFFFFu;
-  const u32 y = div_by(i, qpr, a.magic);
-  const int c = (int)(i - y * qpr);
-  const int m = i < (u32)a.ny * qpr ? min(16, a.nx - 16 * c) : 0;
+  u32 seg, sub;
+  const u32 y = place(a, i, 4, &seg, &sub);
+  const int c = (int)(4 * seg + sub);
+  const int m = i < 4u * a.words && y < (u32)a.ny ? min(16, a.nx - 16 * c) : 0;
   if (m > 0)
     for (int z = (int)by; z < a.nz; z += (int)h.gy) {
       const u64 i0 = ((u64)z * (u32)a.ny + y) * (u32)a.nx + (u32)(16 * c);
@@ -266,10 +279,10 @@ __global__ __launch_bounds__(256) void plane_pair_kernel(PlaneArgs a) {
 // change; a change of a block at the item's first or last word bit, row, layer; any
 // change in the last pass alone.  A flag may be set without need, never missing.
 //
-// Bound by the 128-byte lines around the 16-byte words it visits: sand columns over a
-// pool at 2048^3, where 12 % of the items have work, read 2.1 GB and write 0.5 GB per
-// pass (0.69 ms for two ticks, 0.13 ms of it instructions), against 4.3 GB (0.82 ms)
-// over everything; the byte kernels' packed schedule takes 2 x 0.36 ms.
+// Sand columns over a pool at 2048^3, where 12 % of the items have work: 145 us per
+// pair of ticks (123 us of it instructions).  With planes kept as rows, where the line
+// around a word holds 512 cells of one row, the same pass took 280 us; a pass over
+// everything takes 820, the byte kernels' packed schedule 2 x 360.
 enum { kAny = 0, kXFirst, kXLast, kYFirst, kYLast, kZFirst, kZLast, kNow, kFlags };
 
 // One thread per cell: which items have work, appended to the list in word order;
@@ -350,7 +363,7 @@ __global__ __launch_bounds__(256) void plane_list_kernel(PlaneArgs a, const u32 
   const u32 t = (u32)tick_of(a);
   const u32 n = *count;
   const Planes src(a.src, a.bytes), dst(a.dst, a.bytes);
-  const u32 row = (u32)a.lr * 16u, layer = row * (u32)(a.ny + 1);
+  const u32 tile = (u32)a.lr * 128u, layer = tile * (u32)((a.ny + 2) / 8 + 1);
   const int m = a.zlen;
   const int prev = (lane ? lane - 1 : 0) * 4, next = (lane < 63 ? lane + 1 : 63) * 4;
   for (u32 w = wave; w * 62u < n; w += nwaves) {
@@ -366,8 +379,13 @@ __global__ __launch_bounds__(256) void plane_list_kernel(PlaneArgs a, const u32 
     const bool has_next = in && lane < 63 && seg + 1 < (int)per && cn == code + 1u;
     const bool word = in && seg < a.lr;  // not the virtual word
     const bool mine = word && lane > 0 && lane < 63;
-    // row y0 - 1 of layer z0 - 1
-    const u32 off = word ? (u32)z0 * layer + (u32)y0 * row + (u32)seg * 16u : kOutside;
+    // rows y0 - 1 + 2 i and the one after, of layer z0 - 1
+    u32 off[K + 1];
+#pragma unroll
+    for (int i = 0; i <= K; i++) {
+      const u32 pr = (u32)(st * K + i);  // pair of rows: four to a tile
+      off[i] = word ? (u32)z0 * layer + (pr >> 2) * tile + (u32)seg * 128u + (pr & 3u) * 32u : kOutside;
+    }
     bool on[2 * K];
 #pragma unroll
     for (int j = 0; j < 2 * K; j++) on[j] = mine && y0 + j < a.ny;
@@ -422,19 +440,19 @@ __global__ __launch_bounds__(256) void plane_list_kernel(PlaneArgs a, const u32 
           u32x4 q[4];
 #pragma unroll
           for (int r = 0; r < 4; r++)
-            q[r] = src.load(off, base + (u32)(2 * j + 1 + (r & 1)) * row + (r >> 1 ? layer : 0u));
+            q[r] = src.load(off[j + (r & 1)], base + (r & 1 ? 0u : 16u) + (r >> 1 ? layer : 0u));
           const u32 c = quad_even(q, (u32)seg, variant_base((u32)(by0 + j), (u32)(bz0 + b), t));
           note(c, 2 * j, 2 * b, j == 0, j == K - 1, b == 0, b == m - 1);
 #pragma unroll
           for (int r = 0; r < 4; r++)
             dst.store(on[2 * j + (r & 1)] && 2 * b + (r >> 1) < zleft,
-                      off + (base + (u32)(2 * j + 1 + (r & 1)) * row + (r >> 1 ? layer : 0u)), q[r]);
+                      off[j + (r & 1)] + (base + (r & 1 ? 0u : 16u) + (r >> 1 ? layer : 0u)), q[r]);
         }
     } else {
       u32x4 top[2 * K], nx[4];
       u32 base = 0;  // layer 2 s - 1
 #pragma unroll
-      for (int r = 0; r < 4; r++) nx[r] = src.load(off, (r & 1 ? row : 0u) + (r >> 1 ? layer : 0u));
+      for (int r = 0; r < 4; r++) nx[r] = src.load(off[0], (r & 1 ? 16u : 0u) + (r >> 1 ? layer : 0u));
 #pragma unroll 1
       for (int s = 0; s <= m; s++, base += 2u * layer) {
         u32x4 lowp, upp;
@@ -443,9 +461,10 @@ __global__ __launch_bounds__(256) void plane_list_kernel(PlaneArgs a, const u32 
           u32x4 q[4];
 #pragma unroll
           for (int r = 0; r < 4; r++) q[r] = nx[r];
-          const u32 at = i < K ? base + (u32)(2 * i + 2) * row : base + 2u * layer;
+          const u32 at = i < K ? base : base + 2u * layer;
 #pragma unroll
-          for (int r = 0; r < 4; r++) nx[r] = src.load(off, at + (r & 1 ? row : 0u) + (r >> 1 ? layer : 0u));
+          for (int r = 0; r < 4; r++)
+            nx[r] = src.load(off[i < K ? i + 1 : 0], at + (r & 1 ? 16u : 0u) + (r >> 1 ? layer : 0u));
           __builtin_amdgcn_sched_barrier(0);
           const u32 c = odd(q, i, s);
           note(c, 2 * i - 1, 2 * s - 1, i == 0, i == K, s == 0, s == m);
@@ -456,7 +475,7 @@ __global__ __launch_bounds__(256) void plane_list_kernel(PlaneArgs a, const u32 
               const int dy = 2 * i - 1 + (r & 1), dz = 2 * s - 1 + (r >> 1);
               if (dy >= 0 && dy < 2 * K)
                 dst.store(on[dy] && (unsigned)dz < (unsigned)min(2 * m, zleft),
-                          off + (base + (u32)(dy + 1) * row + (r >> 1 ? layer : 0u)), q[r]);
+                          off[i] + (base + (r & 1 ? 16u : 0u) + (r >> 1 ? layer : 0u)), q[r]);
             }
           } else {
             if (i > 0) {
@@ -467,7 +486,7 @@ __global__ __launch_bounds__(256) void plane_list_kernel(PlaneArgs a, const u32 
 #pragma unroll
                 for (int r = 0; r < 4; r++)
                   dst.store(on[2 * i - 2 + (r & 1)] && 2 * s - 2 + (r >> 1) < zleft,
-                            off + (base - layer + (u32)(2 * i - 1 + (r & 1)) * row + (r >> 1 ? layer : 0u)), v[r]);
+                            off[i - 1 + (r & 1)] + (base - layer + (r & 1 ? 0u : 16u) + (r >> 1 ? layer : 0u)), v[r]);
               }
               top[2 * i - 2] = upp;
               top[2 * i - 1] = q[2];
@@ -502,9 +521,11 @@ __global__ __launch_bounds__(256) void plane_list_kernel(PlaneArgs a, const u32 
 __global__ __launch_bounds__(256) void plane_pack_kernel(const u8 *g, u32x4 *out, LayerArgs a, u32 *reserved) {
   bool any = false;
   const u32 i = blockIdx.x * 256u + threadIdx.x;
-  const bool in = i < (u32)a.ny * (u32)a.lr;
-  const u32 y = in ? div_by(i, (u32)a.lr, a.magic) : 0u;
-  const int x0 = in ? (int)(i - y * (u32)a.lr) * 64 : 0;
+  u32 seg, sub;
+  u32 y = place(a, i, 1, &seg, &sub);
+  const bool in = i < a.words && y < (u32)a.ny;
+  const int x0 = in ? (int)seg * 64 : 0;
+  y = in ? y : 0u;
   for (int z = (int)blockIdx.y; z < a.nz; z += (int)gridDim.y) {
     // loads may run up to 63 bytes past the last row, into the guard bytes
     const u32x4 v = word_from_bytes(g + ((size_t)z * (u32)a.ny + y) * (u32)a.nx + (u32)x0, min(64, a.nx - x0), &any);
@@ -516,11 +537,11 @@ __global__ __launch_bounds__(256) void plane_pack_kernel(const u8 *g, u32x4 *out
 // Planes to bytes, four lanes per word so that a wave stores 1 KiB in a row.
 __global__ __launch_bounds__(256) void plane_unpack_kernel(const u32x4 *in, u8 *g, LayerArgs a, const u32 *reserved) {
   const bool keep = *reserved != 0;
-  const u32 i = blockIdx.x * 256u + threadIdx.x, qpr = 4u * (u32)a.lr;
-  if (i >= (u32)a.ny * qpr) return;
-  const u32 y = div_by(i, qpr, a.magic);
-  const int c = (int)(i - y * qpr), m = min(16, a.nx - 16 * c);
-  if (m <= 0) return;
+  const u32 i = blockIdx.x * 256u + threadIdx.x;
+  u32 seg, sub;
+  const u32 y = place(a, i, 4, &seg, &sub);
+  const int c = (int)(4 * seg + sub), m = min(16, a.nx - 16 * c);
+  if (i >= 4u * a.words || y >= (u32)a.ny || m <= 0) return;
   for (int z = (int)blockIdx.y; z < a.nz; z += (int)gridDim.y) {
     u32 d[4];
     unpack_quarter(in[layer_word(a, z) + (i >> 2)], c & 3, d);
@@ -552,7 +573,7 @@ __global__ __launch_bounds__(256) void plane_pad_kernel(u32x4 *p, int ny, int nz
 // they lie in are marked: reading the bricks of what moved in ten ticks of 1024^3 sand
 // columns takes 76 us, reading all of them 204.
 __global__ __launch_bounds__(256) void plane_unpack_cells_kernel(const u32x4 *in, u8 *g, int nx, int ny, int nz, int lr,
-                                                                 int strips, int ncell, int rows, int layers,
+                                                                 u32 layer, int strips, int ncell, int rows, int layers,
                                                                  const u64 *flags, u64 *since, const u32 *reserved,
                                                                  u64 *dirty) {
   const int lane = threadIdx.x & 63;
@@ -576,7 +597,8 @@ __global__ __launch_bounds__(256) void plane_unpack_cells_kernel(const u32x4 *in
         const int y = st * rows + dy;
         if (y < ny) {
           u32 d[4];
-          unpack_quarter(in[((size_t)(z + 1) * (u32)(ny + 1) + (u32)(y + 1)) * (u32)lr + (u32)seg], q, d);
+          const u32 row = (u32)(y + 1);  // (tiled planes)
+          unpack_quarter(in[(size_t)(z + 1) * layer + ((row >> 3) * (u32)lr + (u32)seg) * 8u + (row & 7u)], q, d);
           store_quarter(g + ((size_t)z * (u32)ny + (u32)y) * (u32)nx + (u32)x0, m, d, keep);
         }
       }
@@ -610,8 +632,10 @@ static void fill_args(PlaneArgs &a, const PlaneShape &ps) {
 // per: lanes per word.  Layers per lane: enough blocks for the chip, few enough that
 // the row's division and a hash's reduction are shared by several layers.
 static LayerArgs layer_args(const PlaneShape &ps, int per, dim3 *grid) {
-  const u64 d = (u64)per * (u64)ps.lr, n = d * (u64)ps.ny;
-  LayerArgs a{ps.nx, ps.ny, ps.nz, ps.lr, 0};
+  const u64 rows = ps.tiled ? (u64)plane_tiles(ps) : (u64)ps.ny;
+  const u64 d = (u64)per * (u64)ps.lr * (ps.tiled ? 8 : 1), n = d * rows;
+  LayerArgs a{ps.nx, ps.ny, ps.nz, ps.lr, 0, (u32)(n / (u64)per), plane_word(ps, 0, ps.tiled ? -1 : 0, 0),
+              plane_word(ps, 0, 0, 1) - plane_word(ps, 0, 0, 0), ps.tiled};
   if (n * d < (1ull << 32) && d > 1) a.magic = (u32)(((1ull << 32) + d - 1) / d);
   const unsigned gx = (unsigned)((n + 255) / 256);
   const unsigned gy = (unsigned)std::min<u64>((u64)std::min(ps.nz, 65535), std::max<u64>(1, 16384 / std::max(gx, 1u)));
@@ -630,7 +654,7 @@ static HashArgs hash_args(const PlaneShape &ps, const PlaneHash &ph, const void 
   h.gy = grid.y;
   const bool direct = plane_hash_direct(ps);
   h.split = plane_words(ps) <= kSplitHashWords ? 4 : 1;
-  if (h.split == 4) h.gx = (unsigned)(((size_t)16 * (u32)ps.lr * (u32)ps.ny + 255) / 256);
+  if (h.split == 4) h.gx = (unsigned)(((size_t)16 * h.l.words + 255) / 256);
   h.out = direct ? ph.out : ph.parts;
   h.slots = direct ? 1 : kHashParts;
   return h;
@@ -785,12 +809,14 @@ hipError_t launch_plane_unpack_cells(const PlaneShape &ps, const void *planes, u
   const PlaneCells c = plane_cells(ps);
   const int ncell = (int)c.since_words;
   hipLaunchKernelGGL(plane_unpack_cells_kernel, dim3((unsigned)((ncell + 3) / 4)), dim3(256), 0, s,
-                     static_cast<const u32x4 *>(planes), g, ps.nx, ps.ny, ps.nz, ps.lr, c.strips, ncell,
+                     static_cast<const u32x4 *>(planes), g, ps.nx, ps.ny, ps.nz, ps.lr,
+                     (u32)(plane_tiles(ps) * 8 * ps.lr), c.strips, ncell,
                      2 * kItemQuads, 2 * kItemLayers, flags, since, reserved, dirty);
   return hipGetLastError();
 }
 
 hipError_t launch_plane_pad(const PlaneShape &ps, void *planes, hipStream_t s) {
+  if (ps.tiled) return launch_fill_u64(static_cast<u64 *>(planes), 2 * plane_words(ps), 0, s);
   const size_t n = ((size_t)2 * (u32)(ps.ny + 1) + (u32)ps.nz + 1) * (u32)ps.lr;
   hipLaunchKernelGGL(plane_pad_kernel, dim3((unsigned)std::min<size_t>((n + 255) / 256, 4096)), dim3(256), 0, s,
                      static_cast<u32x4 *>(planes), ps.ny, ps.nz, ps.lr);
@@ -818,7 +844,9 @@ hipError_t launch_plane_hash(const PlaneShape &ps, const void *planes, const Pla
 }
 
 size_t plane_word(const PlaneShape &ps, int x, int y, int z) {
-  return ((size_t)(z + 1) * (u32)(ps.ny + 1) + (u32)(y + 1)) * (u32)ps.lr + (u32)(x >> 6);
+  const size_t lr = (size_t)ps.lr, row = (size_t)(y + 1);
+  if (ps.tiled) return (((size_t)(z + 1) * plane_tiles(ps) + row / 8) * lr + (size_t)(x >> 6)) * 8 + row % 8;
+  return ((size_t)(z + 1) * (size_t)(ps.ny + 1) + row) * lr + (size_t)(x >> 6);
 }
 
 size_t plane_cell_flags(const PlaneShape &ps, int y, int z, int *n) {
