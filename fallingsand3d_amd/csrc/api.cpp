@@ -338,19 +338,26 @@ int enqueue_planes(fs3d_world *w, int nticks, int hash_every, const u64 *tick_de
   const PlaneShape ps = shape_of(w);
   const bool items = item_ticks(w);
   int src = w->planes_valid ? w->pcur : 0, f = w->fcur;
-  bool fresh = !w->planes_valid || !w->pflags_valid;
-  if (launch && !w->planes_valid) {
+  // an even first tick is done while packing
+  const bool packs = !w->planes_valid, ticks_too = packs && !(w->tick & 1u);
+  int first = ticks_too ? kAfterPackTick : packs || !w->pflags_valid ? kAfterPack : kNotFirst;
+  if (launch && packs) {
     FS3D_HIP(launch_fill_u32(w->d_reserved, 1, 0, w->stream));
-    FS3D_HIP(launch_plane_pack(ps, w->buf[w->cur], w->planes[src], w->d_reserved, w->stream));
+    if (ticks_too)
+      FS3D_HIP(launch_plane_pack_even(ps, w->buf[w->cur], w->planes[src], w->d_reserved, w->tick, tick_dev, 0,
+                                      items ? w->pflags[f] : nullptr, w->planes[src ^ 1], w->stream));
+    else
+      FS3D_HIP(launch_plane_pack(ps, w->buf[w->cur], w->planes[src], w->d_reserved, w->stream));
   }
-  if (launch && items && fresh)
+  if (launch && items && first == kAfterPack)
     FS3D_HIP(launch_fill_u64(w->pflags[f], plane_cells(ps).flag_words, ~0ull, w->stream));
   auto hashed_after = [&](int k) { return hash_every > 0 && (k + 1) % hash_every == 0; };
   const bool direct = plane_hash_direct(ps);
   if (launch && direct && hash_every > 0 && nticks >= hash_every)
     FS3D_HIP(launch_fill_u64(w->d_small + 1, (size_t)(nticks / hash_every), 0, w->stream));
   PlaneHash hash{w->buf[w->cur], w->d_reserved, w->d_parts, nullptr};  // out: due for planes[src]
-  for (int k = 0; k < nticks;) {
+  if (ticks_too && hashed_after(0)) hash.out = w->d_small + 1;
+  for (int k = ticks_too ? 1 : 0; k < nticks;) {
     const u64 t = w->tick + (u64)k;
     const bool pair = (t & 1u) && k + 1 < nticks && !hashed_after(k);
     if (launch) {
@@ -358,7 +365,7 @@ int enqueue_planes(fs3d_world *w, int nticks, int hash_every, const u64 *tick_de
       const bool with = hash.out && !items && !pair;
       if (hash.out && !with) FS3D_HIP(launch_plane_hash(ps, w->planes[src], hash, w->stream));
       if (items)
-        FS3D_HIP(launch_plane_list(ps, w->planes[src], w->planes[src ^ 1], t, tick_dev, (u32)k, pair, fresh,
+        FS3D_HIP(launch_plane_list(ps, w->planes[src], w->planes[src ^ 1], t, tick_dev, (u32)k, pair, first,
                                    w->pflags[f], w->pflags[f ^ 1], w->d_since, w->d_items, w->d_nitems,
                                    w->item_waves, w->stream));
       else if (pair)
@@ -370,7 +377,7 @@ int enqueue_planes(fs3d_world *w, int nticks, int hash_every, const u64 *tick_de
     }
     src ^= 1;
     f ^= 1;
-    fresh = false;
+    first = kNotFirst;
     k += pair ? 2 : 1;
     hash.out = hashed_after(k - 1) ? w->d_small + k / hash_every : nullptr;
   }

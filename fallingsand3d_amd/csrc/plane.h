@@ -20,8 +20,9 @@ struct PlaneShape {
 inline PlaneShape plane_shape(int nx, int ny, int nz, bool tiled = false) {
   return PlaneShape{nx, ny, nz, (nx + 63) / 64, tiled};
 }
-// Tiles along y: rows -1 .. ny + 1 of a layer.
-inline int plane_tiles(const PlaneShape &p) { return (p.ny + 2) / 8 + 1; }
+// Tiles along y: one before row 0, so that four strips of an even tick's row quads are
+// a tile, and rows 0 .. ny + 1.
+inline int plane_tiles(const PlaneShape &p) { return (p.ny + 9) / 8 + 1; }
 // 16-byte words of a plane grid with the zero rows around it.
 inline size_t plane_words(const PlaneShape &p) {
   if (p.tiled) return (size_t)p.lr * 8 * (size_t)plane_tiles(p) * (size_t)(p.nz + 2);
@@ -62,6 +63,11 @@ hipError_t launch_plane_pad(const PlaneShape &ps, void *planes, hipStream_t s);
 // Bytes (values >= 4 as STATIC, *reserved set) to planes and back (with *reserved,
 // bytes >= 4 already in g stay).
 hipError_t launch_plane_pack(const PlaneShape &ps, const u8 *g, void *planes, u32 *reserved, hipStream_t s);
+// Packing and the even tick t on it: planes hold the state after the tick, flags
+// (of items; or nullptr) what the next pass needs with kAfterPackTick; other: the
+// buffer that it will write.
+hipError_t launch_plane_pack_even(const PlaneShape &ps, const u8 *g, void *planes, u32 *reserved, u64 t,
+                                  const u64 *tick_dev, u32 k_off, u64 *flags, void *other, hipStream_t s);
 hipError_t launch_plane_unpack(const PlaneShape &ps, const void *planes, u8 *g, const u32 *reserved, hipStream_t s);
 
 // The word that holds a cell.
@@ -81,10 +87,12 @@ size_t plane_cell_flags(const PlaneShape &ps, int y, int z, int *n);
 int plane_list_blocks_per_cu();
 // A pass over the active items: ticks t and t + 1 (pair, t odd) or tick t (of
 // either parity; *tick_dev + k_off has t's).  flags_in: the pass before; flags_out:
-// this one's; since: items changed since the bytes were written; fresh: the first
-// pass after packing (every flag set).
+// this one's; since: items changed since the bytes were written; first: kAfterPack
+// for the first pass after packing (every flag set), kAfterPackTick for the first one
+// after launch_plane_pack_even.
+enum { kNotFirst = 0, kAfterPack, kAfterPackTick };
 hipError_t launch_plane_list(const PlaneShape &ps, const void *src, void *dst, u64 t, const u64 *tick_dev, u32 k_off,
-                             bool pair, bool fresh, const u64 *flags_in, u64 *flags_out, u64 *since, u32 *list,
+                             bool pair, int first, const u64 *flags_in, u64 *flags_out, u64 *since, u32 *list,
                              u32 *count, u32 nwaves, hipStream_t s);
 // Writes the bytes of the items in since or flags (the last pass's) and clears since;
 // dirty (or nullptr): a bit per 8^3 brick, set for those that hold a written item.

@@ -73,7 +73,7 @@ __device__ __forceinline__ u32 place(const LayerArgs &a, u32 i, u32 per, u32 *se
   *sub = rest % per;
   const u32 w = rest / per;
   *seg = a.tiled ? w >> 3 : w;
-  return a.tiled ? 8u * q + (w & 7u) - 1u : q;
+  return a.tiled ? 8u * q + (w & 7u) - 8u : q;
 }
 
 // First word of a layer.
@@ -293,7 +293,7 @@ enum { kAny = 0, kXFirst, kXLast, kYFirst, kYLast, kZFirst, kZLast, kNow, kFlags
 // lane evaluates the half blocks at the row's end.
 __global__ __launch_bounds__(256) void plane_plan_kernel(const u64 *__restrict__ in, u64 *__restrict__ out,
                                                          u64 *__restrict__ since, int strips, int zcells, int lr,
-                                                         int virt, int carry, int fresh, u32 *list, u32 *count) {
+                                                         int virt, int carry, int first, u32 *list, u32 *count) {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int ncell = strips * zcells;
   const int c = (int)blockIdx.x * 256 + (int)threadIdx.x;
@@ -311,15 +311,20 @@ __global__ __launch_bounds__(256) void plane_plan_kernel(const u64 *__restrict__
         if (y < 0 || y >= strips || z < 0 || z >= zcells) continue;
         const u64 *f = in + (size_t)(z * strips + y) * kFlags;
         u64 m = f[kAny];
+        if (first == kAfterPackTick) {  // what can move in an item may touch all its sides
+          act |= m | (m >> 1) | (m << 1);
+          continue;
+        }
         if (dy) m &= f[dy > 0 ? kYFirst : kYLast];
         if (dz) m &= f[dz > 0 ? kZFirst : kZLast];
         act |= m | ((m & f[kXFirst]) >> 1) | ((m & f[kXLast]) << 1);
       }
     act &= bits;
     const u64 *f = in + (size_t)c * kFlags;
-    since[c] = fresh ? 0ull : since[c] | f[kNow];
+    since[c] = first == kAfterPack ? 0ull : first == kAfterPackTick ? f[kNow] : since[c] | f[kNow];
 #pragma unroll
-    for (int i = 0; i < kFlags; i++) out[(size_t)c * kFlags + i] = carry && i != kNow ? f[i] : 0ull;
+    for (int i = 0; i < kFlags; i++)
+      out[(size_t)c * kFlags + i] = carry && i != kNow ? f[first == kAfterPackTick ? kAny : i] : 0ull;
   }
   const int n = __builtin_popcountll(act) + (virt && ((act >> (lr - 1)) & 1u) ? 1 : 0);
   int incl = n;
@@ -363,7 +368,7 @@ __global__ __launch_bounds__(256) void plane_list_kernel(PlaneArgs a, const u32 
   const u32 t = (u32)tick_of(a);
   const u32 n = *count;
   const Planes src(a.src, a.bytes), dst(a.dst, a.bytes);
-  const u32 tile = (u32)a.lr * 128u, layer = tile * (u32)((a.ny + 2) / 8 + 1);
+  const u32 tile = (u32)a.lr * 128u, layer = tile * (u32)((a.ny + 9) / 8 + 1);
   const int m = a.zlen;
   const int prev = (lane ? lane - 1 : 0) * 4, next = (lane < 63 ? lane + 1 : 63) * 4;
   for (u32 w = wave; w * 62u < n; w += nwaves) {
@@ -379,11 +384,11 @@ __global__ __launch_bounds__(256) void plane_list_kernel(PlaneArgs a, const u32 
     const bool has_next = in && lane < 63 && seg + 1 < (int)per && cn == code + 1u;
     const bool word = in && seg < a.lr;  // not the virtual word
     const bool mine = word && lane > 0 && lane < 63;
-    // rows y0 - 1 + 2 i and the one after, of layer z0 - 1
-    u32 off[K + 1];
+    // rows y0 - 2 + 2 i and the one after, of layer z0 - 1
+    u32 off[K + 2];
 #pragma unroll
-    for (int i = 0; i <= K; i++) {
-      const u32 pr = (u32)(st * K + i);  // pair of rows: four to a tile
+    for (int i = 0; i < K + 2; i++) {
+      const u32 pr = (u32)(st * K + i + 3);  // pair of rows: four to a tile
       off[i] = word ? (u32)z0 * layer + (pr >> 2) * tile + (u32)seg * 128u + (pr & 3u) * 32u : kOutside;
     }
     bool on[2 * K];
@@ -440,19 +445,19 @@ __global__ __launch_bounds__(256) void plane_list_kernel(PlaneArgs a, const u32 
           u32x4 q[4];
 #pragma unroll
           for (int r = 0; r < 4; r++)
-            q[r] = src.load(off[j + (r & 1)], base + (r & 1 ? 0u : 16u) + (r >> 1 ? layer : 0u));
+            q[r] = src.load(off[j + 1], base + (r & 1 ? 16u : 0u) + (r >> 1 ? layer : 0u));
           const u32 c = quad_even(q, (u32)seg, variant_base((u32)(by0 + j), (u32)(bz0 + b), t));
           note(c, 2 * j, 2 * b, j == 0, j == K - 1, b == 0, b == m - 1);
 #pragma unroll
           for (int r = 0; r < 4; r++)
             dst.store(on[2 * j + (r & 1)] && 2 * b + (r >> 1) < zleft,
-                      off[j + (r & 1)] + (base + (r & 1 ? 0u : 16u) + (r >> 1 ? layer : 0u)), q[r]);
+                      off[j + 1] + (base + (r & 1 ? 16u : 0u) + (r >> 1 ? layer : 0u)), q[r]);
         }
     } else {
       u32x4 top[2 * K], nx[4];
       u32 base = 0;  // layer 2 s - 1
 #pragma unroll
-      for (int r = 0; r < 4; r++) nx[r] = src.load(off[0], (r & 1 ? 16u : 0u) + (r >> 1 ? layer : 0u));
+      for (int r = 0; r < 4; r++) nx[r] = src.load(off[r & 1], (r & 1 ? 0u : 16u) + (r >> 1 ? layer : 0u));
 #pragma unroll 1
       for (int s = 0; s <= m; s++, base += 2u * layer) {
         u32x4 lowp, upp;
@@ -464,7 +469,7 @@ __global__ __launch_bounds__(256) void plane_list_kernel(PlaneArgs a, const u32 
           const u32 at = i < K ? base : base + 2u * layer;
 #pragma unroll
           for (int r = 0; r < 4; r++)
-            nx[r] = src.load(off[i < K ? i + 1 : 0], at + (r & 1 ? 16u : 0u) + (r >> 1 ? layer : 0u));
+            nx[r] = src.load(off[(i < K ? i + 1 : 0) + (r & 1)], at + (r & 1 ? 0u : 16u) + (r >> 1 ? layer : 0u));
           __builtin_amdgcn_sched_barrier(0);
           const u32 c = odd(q, i, s);
           note(c, 2 * i - 1, 2 * s - 1, i == 0, i == K, s == 0, s == m);
@@ -475,7 +480,7 @@ __global__ __launch_bounds__(256) void plane_list_kernel(PlaneArgs a, const u32 
               const int dy = 2 * i - 1 + (r & 1), dz = 2 * s - 1 + (r >> 1);
               if (dy >= 0 && dy < 2 * K)
                 dst.store(on[dy] && (unsigned)dz < (unsigned)min(2 * m, zleft),
-                          off[i] + (base + (r & 1 ? 16u : 0u) + (r >> 1 ? layer : 0u)), q[r]);
+                          off[i + (r & 1)] + (base + (r & 1 ? 0u : 16u) + (r >> 1 ? layer : 0u)), q[r]);
             }
           } else {
             if (i > 0) {
@@ -486,7 +491,7 @@ __global__ __launch_bounds__(256) void plane_list_kernel(PlaneArgs a, const u32 
 #pragma unroll
                 for (int r = 0; r < 4; r++)
                   dst.store(on[2 * i - 2 + (r & 1)] && 2 * s - 2 + (r >> 1) < zleft,
-                            off[i - 1 + (r & 1)] + (base - layer + (r & 1 ? 0u : 16u) + (r >> 1 ? layer : 0u)), v[r]);
+                            off[i] + (base - layer + (r & 1 ? 16u : 0u) + (r >> 1 ? layer : 0u)), v[r]);
               }
               top[2 * i - 2] = upp;
               top[2 * i - 1] = q[2];
@@ -530,6 +535,69 @@ __global__ __launch_bounds__(256) void plane_pack_kernel(const u8 *g, u32x4 *out
     // loads may run up to 63 bytes past the last row, into the guard bytes
     const u32x4 v = word_from_bytes(g + ((size_t)z * (u32)a.ny + y) * (u32)a.nx + (u32)x0, min(64, a.nx - x0), &any);
     if (in) out[layer_word(a, z) + i] = v;
+  }
+  if (__any(any) && (threadIdx.x & 63) == 0) *reserved = 1u;
+}
+
+// Packing and the tick after it in one pass, for an even tick t, whose blocks lie in
+// their words: the planes are written once instead of written, read and written.  A
+// lane packs and ticks one word of m row quads along z.  flags (of items, 0 before; or
+// nullptr): kNow where a cell changed, kAny where one is sand or fluid and so may; the
+// next pass then leaves items alone that it did not write, so what cannot move goes to
+// its destination (a.src) too.
+//
+// Bound by memory: 2048^3 in 2.30 ms, 12.9 GB at 5.6 TB/s (packing alone takes 2.15, the
+// tick after it took 1.95, and the pair after that 2.3 where it now takes 0.13).  Lines
+// of tiles are written whole by a wave: with the tiles one row further up, so that each
+// wave wrote 7/8 of its lines, it took 4.2.
+template <bool TILED>
+__global__ __launch_bounds__(256) void plane_pack_even_kernel(const u8 *g, int nx, PlaneArgs a, int m, int strips,
+                                                              u64 *flags, u32 *reserved) {
+  const u32 t = (u32)tick_of(a);
+  const Planes dst(a.dst, a.bytes), other(a.src, a.bytes);
+  const int nzq = (a.nz + 1) >> 1;
+  const u32 i = blockIdx.x * 256u + threadIdx.x, lr = (u32)a.lr;
+  // rows: words along a row; tiles: a tile's four strips of a word, so that its lines
+  // are written whole
+  const u32 over = i / (TILED ? 4u * lr : lr), rest = i - over * (TILED ? 4u * lr : lr);
+  const u32 st = TILED ? 4u * over + (rest & 3u) : over, seg = TILED ? rest >> 2 : rest;
+  const u32 tiles = (u32)(a.ny + 9) / 8u + 1u;
+  const int y0 = 2 * (int)st;
+  const bool in = y0 < a.ny;
+  bool any = false;
+  for (int zr = (int)blockIdx.y; zr * m < nzq; zr += (int)gridDim.y) {
+    u32 acc = 0, mobile = 0;
+    for (int zq = zr * m; zq < min((zr + 1) * m, nzq); zq++) {
+      u32x4 q[4];
+      u32 off[4];
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int y = y0 + (r & 1), z = 2 * zq + (r >> 1);
+        const bool ok = in && y < a.ny && z < a.nz;
+        const u32 row = (u32)(y + (TILED ? 8 : 1));
+        const u32 word = TILED ? (((u32)(z + 1) * tiles + (row >> 3)) * lr + seg) * 8u + (row & 7u)
+                               : ((u32)(z + 1) * (u32)(a.ny + 1) + row) * lr + seg;
+        off[r] = ok ? word * 16u : kOutside;
+        q[r] = word_from_bytes(ok ? g + ((size_t)z * (u32)a.ny + (u32)y) * (u32)nx + 64u * seg : g,
+                               ok ? min(64, nx - 64 * (int)seg) : 0, &any);
+      }
+      acc |= quad_even(q, seg, variant_base(st, (u32)zq, t));
+      u32 high = 0;
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        high |= q[r].z | q[r].w;
+        dst.store(off[r], q[r]);
+      }
+      mobile |= high;
+      if (flags)  // an item in which nothing can move may be left alone by the next pass
+#pragma unroll
+        for (int r = 0; r < 4; r++) other.store(high == 0, off[r], q[r]);
+    }
+    if (flags && in) {
+      unsigned long long *f = (unsigned long long *)(flags + ((size_t)zr * (u32)strips + st) * kFlags);
+      if (acc) atomicOr(f + kNow, 1ull << seg);
+      if (mobile) atomicOr(f + kAny, 1ull << seg);
+    }
   }
   if (__any(any) && (threadIdx.x & 63) == 0) *reserved = 1u;
 }
@@ -597,7 +665,7 @@ __global__ __launch_bounds__(256) void plane_unpack_cells_kernel(const u32x4 *in
         const int y = st * rows + dy;
         if (y < ny) {
           u32 d[4];
-          const u32 row = (u32)(y + 1);  // (tiled planes)
+          const u32 row = (u32)(y + 8);  // (tiled planes)
           unpack_quarter(in[(size_t)(z + 1) * layer + ((row >> 3) * (u32)lr + (u32)seg) * 8u + (row & 7u)], q, d);
           store_quarter(g + ((size_t)z * (u32)ny + (u32)y) * (u32)nx + (u32)x0, m, d, keep);
         }
@@ -634,7 +702,7 @@ static void fill_args(PlaneArgs &a, const PlaneShape &ps) {
 static LayerArgs layer_args(const PlaneShape &ps, int per, dim3 *grid) {
   const u64 rows = ps.tiled ? (u64)plane_tiles(ps) : (u64)ps.ny;
   const u64 d = (u64)per * (u64)ps.lr * (ps.tiled ? 8 : 1), n = d * rows;
-  LayerArgs a{ps.nx, ps.ny, ps.nz, ps.lr, 0, (u32)(n / (u64)per), plane_word(ps, 0, ps.tiled ? -1 : 0, 0),
+  LayerArgs a{ps.nx, ps.ny, ps.nz, ps.lr, 0, (u32)(n / (u64)per), plane_word(ps, 0, ps.tiled ? -8 : 0, 0),
               plane_word(ps, 0, 0, 1) - plane_word(ps, 0, 0, 0), ps.tiled};
   if (n * d < (1ull << 32) && d > 1) a.magic = (u32)(((1ull << 32) + d - 1) / d);
   const unsigned gx = (unsigned)((n + 255) / 256);
@@ -774,7 +842,7 @@ int plane_list_blocks_per_cu() {
 }
 
 hipError_t launch_plane_list(const PlaneShape &ps, const void *src, void *dst, u64 t, const u64 *tick_dev, u32 k_off,
-                             bool pair, bool fresh, const u64 *flags_in, u64 *flags_out, u64 *since, u32 *list,
+                             bool pair, int first, const u64 *flags_in, u64 *flags_out, u64 *since, u32 *list,
                              u32 *count, u32 nwaves, hipStream_t s) {
   PlaneArgs a{};
   fill_args(a, ps);
@@ -789,7 +857,7 @@ hipError_t launch_plane_list(const PlaneShape &ps, const void *src, void *dst, u
   hipError_t e = launch_fill_u32(count, 1, 0, s);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(plane_plan_kernel, dim3(plan), dim3(256), 0, s, flags_in, flags_out, since, c.strips, c.zcells,
-                     ps.lr, c.virt, pair ? 0 : 1, fresh ? 1 : 0, list, count);
+                     ps.lr, c.virt, pair ? 0 : 1, first, list, count);
   const dim3 grid(nwaves / 4);
   // the caller's t has the tick's parity, on replays too
   if (pair)
@@ -830,6 +898,32 @@ hipError_t launch_plane_pack(const PlaneShape &ps, const u8 *g, void *planes, u3
   return hipGetLastError();
 }
 
+hipError_t launch_plane_pack_even(const PlaneShape &ps, const u8 *g, void *planes, u32 *reserved, u64 t,
+                                  const u64 *tick_dev, u32 k_off, u64 *flags, void *other, hipStream_t s) {
+  PlaneArgs a{};
+  fill_args(a, ps);
+  a.src = static_cast<const u32x4 *>(flags ? other : planes);
+  a.dst = static_cast<u32x4 *>(planes);
+  a.t = t;
+  a.tick_dev = tick_dev;
+  a.k_off = k_off;
+  const PlaneCells c = plane_cells(ps);
+  if (flags) {
+    const hipError_t e = launch_fill_u64(flags, c.flag_words, 0, s);
+    if (e != hipSuccess) return e;
+  }
+  const int nyq = (ps.ny + 1) >> 1, nzq = (ps.nz + 1) >> 1;
+  const u32 gx = (u32)(((u64)(ps.tiled ? (nyq + 3) / 4 * 4 : nyq) * (u64)ps.lr + 255) / 256);
+  // items' layers, or what keeps the chip busy
+  const int m = flags ? kItemLayers : (int)std::min<u64>(8, std::max<u64>(1, (u64)gx * (u64)nzq / 4096));
+  const dim3 grid(gx, (unsigned)std::min((nzq + m - 1) / m, 65535));
+  if (ps.tiled)
+    hipLaunchKernelGGL(plane_pack_even_kernel<true>, grid, dim3(256), 0, s, g, ps.nx, a, m, c.strips, flags, reserved);
+  else
+    hipLaunchKernelGGL(plane_pack_even_kernel<false>, grid, dim3(256), 0, s, g, ps.nx, a, m, c.strips, flags, reserved);
+  return hipGetLastError();
+}
+
 hipError_t launch_plane_unpack(const PlaneShape &ps, const void *planes, u8 *g, const u32 *reserved, hipStream_t s) {
   dim3 grid;
   const LayerArgs a = layer_args(ps, 4, &grid);
@@ -844,9 +938,9 @@ hipError_t launch_plane_hash(const PlaneShape &ps, const void *planes, const Pla
 }
 
 size_t plane_word(const PlaneShape &ps, int x, int y, int z) {
-  const size_t lr = (size_t)ps.lr, row = (size_t)(y + 1);
-  if (ps.tiled) return (((size_t)(z + 1) * plane_tiles(ps) + row / 8) * lr + (size_t)(x >> 6)) * 8 + row % 8;
-  return ((size_t)(z + 1) * (size_t)(ps.ny + 1) + row) * lr + (size_t)(x >> 6);
+  const size_t lr = (size_t)ps.lr, t = (size_t)(y + 8);
+  if (ps.tiled) return (((size_t)(z + 1) * plane_tiles(ps) + t / 8) * lr + (size_t)(x >> 6)) * 8 + t % 8;
+  return ((size_t)(z + 1) * (size_t)(ps.ny + 1) + (size_t)(y + 1)) * lr + (size_t)(x >> 6);
 }
 
 size_t plane_cell_flags(const PlaneShape &ps, int y, int z, int *n) {
