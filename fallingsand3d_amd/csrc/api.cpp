@@ -308,7 +308,8 @@ bool ensure_planes(fs3d_world *w) {
     w->item_waves = (u32)(std::max(cus, 1) * plane_list_blocks_per_cu() * 4);
     for (int i = 0; i < 2 && e == hipSuccess; i++) e = hipMalloc(&w->pflags[i], c.flag_words * sizeof(u64));
     if (e == hipSuccess) e = hipMalloc(&w->d_since, c.since_words * sizeof(u64));
-    if (e == hipSuccess) e = hipMalloc(&w->d_nitems, sizeof(u32));
+    if (e == hipSuccess) e = hipMalloc(&w->d_nitems, 2 * sizeof(u32));
+    if (e == hipSuccess) e = launch_fill_u32(w->d_nitems, 2, 0, w->stream);
     if (e == hipSuccess) e = hipMalloc(&w->d_items, c.list_words * sizeof(u32));
   }
   if (e == hipSuccess) return true;
@@ -366,8 +367,8 @@ int enqueue_planes(fs3d_world *w, int nticks, int hash_every, const u64 *tick_de
       if (hash.out && !with) FS3D_HIP(launch_plane_hash(ps, w->planes[src], hash, w->stream));
       if (items)
         FS3D_HIP(launch_plane_list(ps, w->planes[src], w->planes[src ^ 1], t, tick_dev, (u32)k, pair, first,
-                                   w->pflags[f], w->pflags[f ^ 1], w->d_since, w->d_items, w->d_nitems,
-                                   w->item_waves, w->stream));
+                                   w->pflags[f], w->pflags[f ^ 1], w->d_since, w->d_items, w->d_nitems + f,
+                                   w->d_nitems + (f ^ 1), w->item_waves, w->stream));
       else if (pair)
         FS3D_HIP(launch_plane_pair(ps, w->planes[src], w->planes[src ^ 1], t, tick_dev, (u32)k, w->stream));
       else
@@ -659,7 +660,7 @@ int fs3d_world_set_voxel(fs3d_world *w, int32_t x, int32_t y, int32_t z, uint8_t
     e.reserved = w->d_reserved;
     e.word = plane_word(ps, x, y, z);
     e.x = x;
-    if (w->pflags_valid) e.flags = w->pflags[w->fcur] + plane_cell_flags(ps, y, z, &e.nflags);
+    if (w->pflags_valid) e.flags = w->pflags[w->fcur] + plane_cell_flags(ps, y, z, &e.nflags, &e.flag_stride);
   }
   w->occ_valid = false;
   FS3D_HIP(launch_set_cell(e, next_note(w), w->stream));

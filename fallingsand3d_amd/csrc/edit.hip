@@ -24,7 +24,7 @@ __global__ void set_cell_kernel(CellEdit e, Note n) {
     e.masks[p][e.edge_off + e.idx[p]] |= e.bits | (e.bits << 1);
   }
   if (e.planes) {
-    for (int i = 0; i < e.nflags; i++) e.flags[i] |= 1ull << (e.x >> 6);
+    for (int i = 0; i < e.nflags; i++) e.flags[i * e.flag_stride] |= 1ull << (e.x >> 6);
     if (e.value >= 4u) *e.reserved = 1u;
     const u32 code = (e.value >= 4u ? (u32)FS3D_STATIC : e.value) ^ 1u;
     u32 *w = e.planes + 4 * e.word + (e.x & 1);

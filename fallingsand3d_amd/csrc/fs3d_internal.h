@@ -146,7 +146,7 @@ constexpr size_t kHashPostMax = 1u << 18;
 hipError_t launch_hash_post(const u8 *g, size_t n, u64 *hash_parts, const Note &note, hipStream_t s);
 // One cell set by the host: its byte, change bits `bits` of row quad idx[p] at either
 // parity and the edge bits next to them (edge words at offset edge_off), and, with
-// planes, its bits there and the nflags change flags of its item.
+// planes, its bits there and the nflags change flags (flag_stride apart) of its item.
 struct CellEdit {
   u8 *cell;
   u32 value;
@@ -158,6 +158,7 @@ struct CellEdit {
   u64 *flags;
   size_t word;
   int x, nflags;
+  size_t flag_stride;
 };
 hipError_t launch_set_cell(const CellEdit &e, const Note &n, hipStream_t s);
 hipError_t launch_post_byte(const u8 *p, const Note &n, hipStream_t s);

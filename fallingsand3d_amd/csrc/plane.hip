@@ -275,7 +275,8 @@ __global__ __launch_bounds__(256) void plane_pair_kernel(PlaneArgs a) {
 // since does not change.  The destination then already holds the item: it is the
 // state of two passes ago.
 //
-// Flags are u64 masks over the words of a strip (bit = word), kFlags per cell: any
+// Flags are u64 masks over the words of a strip (bit = word), kFlags per cell, each flag
+// of all cells in a row (so that the plan's lanes read neighbouring words): any
 // change; a change of a block at the item's first or last word bit, row, layer; any
 // change in the last pass alone.  A flag may be set without need, never missing.
 //
@@ -309,22 +310,28 @@ __global__ __launch_bounds__(256) void plane_plan_kernel(const u64 *__restrict__
       for (int dy = -1; dy <= 1; dy++) {
         const int y = st + dy, z = zr + dz;
         if (y < 0 || y >= strips || z < 0 || z >= zcells) continue;
-        const u64 *f = in + (size_t)(z * strips + y) * kFlags;
+        const u64 *f = in + (z * strips + y);
         u64 m = f[kAny];
+        if (m == 0) continue;
         if (first == kAfterPackTick) {  // what can move in an item may touch all its sides
           act |= m | (m >> 1) | (m << 1);
           continue;
         }
-        if (dy) m &= f[dy > 0 ? kYFirst : kYLast];
-        if (dz) m &= f[dz > 0 ? kZFirst : kZLast];
-        act |= m | ((m & f[kXFirst]) >> 1) | ((m & f[kXLast]) << 1);
+        if (dy) m &= f[(size_t)(dy > 0 ? kYFirst : kYLast) * ncell];
+        if (dz) m &= f[(size_t)(dz > 0 ? kZFirst : kZLast) * ncell];
+        act |= m | ((m & f[(size_t)kXFirst * ncell]) >> 1) | ((m & f[(size_t)kXLast * ncell]) << 1);
       }
     act &= bits;
-    const u64 *f = in + (size_t)c * kFlags;
-    since[c] = first == kAfterPack ? 0ull : first == kAfterPackTick ? f[kNow] : since[c] | f[kNow];
+    const u64 *f = in + c;
+    const u64 now = first == kAfterPack ? 0ull : f[(size_t)kNow * ncell];
+    if (first != kNotFirst)
+      since[c] = now;
+    else if (now)
+      since[c] |= now;
 #pragma unroll
     for (int i = 0; i < kFlags; i++)
-      out[(size_t)c * kFlags + i] = carry && i != kNow ? f[first == kAfterPackTick ? kAny : i] : 0ull;
+      out[(size_t)i * ncell + c] =
+          carry && i != kNow ? f[(size_t)(first == kAfterPackTick ? kAny : i) * ncell] : 0ull;
   }
   const int n = __builtin_popcountll(act) + (virt && ((act >> (lr - 1)) & 1u) ? 1 : 0);
   int incl = n;
@@ -362,8 +369,10 @@ enum { kPair = 0, kOdd, kEven };
 // those cells there blocks the moves among the others).
 template <int MODE, int K>
 __global__ __launch_bounds__(256) void plane_list_kernel(PlaneArgs a, const u32 *__restrict__ list, const u32 *count,
-                                                         u64 *flags, int strips, int virt, u32 nwaves) {
+                                                         u64 *flags, u32 *next_count, int strips, int ncell, int virt,
+                                                         u32 nwaves) {
   const int lane = threadIdx.x & 63;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *next_count = 0;
   const u32 wave = blockIdx.x * 4 + (u32)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const u32 t = (u32)tick_of(a);
   const u32 n = *count;
@@ -515,7 +524,7 @@ __global__ __launch_bounds__(256) void plane_list_kernel(PlaneArgs a, const u32 
       const u64 b = __ballot(mine && acc[f] != 0u);
       const u64 bits = ((b >> lane) & run) << (seg & 63);
       if (!has_prev && in && bits)
-        atomicOr((unsigned long long *)(flags + (size_t)cell * kFlags + f), (unsigned long long)bits);
+        atomicOr((unsigned long long *)(flags + (size_t)f * ncell + cell), (unsigned long long)bits);
     }
   }
 }
@@ -552,7 +561,7 @@ __global__ __launch_bounds__(256) void plane_pack_kernel(const u8 *g, u32x4 *out
 // wave wrote 7/8 of its lines, it took 4.2.
 template <bool TILED>
 __global__ __launch_bounds__(256) void plane_pack_even_kernel(const u8 *g, int nx, PlaneArgs a, int m, int strips,
-                                                              u64 *flags, u32 *reserved) {
+                                                              int ncell, u64 *flags, u32 *reserved) {
   const u32 t = (u32)tick_of(a);
   const Planes dst(a.dst, a.bytes), other(a.src, a.bytes);
   const int nzq = (a.nz + 1) >> 1;
@@ -594,9 +603,9 @@ __global__ __launch_bounds__(256) void plane_pack_even_kernel(const u8 *g, int n
         for (int r = 0; r < 4; r++) other.store(high == 0, off[r], q[r]);
     }
     if (flags && in) {
-      unsigned long long *f = (unsigned long long *)(flags + ((size_t)zr * (u32)strips + st) * kFlags);
-      if (acc) atomicOr(f + kNow, 1ull << seg);
-      if (mobile) atomicOr(f + kAny, 1ull << seg);
+      unsigned long long *f = (unsigned long long *)(flags + ((size_t)zr * (u32)strips + st));
+      if (acc) atomicOr(f + (size_t)kNow * ncell, 1ull << seg);
+      if (mobile) atomicOr(f + (size_t)kAny * ncell, 1ull << seg);
     }
   }
   if (__any(any) && (threadIdx.x & 63) == 0) *reserved = 1u;
@@ -647,7 +656,7 @@ __global__ __launch_bounds__(256) void plane_unpack_cells_kernel(const u32x4 *in
   const int lane = threadIdx.x & 63;
   const int c = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   if (c >= ncell) return;
-  const u64 bits = since[c] | flags[(size_t)c * kFlags + kNow];
+  const u64 bits = since[c] | flags[(size_t)kNow * ncell + c];
   if (bits == 0) return;
   const bool keep = *reserved != 0;
   const int zr = c / strips, st = c - zr * strips;
@@ -843,7 +852,7 @@ int plane_list_blocks_per_cu() {
 
 hipError_t launch_plane_list(const PlaneShape &ps, const void *src, void *dst, u64 t, const u64 *tick_dev, u32 k_off,
                              bool pair, int first, const u64 *flags_in, u64 *flags_out, u64 *since, u32 *list,
-                             u32 *count, u32 nwaves, hipStream_t s) {
+                             u32 *count, u32 *next_count, u32 nwaves, hipStream_t s) {
   PlaneArgs a{};
   fill_args(a, ps);
   a.src = static_cast<const u32x4 *>(src);
@@ -854,21 +863,19 @@ hipError_t launch_plane_list(const PlaneShape &ps, const void *src, void *dst, u
   a.zlen = kItemLayers;
   const PlaneCells c = plane_cells(ps);
   const unsigned plan = (unsigned)((c.since_words + 255) / 256);
-  hipError_t e = launch_fill_u32(count, 1, 0, s);
-  if (e != hipSuccess) return e;
   hipLaunchKernelGGL(plane_plan_kernel, dim3(plan), dim3(256), 0, s, flags_in, flags_out, since, c.strips, c.zcells,
                      ps.lr, c.virt, pair ? 0 : 1, first, list, count);
   const dim3 grid(nwaves / 4);
   // the caller's t has the tick's parity, on replays too
   if (pair)
     hipLaunchKernelGGL((plane_list_kernel<kPair, kItemQuads>), grid, dim3(256), 0, s, a, list, count, flags_out,
-                       c.strips, c.virt, nwaves);
+                       next_count, c.strips, (int)c.since_words, c.virt, nwaves);
   else if (t & 1u)
     hipLaunchKernelGGL((plane_list_kernel<kOdd, kItemQuads>), grid, dim3(256), 0, s, a, list, count, flags_out,
-                       c.strips, c.virt, nwaves);
+                       next_count, c.strips, (int)c.since_words, c.virt, nwaves);
   else
     hipLaunchKernelGGL((plane_list_kernel<kEven, kItemQuads>), grid, dim3(256), 0, s, a, list, count, flags_out,
-                       c.strips, c.virt, nwaves);
+                       next_count, c.strips, (int)c.since_words, c.virt, nwaves);
   return hipGetLastError();
 }
 
@@ -918,9 +925,9 @@ hipError_t launch_plane_pack_even(const PlaneShape &ps, const u8 *g, void *plane
   const int m = flags ? kItemLayers : (int)std::min<u64>(8, std::max<u64>(1, (u64)gx * (u64)nzq / 4096));
   const dim3 grid(gx, (unsigned)std::min((nzq + m - 1) / m, 65535));
   if (ps.tiled)
-    hipLaunchKernelGGL(plane_pack_even_kernel<true>, grid, dim3(256), 0, s, g, ps.nx, a, m, c.strips, flags, reserved);
+    hipLaunchKernelGGL(plane_pack_even_kernel<true>, grid, dim3(256), 0, s, g, ps.nx, a, m, c.strips, (int)c.since_words, flags, reserved);
   else
-    hipLaunchKernelGGL(plane_pack_even_kernel<false>, grid, dim3(256), 0, s, g, ps.nx, a, m, c.strips, flags, reserved);
+    hipLaunchKernelGGL(plane_pack_even_kernel<false>, grid, dim3(256), 0, s, g, ps.nx, a, m, c.strips, (int)c.since_words, flags, reserved);
   return hipGetLastError();
 }
 
@@ -943,9 +950,11 @@ size_t plane_word(const PlaneShape &ps, int x, int y, int z) {
   return ((size_t)(z + 1) * (size_t)(ps.ny + 1) + (size_t)(y + 1)) * lr + (size_t)(x >> 6);
 }
 
-size_t plane_cell_flags(const PlaneShape &ps, int y, int z, int *n) {
+size_t plane_cell_flags(const PlaneShape &ps, int y, int z, int *n, size_t *stride) {
+  const PlaneCells c = plane_cells(ps);
   *n = kFlags;
-  return ((size_t)(z / (2 * kItemLayers)) * plane_cells(ps).strips + (size_t)(y / (2 * kItemQuads))) * kFlags;
+  *stride = c.since_words;
+  return (size_t)(z / (2 * kItemLayers)) * c.strips + (size_t)(y / (2 * kItemQuads));
 }
 
 }  // namespace fs3d
