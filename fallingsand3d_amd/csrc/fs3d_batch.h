@@ -24,6 +24,9 @@ struct BWorld {
 __device__ __forceinline__ u8 *grid_of(const BWorld &w) {
   return (u8 *)(__attribute__((address_space(1))) u8 *)(uintptr_t)w.g;
 }
+__device__ __forceinline__ const u8 *grid_at(const u8 *g) {
+  return (const u8 *)(const __attribute__((address_space(1))) u8 *)(uintptr_t)g;
+}
 
 bool batch_config_ok(int seg, int threads, int groups);
 // Workgroups of the persistent kernel that share a CU, the plane words one of
@@ -58,7 +61,16 @@ hipError_t launch_wide(int seg, const BWorld *ents, const long long *bpre, const
                        long long blocks, int k, const u64 *rule, u64 *hashes, hipStream_t s, u32 *chg = nullptr);
 // The same on grids kept as bit planes.
 hipError_t launch_wide_planes(const BWorld *ents, const long long *bpre, const int *blk2ent, long long blk0,
-                              long long blocks, int k, u64 *hashes, hipStream_t s, u32 *chg);
+                              long long blocks, int k, hipStream_t s, u32 *chg);
+// Hashes of the plane grids that finish, added to hashes[slot]: entry i owns workgroups
+// [first, first + hash_blocks(its words)).
+struct HashEntry {
+  const u8 *g;
+  int nx, ny, nz, slot;
+  unsigned first;
+};
+unsigned hash_blocks(size_t words);
+hipError_t launch_wide_hash(const HashEntry *ents, int n, unsigned blocks, u64 *hashes, hipStream_t s);
 // Rain fills of worlds kept as bit planes, 256 plane words per workgroup.
 struct FillEntry {
   u8 *g;

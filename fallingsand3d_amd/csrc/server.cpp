@@ -361,16 +361,26 @@ int launch_round(fs3d_server *s) {
   std::vector<long long> fin;
   for (int i = 0; i < n; i++)
     if (s->reqs[s->active[i]].remaining == ents[i].nt) fin.push_back(s->active[i]);
-  const size_t koff_bytes = sizeof(long long) * (size_t)(K + 1), fin_bytes = sizeof(int) * fin.size();
-  const size_t table_bytes = ent_bytes + pre_bytes + koff_bytes + fin_bytes;
+  const size_t koff_bytes = sizeof(long long) * (size_t)(K + 1), hash_bytes = sizeof(HashEntry) * fin.size();
+  const size_t fin_bytes = sizeof(int) * fin.size();
+  const size_t table_bytes = ent_bytes + pre_bytes + koff_bytes + hash_bytes + fin_bytes;
   if (int rc = ensure_round_cap(rd, table_bytes, blks, (int)fin.size(), K + 1)) return rc;
   std::copy(ents.begin(), ents.end(), (BWorld *)rd.h_buf);
   std::copy(pre.begin(), pre.end(), (long long *)(rd.h_buf + ent_bytes));
   long long *koff = (long long *)(rd.h_buf + ent_bytes + pre_bytes);
   koff[0] = 0;
   for (int k = 0; k < K; k++) koff[k + 1] = koff[k] + tot[k];
-  int *fin_slots = (int *)(rd.h_buf + ent_bytes + pre_bytes + koff_bytes);
-  for (size_t i = 0; i < fin.size(); i++) fin_slots[i] = s->reqs[fin[i]].slot;
+  HashEntry *hash_ents = (HashEntry *)(rd.h_buf + ent_bytes + pre_bytes + koff_bytes);
+  int *fin_slots = (int *)(rd.h_buf + ent_bytes + pre_bytes + koff_bytes + hash_bytes);
+  int n_hash = 0;  // plane grids; the byte kernel hashes as it ticks
+  unsigned hash_blk = 0;
+  for (size_t i = 0; i < fin.size(); i++) {
+    const Request &r = s->reqs[fin[i]];
+    fin_slots[i] = r.slot;
+    if (!planes_fit(r)) continue;
+    hash_ents[n_hash++] = HashEntry{r.g, r.nx, r.ny, r.nz, r.slot, hash_blk};
+    hash_blk += hash_blocks((size_t)((r.nx + 63) / 64) * (size_t)r.ny * (size_t)r.nz);
+  }
   FS3D_HIP(hipMemcpyAsync(rd.d_buf, rd.h_buf, table_bytes, hipMemcpyHostToDevice, s->s_tick));
   const BWorld *d_ents = (const BWorld *)rd.d_buf;
   const long long *d_pre = (const long long *)(rd.d_buf + ent_bytes);
@@ -383,13 +393,15 @@ int launch_round(fs3d_server *s) {
   for (int k = 0; k < K; k++) {
     const long long *pk = d_pre + (size_t)k * (n + 1);
     const long long bp = pre[(size_t)k * (n + 1) + n_planes];  // workgroups of the plane grids
-    FS3D_HIP(launch_wide_planes(d_ents, pk, rd.d_blk + boff, 0, bp, k, s->d_hashes, s->s_tick, s->d_chg));
+    FS3D_HIP(launch_wide_planes(d_ents, pk, rd.d_blk + boff, 0, bp, k, s->s_tick, s->d_chg));
     FS3D_HIP(launch_wide(s->seg, d_ents, pk, rd.d_blk + boff, bp, tot[k] - bp, k, rule, s->d_hashes, s->s_tick,
                          s->d_chg));
     FS3D_HIP(hipEventRecord(rd.ev[k + 1], s->s_tick));
     boff += (size_t)tot[k];
   }
-  FS3D_HIP(launch_gather_hashes(s->d_hashes, (const int *)(rd.d_buf + ent_bytes + pre_bytes + koff_bytes),
+  FS3D_HIP(launch_wide_hash((const HashEntry *)(rd.d_buf + ent_bytes + pre_bytes + koff_bytes), n_hash, hash_blk,
+                            s->d_hashes, s->s_tick));
+  FS3D_HIP(launch_gather_hashes(s->d_hashes, (const int *)(rd.d_buf + ent_bytes + pre_bytes + koff_bytes + hash_bytes),
                                 (int)fin.size(), rd.h_hash, s->s_tick));
   FS3D_HIP(hipEventRecord(rd.done, s->s_tick));
   rd.finishing = fin;

@@ -61,12 +61,17 @@ __global__ __launch_bounds__(256) void wide_kernel(const BWorld *__restrict__ en
 
 // The same tick on grids kept as bit planes, in place: lr and rqpw of an entry
 // count 64-cell words.  A wave holds all rows of its row quads before it stores any.
+// (Final states are hashed by wide_hash_kernel.)
+//
 // Serving 1500 requests of 32-256 cells a side and 10-500 ticks submitted at once:
-// 187 ms with the byte kernel (336 us per launch), 41.5 ms here (69 us).
+// 187 ms with the byte kernel (336 us per launch), 31.3 ms here (44 us).  A launch over
+// all of them takes up to 186 us and reads 0.44 GB; storing every word, changed or not,
+// it took 222.  Several groups of row quads per wave, with the next one's rows loaded
+// ahead, were slower (2: 13 %, 4: 48 %): more waves hide more than longer ones.
 __global__ __launch_bounds__(256) void wide_plane_kernel(const BWorld *__restrict__ ents,
                                                          const long long *__restrict__ bpre,
                                                          const int *__restrict__ blk2ent, long long blk0, int k,
-                                                         u64 *hashes, u32 *chg) {
+                                                         u32 *chg) {
   using namespace planedev;
   const long long blk = blk0 + blockIdx.x;
   const int e = __builtin_amdgcn_readfirstlane(blk2ent[blk]);
@@ -75,12 +80,9 @@ __global__ __launch_bounds__(256) void wide_plane_kernel(const BWorld *__restric
   const int wave = (int)(blk - bpre[e]) * 4 + wid;
   const u32 t = (u32)(w.tick + (u64)k);
   const int p = (int)(t & 1u);
-  const bool final_hash = k + 1 == w.nt && w.fin && hashes;
-  u32 *flags = chg ? chg + (size_t)w.slot * 4 : nullptr;
-  if (flags) {
-    if (wave == 0 && threadIdx.x == 0) flags[(t + 1u) & 3u] = 0;
-    if (!final_hash && flags[(t - 1u) & 3u] == 0 && flags[(t - 2u) & 3u] == 0) return;  // settled world
-  }
+  u32 *flags = chg + (size_t)w.slot * 4;
+  if (wave == 0 && threadIdx.x == 0) flags[(t + 1u) & 3u] = 0;
+  if (flags[(t - 1u) & 3u] == 0 && flags[(t - 2u) & 3u] == 0) return;  // settled world
   const u32 nyq = (u32)(w.ny + p + 1) >> 1, nrq = nyq * ((u32)(w.nz + p + 1) >> 1);
   const u32 q0 = (u32)wave * (u32)w.rqpw;
   if (q0 >= nrq) return;  // wave-uniform; no barriers below
@@ -101,27 +103,57 @@ __global__ __launch_bounds__(256) void wide_plane_kernel(const BWorld *__restric
     r[i] = g.load(off[i]);
   }
   const u32 base = variant_base(yq, zq, t);
+  const int next = (in ? dn : lane) * 4;
   u32 ch;
   if (p)
-    ch = quad_odd<true>(r, (u32)seg, base, (in ? up : lane) * 4, (in ? dn : lane) * 4,
-                        (w.nx & 63) == 0 && seg == 0 ? 1u : 0u);
+    ch = quad_odd<true>(r, (u32)seg, base, (in ? up : lane) * 4, next, (w.nx & 63) == 0 && seg == 0 ? 1u : 0u);
   else
     ch = quad_even(r, (u32)seg, base);
+  // in place: a word is as it was unless a block of it changed, or at odd ticks the
+  // block that it shares with the word after it
+  const u32 after = from_lane(next, ch) & 1u;
+  const bool store = ch != 0 || (p && after);
 #pragma unroll
-  for (int i = 0; i < 4; i++) g.store(off[i], r[i]);
-  if (final_hash) {
-    u64 acc = 0;
-    const int m = min(64, w.nx - 64 * seg);
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      if (off[i] == kOutside) continue;
-      const u64 i0 = ((u64)(z0 + (i >> 1)) * (u64)w.ny + (u64)(y0 + (i & 1))) * (u64)w.nx + (u64)(64 * seg);
-      for (int c = 0; c < 4; c++) acc += hash_quarter(r[i], c, min(16, m - 16 * c), i0 + 16u * (u32)c, nullptr);
-    }
-    acc = wave_sum_u64(acc);
-    if (lane == 0 && acc) atomicAdd((unsigned long long *)(hashes + w.slot), (unsigned long long)acc);
+  for (int i = 0; i < 4; i++) g.store(store, off[i], r[i]);
+  if (__ballot(ch != 0) && lane == 0) flags[t & 3u] = 1;
+}
+
+// State hashes of the plane grids that finish in a round, in one launch: entry i owns
+// workgroups [first[i], first[i + 1]), four lanes per word, two words of them apart.
+// Hashed by the waves of their last tick, at up to 256 mixes in a row per lane, they
+// made every launch in which a request finished take 28 us or more (41.5 ms for the
+// 1500 requests, 37.2 with this: 24 us a round).  A workgroup adds to the entry's hash
+// once: an addition to one word takes it 13 ns.
+constexpr u32 kHashThreads = 1024, kHashWords = 2 * kHashThreads / 4;  // words of a workgroup
+__global__ __launch_bounds__(1024) void wide_hash_kernel(const HashEntry *__restrict__ ents, int n, u64 *hashes) {
+  using namespace planedev;
+  int lo = 0, hi = n;  // first of entry lo <= block < first of entry hi
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (ents[mid].first <= blockIdx.x) lo = mid; else hi = mid;
   }
-  if (flags && __ballot(ch != 0) && lane == 0) flags[t & 3u] = 1;
+  const HashEntry f = ents[__builtin_amdgcn_readfirstlane(lo)];
+  const u32 lr = (u32)((f.nx + 63) >> 6), words = lr * (u32)f.ny * (u32)f.nz;
+  const u32x4 *g = reinterpret_cast<const u32x4 *>(grid_at(f.g));
+  u64 acc = 0;
+#pragma unroll
+  for (u32 k = 0; k < 2; k++) {
+    const u32 i = (blockIdx.x - f.first) * kHashWords + k * (kHashThreads / 4) + (threadIdx.x >> 2);
+    if (i < words) {
+      const u32 row = i / lr, c = 4u * (i - row * lr) + (threadIdx.x & 3u);
+      const u64 i0 = (u64)row * (u64)f.nx + (u64)(16u * c);
+      acc += hash_quarter(g[i], (int)(c & 3u), min(16, f.nx - 16 * (int)c), i0, nullptr);
+    }
+  }
+  __shared__ u64 wsum[kHashThreads / 64];
+  acc = wave_sum_u64(acc);
+  if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    acc = threadIdx.x < kHashThreads / 64 ? wsum[threadIdx.x] : 0;
+    acc = wave_sum_u64(acc);
+    if (threadIdx.x == 0 && acc) atomicAdd((unsigned long long *)(hashes + f.slot), (unsigned long long)acc);
+  }
 }
 
 // Rain fills of newly admitted worlds, all in one launch: entry i owns workgroups
@@ -227,10 +259,17 @@ hipError_t launch_wide(int seg, const BWorld *ents, const long long *bpre, const
 }
 
 hipError_t launch_wide_planes(const BWorld *ents, const long long *bpre, const int *blk2ent, long long blk0,
-                              long long blocks, int k, u64 *hashes, hipStream_t s, u32 *chg) {
+                              long long blocks, int k, hipStream_t s, u32 *chg) {
   if (blocks <= 0) return hipSuccess;
-  hipLaunchKernelGGL(wide_plane_kernel, dim3((unsigned)blocks), dim3(256), 0, s, ents, bpre, blk2ent, blk0, k, hashes,
-                     chg);
+  hipLaunchKernelGGL(wide_plane_kernel, dim3((unsigned)blocks), dim3(256), 0, s, ents, bpre, blk2ent, blk0, k, chg);
+  return hipGetLastError();
+}
+
+unsigned hash_blocks(size_t words) { return (unsigned)((words + kHashWords - 1) / kHashWords); }
+
+hipError_t launch_wide_hash(const HashEntry *ents, int n, unsigned blocks, u64 *hashes, hipStream_t s) {
+  if (n <= 0) return hipSuccess;
+  hipLaunchKernelGGL(wide_hash_kernel, dim3(blocks), dim3(kHashThreads), 0, s, ents, n, hashes);
   return hipGetLastError();
 }
 
