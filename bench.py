@@ -9,16 +9,18 @@ Default run (one JSON line on stdout):
            counts every voxel of every tick.
   parity   every hash of the timed region against the oracle's per-tick hashes of
            the same scene (tests/golden/boxes512_hashes.txt).
-  roofline the timed region: algorithmic bytes actually moved (2 per swept
-           voxel-update, 1 per voxel only read on hash ticks; counted by replaying
-           the same ticks with sweep counters) / device time of the timed graphs
-           (HIP events on the world's stream), against 8.0 TB/s.  "traffic" is
+  roofline the timed region: the bytes its passes move (the world ticks as two bit
+           planes, 0.25 bytes per voxel: read and written by every pass, one or two
+           ticks each, read by every hash, written back as bytes at the end of each
+           run) / device time of the timed graphs (HIP events on the world's
+           stream), against 8.0 TB/s.  The same ticks are replayed on the byte
+           kernels with sweep counters, whose hashes must agree.  "traffic" is
            measured for the same window: this script runs the window again in two
            child processes under rocprofv3 --pmc (FETCH_SIZE, then WRITE_SIZE),
            scaled by the counters of a copy of known size in the same process.
-           "dense" holds the dense tick kernel on the same world; "hbm2048" the
-           dense tick of the 2048^3 pillar scene, whose buffers (2 x 8 GiB) do not
-           fit the 256 MB Infinity Cache: the HBM-bound figure.
+           "dense" holds dense ticks of the same world; "hbm2048" the dense byte
+           tick of the 2048^3 pillar scene, whose buffers (2 x 8 GiB) do not fit
+           the 256 MB Infinity Cache: the HBM-bound figure.
   extra    pillars2048: the 2048^3 pillar scene, skipping, dense and dense fused
            in pairs; pillars2048_render: that scene with a 1920x1080 voxel render
            every 10 ticks; copy: a plain device copy of the same bytes, with
@@ -50,6 +52,7 @@ sys.path.insert(0, ROOT)
 HBM_PEAK = 8.0e12
 XGMI_LINK_BPS = 153e9  # one MI355X xGMI link, per direction (published figure; one GPU here)
 BYTES_PER_UPDATE = 2
+PAIR_BYTES_PER_UPDATE = 0.25  # a pair of plane ticks reads and writes 0.25 bytes per voxel
 HASH_EVERY = 50
 COPY_CAL_BYTES = 1 << 30  # the known-size copy that scales the byte counters
 GOLDEN = os.path.join(ROOT, "tests", "golden")
@@ -112,13 +115,32 @@ def timed_boxes_window(w, warmup, steps):
     return wall, dev / steps, hashes, ticks
 
 
+def plane_passes(start, steps):
+    """Passes over the planes in timed_boxes_window's runs: a pair of ticks from an
+    odd one on, single ticks elsewhere and before a hash that falls between the two."""
+    n, t = 0, start
+    for nt, he in hash_segments(steps):
+        k = 0
+        while k < nt:
+            k += 2 if (t + k) & 1 and k + 1 < nt and (k + 1) % he else 1
+            n += 1
+        t += nt
+    return n
+
+
+def plane_bytes(vox, start, steps):
+    """Bytes of those passes, of the hashes and of the runs' write-back as bytes."""
+    segs = hash_segments(steps)
+    hashes = sum(nt // he for nt, he in segs)
+    return vox * (0.5 * plane_passes(start, steps) + 0.25 * hashes + 1.25 * len(segs))
+
+
 def bench_boxes512(F, steps, warmup, kernel_ticks=200):
-    """The 512^3 box scene with the library's default tick (settled segments are
-    skipped): warm-up ticks, then the timed graphs of `steps` ticks with a fused
-    hash every 50 and on the last tick.  The same tick sequence is replayed with
-    sweep counters on to get the algorithmic bytes of the timed region (skipping
-    is deterministic), and a dense world runs the plain tick kernel for the dense
-    roofline."""
+    """The 512^3 box scene with the library's default tick: warm-up ticks, then the
+    timed graphs of `steps` ticks with a fused hash every 50 and on the last tick.
+    The same tick sequence is replayed with sweep counters on (byte kernels that skip
+    settled segments): its hashes must agree.  A dense world runs for the dense
+    figure."""
     n = 512
     with F.World((n, n, n)) as w:
         t0 = time.perf_counter()
@@ -246,8 +268,9 @@ def pmc_traffic(mode, steps, warmup, kernel_sub, last_n):
 
 def bench_pillars2048(F, ticks):
     """The 2048^3 pillar scene: `ticks` plain ticks in one graph with the default
-    (skipping) tick, with the dense single-tick kernel (the HBM roofline figure)
-    and with dense ticks fused in pairs (two ticks per pass over the grid)."""
+    tick (items in which something moves), with the dense single-tick byte kernel (the
+    HBM roofline figure) and with dense ticks in pairs (two ticks per pass over the
+    planes)."""
     n = 2048
     out = {}
     for kind in ("skip", "dense", "fused"):
@@ -262,16 +285,22 @@ def bench_pillars2048(F, ticks):
             w.run(4, 0)
             w.fill_pillars(2)
             w.tick_count = 0
-            if kind == "skip":
-                w.sweep_stats(True)
             w.prepare_run(ticks, 0)
             w.sync()
             t0 = time.perf_counter()
             w.run(ticks, 0)
             wall = time.perf_counter() - t0
             kern_ms = w.last_run_ms_per_tick()
-            st = w.sweep_stats(False) if kind == "skip" else None
             h = w.hash()
+            st = None
+            if kind == "skip":  # again on the byte kernels, with counters
+                w.fill_pillars(2)
+                w.tick_count = 0
+                w.sweep_stats(True)
+                w.run(ticks, 0)
+                st = w.sweep_stats(False)
+                if w.hash() != h:
+                    raise SystemExit("pillars2048: counter replay diverged from the timed run")
             log(f"[bench] pillars2048 {kind}: {ticks} ticks in {wall * 1e3:.1f} ms ({kern_ms:.3f} ms/tick)")
             out[kind] = dict(wall=wall, kern_ms=kern_ms, hash=int(h), swept=st["swept"] if st else None,
                              seg=w.segment)
@@ -659,7 +688,8 @@ def main():
     # the counter runs are child processes started before this one touches the GPU
     traffic = traffic2048 = None
     if args.only in (None, "boxes512") and not args.no_traffic:
-        traffic = pmc_traffic("boxes512-window", args.steps, args.warmup, ("tick_kernel<",), args.steps)
+        traffic = pmc_traffic("boxes512-window", args.steps, args.warmup, ("plane_pair_kernel<", "plane_tick_kernel<", "plane_pack_even_kernel<"),
+                              plane_passes(args.warmup, args.steps))
         if args.only is None:
             traffic2048 = pmc_traffic("dense2048-window", DENSE2048_WINDOW, 0, DENSE2048_KERNELS, DENSE2048_WINDOW)
 
@@ -701,32 +731,35 @@ def main():
     r = bench_boxes512(F, args.steps, args.warmup)
     vox = r["vox"]
     value = vox * args.steps / r["wall"] / 1e9
-    # the timed region: algorithmic bytes actually moved (2 per swept voxel-update,
-    # 1 per voxel only read on hash ticks) over its device time (HIP events)
-    alg_bytes = 2 * r["swept"] + r["read_only"]
+    # the timed region: the bytes its passes move over its device time (HIP events)
+    alg_bytes = plane_bytes(vox, args.warmup, args.steps)
     ach = alg_bytes / (r["dev_ms"] * 1e-3 * args.steps)
     frac = ach / HBM_PEAK
-    ach_d, frac_d = roofline(vox, r["kern_ms"])
-    sched = {1: "auto", 2: "listed", 3: "waves"}.get(r["mode"], str(r["mode"]))
+    ach_d = PAIR_BYTES_PER_UPDATE * vox / (r["kern_ms"] * 1e-3)
+    frac_d = ach_d / HBM_PEAK
     alg_per_tick = alg_bytes / args.steps
     roof = {"bound": "hbm", "achieved": round(ach / 1e9, 1), "peak": HBM_PEAK / 1e9, "unit": "GB/s",
             "frac": round(frac, 4), "traffic": None,
-            "kernel": f"tick_kernel<{r['seg']},*,skip> ({sched} schedule), every tick of the timed region",
+            "kernel": "plane_pair_kernel, plane_tick_kernel: every tick of the timed region",
             "ms_per_tick_device": round(r["dev_ms"], 5), "alg_bytes_per_tick": int(alg_per_tick),
             "swept_fraction": round(r["swept"] / (vox * args.steps), 4), "skip_violations": r["violations"],
-            "note": "the 128 MiB grid (updated in place) fits the 256 MB Infinity Cache: cache-assisted; "
-                    "hbm2048 is the HBM-bound figure"}
+            "swept_note": "of the byte kernels' replay",
+            "note": "the planes (2 x 32 MiB) fit the 256 MB Infinity Cache, and a pair of ticks is bound by its "
+                    "instructions; hbm2048 is the HBM-bound figure"}
     if traffic is not None:
         if "error" in traffic:
             roof["traffic_error"] = traffic["error"]
         else:
+            per_tick = plane_passes(args.warmup, args.steps) / args.steps
+            for k in ("bytes", "read", "written"):
+                traffic[k] *= per_tick
             roof["traffic"] = round(traffic["bytes"])
             roof["traffic_detail"] = {
                 "source": "rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE of this window (--only boxes512-window, "
-                          "same --steps/--warmup), mean over its timed tick dispatches, scaled by a 1 GiB copy",
+                          "same --steps/--warmup), its timed tick dispatches, per tick, scaled by a 1 GiB copy",
                 "read": round(traffic["read"]), "written": round(traffic["written"]),
                 "vs_algorithmic": round(traffic["bytes"] / alg_per_tick, 3), "scale": traffic["scale"]}
-    roof["dense"] = {"kernel": f"tick_kernel<{r['seg']},false> (every voxel, no skipping)",
+    roof["dense"] = {"kernel": "plane_pair_kernel (every voxel, 0.25 bytes per voxel-update)",
                      "kernel_ms": round(r["kern_ms"], 5), "achieved": round(ach_d / 1e9, 1), "frac": round(frac_d, 4)}
     out = {
         "metric": METRIC,
@@ -799,12 +832,12 @@ def main():
             "dense_kernel_ms": round(pd["kern_ms"], 4), "dense_achieved_GBps": round(ach2 / 1e9, 1),
             "dense_hbm_frac": round(frac2, 4), "dense_frac_of_copy": round(ach2 / 1e9 / c["GBps"], 4),
             "dense_frac_of_streaming_copy": round(ach2 / 1e9 / c["streaming"]["GBps"], 4),
-            "fused_pairs": {"kernel": "tick2c_kernel<16> (two dense ticks per pass in 16-byte x-chunks of 1 KiB, "
-                                             "first tick's rows in LDS)",
+            "fused_pairs": {"kernel": "plane_pair_kernel (two dense ticks per pass over the bit planes)",
                             "gvox_per_s": round(p["vox"] * p["ticks"] / p["fused"]["wall"] / 1e9, 2),
                             "ms_per_tick": round(p["fused"]["kern_ms"], 4),
-                            "achieved_GBps": round(p["vox"] * 2 / (2 * p["fused"]["kern_ms"] * 1e-3) / 1e9, 1),
-                            "note": "achieved counts the 2 bytes per voxel that one pass moves for two ticks"},
+                            "achieved_GBps": round(p["vox"] * PAIR_BYTES_PER_UPDATE /
+                                                   (p["fused"]["kern_ms"] * 1e-3) / 1e9, 1),
+                            "note": "achieved counts the 0.5 bytes per voxel that one pass moves for two ticks"},
             "final_hash": pd["hash"], "segment_bytes": pd["seg"], "dense_kernel": DENSE2048_LABEL,
             "parity": {"tick200_matches_oracle": (pd["hash"] == want200) if want200 is not None else None,
                        "fixture": "tests/golden/pillars2048_frames.json"}}

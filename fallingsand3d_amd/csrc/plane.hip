@@ -13,8 +13,8 @@
 // instructions per 2048 blocks, none of them a load, and a pair of ticks moves
 // about 0.3 bytes per voxel-update.  Dense ticks on an MI355X, us per tick, byte
 // kernels / single plane ticks / plane pairs:
-//   512^3            42 / 12.2 / 9.3      (10.99 and 14.5 T voxel-updates/s)
-//   1000 x 701 x 603 186 (fused pairs 182) / 34 / 22.4
+//   512^3            42 / 11.5 / 8.7      (11.7 and 15.4 T voxel-updates/s)
+//   1000 x 701 x 603 186 (fused pairs 182) / 34 / 23.5
 //   2048^3           3070 (fused pairs 2300) / 770 / 416
 // Single ticks are bound by memory (2048^3: 4.3 GB in 770 us, 5.6 TB/s), pairs by
 // their instructions (1.3 evaluations per row quad and tick with the halo).

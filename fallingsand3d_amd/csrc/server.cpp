@@ -8,8 +8,9 @@
 // arrives while others run joins at the next round boundary and its ticks
 // overlap with theirs on the device.  Rounds are planned on the host ahead of
 // the GPU (tick counts are known), two at a time, with double-buffered tables.
-// A request's final tick hashes its state (fused), and its memory returns to the
-// grid arena once that round has completed.  The HBM budget bounds the device
+// A finished request's state is hashed (plane grids by one launch at the end of the
+// round, byte grids by their last tick), and its memory returns to the grid arena once
+// that round has completed.  The HBM budget bounds the device
 // memory the arena has actually allocated (GridArena, arena.h); a request that
 // does not fit waits at the head of the queue until finished grids come back.
 //

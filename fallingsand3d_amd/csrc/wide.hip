@@ -6,9 +6,10 @@
 // entry padded to whole 4-wave workgroups; an entry that sits the launch out
 // has none) and blk2ent, the entry of every workgroup, expanded on the device
 // from the prefix.  Each workgroup reads its entry with one scalar load and its
-// waves run the ordinary row-quad tick in place.  An entry whose final tick
+// waves run the ordinary row-quad tick in place.  A byte grid whose final tick
 // this is (k + 1 == entry.nt with entry.fin set) hashes its new state; every
-// wave adds its share to hashes[entry.slot] with one atomic.
+// wave adds its share to hashes[entry.slot] with one atomic.  Plane grids are hashed
+// at the end of the round.
 //
 // Used by the serving loop (continuous batching at tick granularity) and as the
 // batch's third mode.  The serving loop keeps its grids as bit planes

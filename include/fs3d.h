@@ -119,9 +119,11 @@ int fs3d_world_get_segment(const fs3d_world *w, int32_t *seg_bytes);
  * same list and packs the listed row quads' active 64-byte sectors into full
  * waves (the block update is paid per active sector, not per row quad with
  * one); WAVES launches one wave per row-quad group that skips on its own (lower
- * per-tick overhead; best for small grids).  AUTO picks SEGS above 2^17 waves
- * of work per tick, else WAVES.  Hash ticks read settled segments in all
- * three.  Worlds of up to 2^27 voxels tick in place with WAVES and LISTED (and
+ * per-tick overhead; best for small grids).  AUTO runs three and more ticks
+ * on two bit planes (rows of 16 cells and more, planes under 4 GiB): every voxel
+ * of grids up to 2^29, above that the 64 x 2 x 16 cell items in which something
+ * moves; other ticks take SEGS above 2^17 waves of work per tick, else WAVES.
+ * Hash ticks read settled segments in all three.  Worlds of up to 2^27 voxels tick in place with WAVES and LISTED (and
  * dense single ticks of rows up to 1024 bytes); the grid stays where
  * fs3d_world_device_ptr last pointed only in that case.
  * Every host-side edit (set_voxel, upload, fills, set_tick, set_segment) keeps
@@ -133,6 +135,8 @@ int fs3d_world_get_skip(const fs3d_world *w, int32_t *mode);
 /* Two-tick fusion of the dense tick (used when skipping is off): a pair of
  * ticks, neither hashed, runs as one pass that keeps the first tick's output in
  * LDS and writes only the second's, so the grid crosses HBM once per two ticks.
+ * Until set_fuse is called and while it is on, runs of three and more dense ticks go
+ * through the bit planes where AUTO's would; off keeps them on bytes, one by one.
  * On by default for grids of more than 2^28 voxels that it supports (smaller
  * grids stay in the last-level cache, where single ticks are faster).  Needs
  * 256 < nx <= 3632 (rows up to 1024 bytes whole in a wave, longer ones in
