@@ -66,6 +66,7 @@ hipError_t copy_to_host(const std::vector<HostSpan> &spans, int dev, hipStream_t
 // piece_blocks(out) workgroups that writes bytes [off, off + out.n).
 hipError_t make_on_host(void *host, size_t n, int dev,
                         const std::function<hipError_t(size_t, const PieceOut &, hipStream_t)> &make);
+
 // Worlds alive: the staging memory kept for the next copy goes with the last one.
 void hostcopy_world(int delta);
 

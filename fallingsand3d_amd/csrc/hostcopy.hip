@@ -15,6 +15,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <thread>
 
@@ -45,12 +46,17 @@ __global__ __launch_bounds__(256) void piece_kernel(const u8 *src, PieceOut o) {
   piece_done(o);
 }
 
+constexpr size_t kFlagBytes = kSlots * kFlagStride * sizeof(u32);
+
 struct Staging {
   int dev = 0;
-  u8 *mem = nullptr;             // the slots, then a flag for each
+  size_t bytes = 0;         // of the slots
+  u8 *mem = nullptr;        // a flag for each slot, then the slots
   u32 *counters = nullptr;  // device memory, one per slot
-  hipStream_t stream = nullptr;  // for work that has no stream of its own
-  u32 *flag(size_t k) const { return reinterpret_cast<u32 *>(mem + kSlots * kSlotBytes) + kFlagStride * k; }
+  bool cleared = false;     // the counters have been set to 0
+  hipStream_t stream = nullptr;  // for work that has no stream of its own, once there was some
+  u32 *flag(size_t k) const { return reinterpret_cast<u32 *>(mem) + kFlagStride * k; }
+  u8 *slots() const { return mem + kFlagBytes; }
 };
 
 void destroy(Staging *g) {
@@ -61,36 +67,36 @@ void destroy(Staging *g) {
   delete g;
 }
 
-Staging *create(int dev) {
+// Slots for a copy of `total` bytes: a small copy's are made in a tenth of a
+// millisecond, all twelve in a fifth.
+Staging *create(int dev, size_t total) {
   Staging *g = new (std::nothrow) Staging();
   if (!g) return nullptr;
   g->dev = dev;
-  hipError_t e = hipHostMalloc((void **)&g->mem, kSlots * (kSlotBytes + kFlagStride * sizeof(u32)), hipHostMallocDefault);
+  g->bytes = std::min(kSlots * kSlotBytes, std::max(total, (size_t)1 << 20));
+  hipError_t e = hipHostMalloc((void **)&g->mem, kFlagBytes + g->bytes, hipHostMallocDefault);
   if (e == hipSuccess) e = hipMalloc((void **)&g->counters, kSlots * sizeof(u32));
-  if (e == hipSuccess) e = hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking);
-  if (e == hipSuccess) e = hipMemsetAsync(g->counters, 0, kSlots * sizeof(u32), g->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(g->stream);
   if (e == hipSuccess) return g;
   (void)hipGetLastError();
   destroy(g);
   return nullptr;
 }
 
-// One idle staging is kept (12 MiB); every copy in flight has its own.
+// One idle staging is kept (12 MiB at most); every copy in flight has its own.
 std::mutex g_mutex;
 Staging *g_idle = nullptr;
 int g_worlds = 0;
 
-Staging *acquire(int dev) {
+Staging *acquire(int dev, size_t total) {
   {
     std::lock_guard<std::mutex> lock(g_mutex);
-    if (g_idle && g_idle->dev == dev) {
+    if (g_idle && g_idle->dev == dev && g_idle->bytes >= std::min(total, kSlots * kSlotBytes)) {
       Staging *g = g_idle;
       g_idle = nullptr;
       return g;
     }
   }
-  return create(dev);
+  return create(dev, total);
 }
 
 void give_back(Staging *g) {
@@ -109,66 +115,78 @@ struct Piece {
 // Launches the kernel for bytes [off, off + out.n) of a span.
 typedef std::function<hipError_t(size_t span, size_t off, const PieceOut &out, hipStream_t)> Issue;
 
-// Piece c goes through slot c % kSlots; the slot's flag becomes c + 1.
+// Piece c goes through slot c % slots; the slot's flag becomes c + 1.  Helpers share the
+// job: a thread that gets to run only after the copy is over finds nothing to claim and
+// touches nothing else, so that nobody has to wait for it.  (Joined, threads that were
+// not scheduled for a while made a copy of 0.3 ms take 4.)
 struct Job {
-  const std::vector<Piece> *pieces;
+  std::vector<Piece> pieces;
   const Staging *g;
-  size_t piece;                           // bytes of a slot in use
+  size_t piece, slots;                    // bytes of a slot, slots in use
   std::atomic<size_t> taken{0};           // pieces claimed
+  std::atomic<size_t> copied{0};          // pieces copied out
+  std::atomic<int> busy{0};               // helpers between a claim and its end
   std::atomic<size_t> done[kSlots] = {};  // of a slot: the last piece copied out of it, plus 1
   std::atomic<bool> stop{false};
 };
 
 bool arrived(const Job *j, size_t c) {
-  return __atomic_load_n(j->g->flag(c % kSlots), __ATOMIC_ACQUIRE) == (u32)c + 1u;
+  return __atomic_load_n(j->g->flag(c % j->slots), __ATOMIC_ACQUIRE) == (u32)c + 1u;
 }
 
 void copy_out(Job *j, size_t c) {
-  const Piece &p = (*j->pieces)[c];
-  std::memcpy(p.host, j->g->mem + (c % kSlots) * j->piece, p.n);
-  j->done[c % kSlots].store(c + 1, std::memory_order_release);
+  const Piece &p = j->pieces[c];
+  std::memcpy(p.host, j->g->slots() + (c % j->slots) * j->piece, p.n);
+  j->done[c % j->slots].store(c + 1, std::memory_order_release);
+  j->copied.fetch_add(1);
 }
 
-void help(Job *j) {
+void help(std::shared_ptr<Job> job) {
+  Job *j = job.get();
   for (;;) {
-    const size_t c = j->taken.fetch_add(1);
-    if (c >= j->pieces->size()) return;
-    while (!arrived(j, c)) {
-      if (j->stop.load()) return;
+    j->busy.fetch_add(1);
+    const size_t c = j->stop.load() ? j->pieces.size() : j->taken.fetch_add(1);
+    bool mine = c < j->pieces.size();
+    while (mine && !arrived(j, c)) {
+      if (j->stop.load()) mine = false;
       std::this_thread::yield();
     }
-    copy_out(j, c);
+    if (mine) copy_out(j, c);
+    j->busy.fetch_sub(1);
+    if (!mine) return;
   }
 }
 
 // Runs the pieces through g; the stream is idle when it returns.
-hipError_t run(Staging *g, const std::vector<Piece> &pieces, size_t piece, size_t total, hipStream_t s,
-               const Issue &issue) {
-  Job j;
-  j.pieces = &pieces;
+hipError_t run(Staging *g, std::vector<Piece> all, size_t piece, size_t total, hipStream_t s, const Issue &issue) {
+  const std::shared_ptr<Job> job = std::make_shared<Job>();
+  Job &j = *job;
+  j.pieces = std::move(all);
+  const std::vector<Piece> &pieces = j.pieces;
   j.g = g;
   j.piece = piece;
+  const size_t slots = j.slots = std::min(kSlots, g->bytes / piece);
   for (size_t k = 0; k < kSlots; k++) *g->flag(k) = 0;
   const size_t n = pieces.size();
-  std::thread helpers[kHelpers];
-  hipError_t e = hipSuccess;
+  hipError_t e = g->cleared ? hipSuccess : launch_fill_u32(g->counters, kSlots, 0, s);
+  g->cleared = g->cleared || e == hipSuccess;
   size_t issued = 0;
   // Launches what follows in free neighbouring slots (once a few are free).
   auto issue_free = [&] {
     while (issued < n && e == hipSuccess) {
       const Piece &p = pieces[issued];
       size_t m = 0, bytes = 0;
-      while (issued + m < n && pieces[issued + m].span == p.span && issued % kSlots + m < kSlots &&
-             (issued + m < kSlots || j.done[issued % kSlots + m].load(std::memory_order_acquire) ==
-                                         issued + m - kSlots + 1)) {
+      while (issued + m < n && pieces[issued + m].span == p.span && issued % slots + m < slots &&
+             (issued + m < slots || j.done[issued % slots + m].load(std::memory_order_acquire) ==
+                                         issued + m - slots + 1)) {
         bytes += pieces[issued + m].n;
         m++;
       }
-      const bool all = issued + m == n || issued % kSlots + m == kSlots || pieces[issued + m].span != p.span;
-      if (m == 0 || (m < kSlots / 4 && !all)) return;
-      const size_t k = issued % kSlots;
+      const bool all = issued + m == n || issued % slots + m == slots || pieces[issued + m].span != p.span;
+      if (m == 0 || (m < slots / 4 && !all)) return;
+      const size_t k = issued % slots;
       e = issue(p.span, p.off,
-                PieceOut{g->mem + k * piece, (u32)bytes, (u32)piece, g->counters + k, g->flag(k), (u32)issued + 1u}, s);
+                PieceOut{g->slots() + k * piece, (u32)bytes, (u32)piece, g->counters + k, g->flag(k), (u32)issued + 1u}, s);
       issued += m;
     }
   };
@@ -176,7 +194,7 @@ hipError_t run(Staging *g, const std::vector<Piece> &pieces, size_t piece, size_
   if (total > kAloneMax)
     for (int i = 0; i < (int)std::min<size_t>(kHelpers, n - 1); i++) {
       try {
-        helpers[i] = std::thread(help, &j);
+        std::thread(help, job).detach();
       } catch (...) {
         break;  // fewer threads do the same work
       }
@@ -203,8 +221,7 @@ hipError_t run(Staging *g, const std::vector<Piece> &pieces, size_t piece, size_
     if (e == hipSuccess && c < n) copy_out(&j, c);
   }
   if (e != hipSuccess) j.stop.store(true);
-  for (std::thread &t : helpers)
-    if (t.joinable()) t.join();
+  while (e == hipSuccess ? j.copied.load() < n : j.busy.load() != 0) std::this_thread::yield();
   const hipError_t last = hipStreamSynchronize(s);  // no slot is in use any more
   return e != hipSuccess ? e : last;
 }
@@ -238,7 +255,7 @@ hipError_t copy_to_host(const std::vector<HostSpan> &spans, int dev, hipStream_t
     total += h.n;
     staged = staged && pageable(h.host) && (uintptr_t)h.dev % 16 == 0;
   }
-  Staging *g = staged && total >= kDirectMax ? acquire(dev) : nullptr;
+  Staging *g = staged && total >= kDirectMax ? acquire(dev, total) : nullptr;
   if (!g) {
     for (const HostSpan &h : spans)
       if (const hipError_t e = hipMemcpyAsync(h.host, h.dev, h.n, hipMemcpyDeviceToHost, s)) return e;
@@ -253,6 +270,7 @@ hipError_t copy_to_host(const std::vector<HostSpan> &spans, int dev, hipStream_t
       return hipGetLastError();
     });
   } catch (...) {
+    e = hipErrorOutOfMemory;
   }
   give_back(g);
   return e;
@@ -260,7 +278,7 @@ hipError_t copy_to_host(const std::vector<HostSpan> &spans, int dev, hipStream_t
 
 hipError_t make_on_host(void *host, size_t n, int dev,
                         const std::function<hipError_t(size_t, const PieceOut &, hipStream_t)> &make) {
-  Staging *g = acquire(dev);
+  Staging *g = acquire(dev, n);
   if (!g) return hipErrorOutOfMemory;
   hipError_t e = hipErrorOutOfMemory;
   try {
@@ -268,10 +286,13 @@ hipError_t make_on_host(void *host, size_t n, int dev,
     if (!pageable(host)) between.resize(n);
     std::vector<Piece> pieces;
     split(&pieces, between.empty() ? host : between.data(), n, 0, piece_of(n));
-    e = run(g, pieces, piece_of(n), n, g->stream,
-            [&](size_t, size_t off, const PieceOut &out, hipStream_t st) { return make(off, out, st); });
+    e = g->stream ? hipSuccess : hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking);
+    if (e == hipSuccess)
+      e = run(g, pieces, piece_of(n), n, g->stream,
+              [&](size_t, size_t off, const PieceOut &out, hipStream_t st) { return make(off, out, st); });
     if (e == hipSuccess && !between.empty()) e = hipMemcpy(host, between.data(), n, hipMemcpyDefault);
   } catch (...) {
+    e = hipErrorOutOfMemory;
   }
   give_back(g);
   return e;
