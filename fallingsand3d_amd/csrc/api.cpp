@@ -280,7 +280,7 @@ bool plane_path(const fs3d_world *w, int nticks) {
   if (w->skip != FS3D_SKIP_OFF && w->skip != FS3D_SKIP_AUTO) return false;
   if (!w->skip && w->fuse_set && !w->fuse) return false;
   if (w->nx < 16 || plane_words(shape_of(w)) > kMaxPlaneWords) return false;
-  return w->planes_valid || nticks >= kPlaneMinTicks;
+  return w->plane.valid || nticks >= kPlaneMinTicks;
 }
 
 // Plane buffers (and the item lists) on first use; false (and the byte kernels from
@@ -298,7 +298,7 @@ bool ensure_planes(fs3d_world *w) {
   }
   if (created || w->planes_tiled != ps.tiled) {
     w->planes_tiled = ps.tiled;
-    w->planes_valid = false;
+    w->plane.valid = false;
     for (int i = 0; i < 2 && e == hipSuccess; i++) e = launch_plane_pad(ps, w->planes[i], w->stream);
   }
   if (item_ticks(w) && !w->d_items && e == hipSuccess) {
@@ -327,74 +327,91 @@ bool ensure_planes(fs3d_world *w) {
   drop(w->d_since);
   drop(w->d_nitems);
   drop(w->d_items);
-  w->planes_valid = false;
+  w->plane.valid = false;
   w->planes_off = true;
   return false;
 }
 
-// Enqueues nticks ticks of the planes (packing them first when they are not the
-// current state) and the unpacking into buf[cur].  *pfinal: the index of the plane
-// buffer holding the result, + 2 * that of the last pass's change flags.
-int enqueue_planes(fs3d_world *w, int nticks, int hash_every, const u64 *tick_dev, int *pfinal, bool launch = true) {
-  const PlaneShape ps = shape_of(w);
-  const bool items = item_ticks(w);
-  int src = w->planes_valid ? w->pcur : 0, f = w->fcur;
-  // an even first tick is done while packing
-  const bool packs = !w->planes_valid, ticks_too = packs && !(w->tick & 1u);
-  int first = ticks_too ? kAfterPackTick : packs || !w->pflags_valid ? kAfterPack : kNotFirst;
-  if (launch && packs) {
+// The launches of a run on the planes (plane_sched.h); t + k is a pass's tick.
+struct PlaneLaunch {
+  fs3d_world *w;
+  PlaneShape ps;
+  const u64 *tick_dev;
+
+  PlaneHash hash_to(int i) const { return PlaneHash{w->buf[w->cur], w->d_reserved, w->d_parts, w->d_small + i}; }
+  int finalize(int i) const {
+    if (!plane_hash_direct(ps)) FS3D_HIP(launch_hash_finalize(w->d_parts, w->d_small + i, w->stream));
+    return FS3D_OK;
+  }
+  int packed(bool items) const {
     FS3D_HIP(launch_fill_u32(w->d_reserved, 1, 0, w->stream));
-    if (ticks_too)
-      FS3D_HIP(launch_plane_pack_even(ps, w->buf[w->cur], w->planes[src], w->d_reserved, w->tick, tick_dev, 0,
-                                      items ? w->pflags[f] : nullptr, w->planes[src ^ 1], w->stream));
-    else
-      FS3D_HIP(launch_plane_pack(ps, w->buf[w->cur], w->planes[src], w->d_reserved, w->stream));
+    if (items) FS3D_HIP(launch_fill_u32(w->d_nitems, 2, 0, w->stream));
+    return FS3D_OK;
   }
-  if (launch && items && first == kAfterPack)
+  int pack(int src) const {
+    FS3D_HIP(launch_plane_pack(ps, w->buf[w->cur], w->planes[src], w->d_reserved, w->stream));
+    return FS3D_OK;
+  }
+  int pack_tick(int src, int f) const {
+    FS3D_HIP(launch_plane_pack_even(ps, w->buf[w->cur], w->planes[src], w->d_reserved, w->tick, tick_dev, 0,
+                                    f < 0 ? nullptr : w->pflags[f], w->planes[src ^ 1], w->stream));
+    return FS3D_OK;
+  }
+  int all_flags(int f) const {
     FS3D_HIP(launch_fill_u64(w->pflags[f], plane_cells(ps).flag_words, ~0ull, w->stream));
-  auto hashed_after = [&](int k) { return hash_every > 0 && (k + 1) % hash_every == 0; };
-  const bool direct = plane_hash_direct(ps);
-  if (launch && direct && hash_every > 0 && nticks >= hash_every)
-    FS3D_HIP(launch_fill_u64(w->d_small + 1, (size_t)(nticks / hash_every), 0, w->stream));
-  PlaneHash hash{w->buf[w->cur], w->d_reserved, w->d_parts, nullptr};  // out: due for planes[src]
-  if (ticks_too && hashed_after(0)) hash.out = w->d_small + 1;
-  for (int k = ticks_too ? 1 : 0; k < nticks;) {
-    const u64 t = w->tick + (u64)k;
-    const bool pair = (t & 1u) && k + 1 < nticks && !hashed_after(k);
-    if (launch) {
-      // a single tick hashes the state that it reads
-      const bool with = hash.out && !items && !pair;
-      if (hash.out && !with) FS3D_HIP(launch_plane_hash(ps, w->planes[src], hash, w->stream));
-      if (items)
-        FS3D_HIP(launch_plane_list(ps, w->planes[src], w->planes[src ^ 1], t, tick_dev, (u32)k, pair, first,
-                                   w->pflags[f], w->pflags[f ^ 1], w->d_since, w->d_items, w->d_nitems + f,
-                                   w->d_nitems + (f ^ 1), w->item_waves, w->stream));
-      else if (pair)
-        FS3D_HIP(launch_plane_pair(ps, w->planes[src], w->planes[src ^ 1], t, tick_dev, (u32)k, w->stream));
-      else
-        FS3D_HIP(launch_plane_tick(ps, w->planes[src], w->planes[src ^ 1], t, tick_dev, (u32)k,
-                                   with ? &hash : nullptr, w->stream));
-      if (hash.out && !direct) FS3D_HIP(launch_hash_finalize(w->d_parts, hash.out, w->stream));
-    }
-    src ^= 1;
-    f ^= 1;
-    first = kNotFirst;
-    k += pair ? 2 : 1;
-    hash.out = hashed_after(k - 1) ? w->d_small + k / hash_every : nullptr;
+    return FS3D_OK;
   }
-  if (launch && hash.out) {
-    FS3D_HIP(launch_plane_hash(ps, w->planes[src], hash, w->stream));
-    if (!direct) FS3D_HIP(launch_hash_finalize(w->d_parts, hash.out, w->stream));
+  int zero_hashes(int n) const {
+    if (plane_hash_direct(ps)) FS3D_HIP(launch_fill_u64(w->d_small + 1, (size_t)n, 0, w->stream));
+    return FS3D_OK;
   }
-  if (launch) {
-    if (items)
+  int hash(int src, int i) const {
+    FS3D_HIP(launch_plane_hash(ps, w->planes[src], hash_to(i), w->stream));
+    return finalize(i);
+  }
+  int pass(const PlanePass &p) const {
+    const u64 t = w->tick + (u64)p.k;
+    const PlaneHash h = hash_to(p.hash);
+    if (p.pair)
+      FS3D_HIP(launch_plane_pair(ps, w->planes[p.src], w->planes[p.src ^ 1], t, tick_dev, (u32)p.k, w->stream));
+    else
+      FS3D_HIP(launch_plane_tick(ps, w->planes[p.src], w->planes[p.src ^ 1], t, tick_dev, (u32)p.k,
+                                 p.hash ? &h : nullptr, w->stream));
+    return p.hash ? finalize(p.hash) : FS3D_OK;
+  }
+  int item_pass(const PlanePass &p) const {
+    FS3D_HIP(launch_plane_list(ps, w->planes[p.src], w->planes[p.src ^ 1], w->tick + (u64)p.k, tick_dev, (u32)p.k,
+                               p.pair, p.first, w->pflags[p.flags], w->pflags[p.flags ^ 1], w->d_since, w->d_items,
+                               w->d_nitems + p.flags, w->d_nitems + (p.flags ^ 1), w->item_waves, w->stream));
+    return FS3D_OK;
+  }
+  int unpack(int src, int f) const {
+    if (f >= 0)
       FS3D_HIP(launch_plane_unpack_cells(ps, w->planes[src], w->buf[w->cur], w->pflags[f], w->d_since, w->d_reserved,
                                          w->occ_track ? w->d_dirty : nullptr, w->stream));
     else
       FS3D_HIP(launch_plane_unpack(ps, w->planes[src], w->buf[w->cur], w->d_reserved, w->stream));
+    return FS3D_OK;
   }
-  if (pfinal) *pfinal = src | f << 1;
-  return FS3D_OK;
+};
+
+// The same without launches: only the state after the run.
+struct NoLaunch {
+  int packed(bool) const { return FS3D_OK; }
+  int pack(int) const { return FS3D_OK; }
+  int pack_tick(int, int) const { return FS3D_OK; }
+  int all_flags(int) const { return FS3D_OK; }
+  int zero_hashes(int) const { return FS3D_OK; }
+  int hash(int, int) const { return FS3D_OK; }
+  int pass(const PlanePass &) const { return FS3D_OK; }
+  int item_pass(const PlanePass &) const { return FS3D_OK; }
+  int unpack(int, int) const { return FS3D_OK; }
+};
+
+// Enqueues nticks ticks of the planes (packing them first when they are not the
+// current state) and the unpacking into buf[cur].  *st becomes the state after them.
+int enqueue_planes(fs3d_world *w, int nticks, int hash_every, const u64 *tick_dev, PlaneState *st) {
+  return plane_passes(st, item_ticks(w), w->tick, nticks, hash_every, PlaneLaunch{w, shape_of(w), tick_dev});
 }
 
 // Which path the next nticks ticks take: decided once per call, with what that
@@ -406,29 +423,40 @@ int choose_path(fs3d_world *w, int nticks, bool *planes) {
   return FS3D_OK;
 }
 
-// The world's bookkeeping after nticks ticks on either path.
-void ticked(fs3d_world *w, int nticks, bool planes, int fin) {
-  if (planes) {
-    w->pcur = fin & 1;
-    w->fcur = fin >> 1;
-    w->planes_valid = true;
-    w->pflags_valid = item_ticks(w);
-    w->masks_stale = true;
-    // the items' unpacking has marked the bricks it wrote
-    w->occ_valid = w->occ_valid && w->pflags_valid && w->occ_track;
-  } else {
-    w->cur = fin;
-    if (nticks > 0) w->planes_valid = false;
-    note_ticks(w);
-  }
+// The world's bookkeeping after nticks ticks on the planes, or on bytes, which leave
+// their state in buf[fin].
+void ticked_planes(fs3d_world *w, int nticks) {
+  w->masks_stale = true;
+  // the items' unpacking has marked the bricks it wrote
+  w->occ_valid = w->occ_valid && w->plane.flags_valid && w->occ_track;
   w->tick += (u64)nticks;
+}
+void ticked_bytes(fs3d_world *w, int nticks, int fin) {
+  w->cur = fin;
+  if (nticks > 0) w->plane.valid = false;
+  note_ticks(w);
+  w->tick += (u64)nticks;
+}
+
+// Enqueues nticks ticks on the path chosen and does the bookkeeping.
+int enqueue_ticks(fs3d_world *w, int nticks, int hash_every, const u64 *tick_dev, int *final, bool launch = true);
+int run_ticks(fs3d_world *w, int nticks, int hash_every, bool planes) {
+  if (planes) {
+    if (int rc = enqueue_planes(w, nticks, hash_every, nullptr, &w->plane)) return rc;
+    ticked_planes(w, nticks);
+  } else {
+    int fin = w->cur;
+    if (int rc = enqueue_ticks(w, nticks, hash_every, nullptr, &fin)) return rc;
+    ticked_bytes(w, nticks, fin);
+  }
+  return FS3D_OK;
 }
 
 // Enqueues nticks ticks starting from buffer w->cur; *final receives the index of
 // the buffer holding the result (a fused pair of dense ticks moves the state to
 // the other buffer once, a single tick from one buffer into the other once, a
 // tick in place not at all).  With launch = false it only computes *final.
-int enqueue_ticks(fs3d_world *w, int nticks, int hash_every, const u64 *tick_dev, int *final, bool launch = true) {
+int enqueue_ticks(fs3d_world *w, int nticks, int hash_every, const u64 *tick_dev, int *final, bool launch) {
   const u64 *rule = device_rule_table(w->dev);
   u64 *const *masks = w->skip ? w->d_masks : nullptr;
   const int sched = w->skip ? skip_schedule(w) : FS3D_SKIP_OFF;
@@ -491,14 +519,15 @@ namespace {
 int world_graph(fs3d_world *w, int nticks, int hash_every, bool planes, hipGraphExec_t *out) {
   // a plane graph pairs its ticks by the start tick's parity
   const int state = !planes ? w->cur
-                            : 64 | w->cur | (w->planes_valid ? 8 | w->pcur << 1 : 0) | (int)(w->tick & 1u) << 2 |
-                                  (item_ticks(w) ? w->fcur << 4 | (w->pflags_valid ? 32 : 0) : 0);
+                            : 64 | w->cur | (w->plane.valid ? 8 | w->plane.cur << 1 : 0) | (int)(w->tick & 1u) << 2 |
+                                  (item_ticks(w) ? w->plane.flags << 4 | (w->plane.flags_valid ? 32 : 0) : 0);
   const auto key = std::make_tuple(nticks, hash_every, state);
   auto it = w->graphs.find(key);
   if (it == w->graphs.end()) {
     hipGraph_t graph = nullptr;
+    PlaneState after = w->plane;
     FS3D_HIP(hipStreamBeginCapture(w->stream, hipStreamCaptureModeThreadLocal));
-    int rc = planes ? enqueue_planes(w, nticks, hash_every, w->d_small, nullptr)
+    int rc = planes ? enqueue_planes(w, nticks, hash_every, w->d_small, &after)
                     : enqueue_ticks(w, nticks, hash_every, w->d_small, nullptr);
     hipError_t e = hipStreamEndCapture(w->stream, &graph);
     if (rc) {
@@ -654,13 +683,13 @@ int fs3d_world_set_voxel(fs3d_world *w, int32_t x, int32_t y, int32_t z, uint8_t
   if (seg > 0) e.bits |= 1ull << (seg - 1);
   if (seg + 1 < lr) e.bits |= 1ull << (seg + 1);
   e.edge_off = w->mask_words;
-  if (w->planes_valid) {
+  if (w->plane.valid) {
     const PlaneShape ps = plane_shape(w->nx, w->ny, w->nz, w->planes_tiled);
-    e.planes = static_cast<u32 *>(w->planes[w->pcur]);
+    e.planes = static_cast<u32 *>(w->planes[w->plane.cur]);
     e.reserved = w->d_reserved;
     e.word = plane_word(ps, x, y, z);
     e.x = x;
-    if (w->pflags_valid) e.flags = w->pflags[w->fcur] + plane_cell_flags(ps, y, z, &e.nflags, &e.flag_stride);
+    if (w->plane.flags_valid) e.flags = w->pflags[w->plane.flags] + plane_cell_flags(ps, y, z, &e.nflags, &e.flag_stride);
   }
   w->occ_valid = false;
   FS3D_HIP(launch_set_cell(e, next_note(w), w->stream));
@@ -685,7 +714,7 @@ int fs3d_world_upload(fs3d_world *w, const uint8_t *host, size_t nbytes) {
   if (int rc = check_world(w)) return rc;
   if (!host || nbytes != w->n) return set_error(FS3D_ERR_INVALID, "upload needs %zu bytes (got %zu)", w->n, nbytes);
   FS3D_HIP(hipSetDevice(w->dev));
-  w->planes_valid = false;
+  w->plane.valid = false;
   FS3D_HIP(hipMemcpyAsync(w->buf[w->cur], host, w->n, hipMemcpyHostToDevice, w->stream));
   if (int rc = mark_all(w)) return rc;
   FS3D_HIP(hipStreamSynchronize(w->stream));
@@ -817,10 +846,7 @@ int fs3d_world_step(fs3d_world *w, int32_t nticks) {
   FS3D_HIP(hipSetDevice(w->dev));
   bool planes = false;
   if (int rc = choose_path(w, nticks, &planes)) return rc;
-  int fin = w->cur;
-  if (int rc = planes ? enqueue_planes(w, nticks, 0, nullptr, &fin) : enqueue_ticks(w, nticks, 0, nullptr, &fin))
-    return rc;
-  ticked(w, nticks, planes, fin);
+  if (int rc = run_ticks(w, nticks, 0, planes)) return rc;
   return clear_error();
 }
 
@@ -830,17 +856,15 @@ int fs3d_world_tick(fs3d_world *w, uint64_t *hash) {
   FS3D_HIP(hipSetDevice(w->dev));
   bool planes = false;
   if (int rc = choose_path(w, 1, &planes)) return rc;
-  int fin = w->cur;
   if (w->n <= kHashPostMax && !w->d_stats) {
-    if (int rc = planes ? enqueue_planes(w, 1, 0, nullptr, &fin) : enqueue_ticks(w, 1, 0, nullptr, &fin)) return rc;
-    FS3D_HIP(launch_hash_post(w->buf[planes ? w->cur : fin], w->n, w->d_parts, next_note(w), w->stream));
+    if (int rc = run_ticks(w, 1, 0, planes)) return rc;
+    FS3D_HIP(launch_hash_post(w->buf[w->cur], w->n, w->d_parts, next_note(w), w->stream));
   } else {
-    if (int rc = planes ? enqueue_planes(w, 1, 1, nullptr, &fin) : enqueue_ticks(w, 1, 1, nullptr, &fin)) return rc;
+    if (int rc = run_ticks(w, 1, 1, planes)) return rc;
     FS3D_HIP(launch_post(w->d_small + 1, next_note(w), w->stream));
   }
   u64 got = 0;
   if (int rc = read_note(w, &got)) return rc;
-  ticked(w, 1, planes, fin);
   *hash = got;
   return clear_error();
 }
@@ -899,11 +923,14 @@ int fs3d_world_run(fs3d_world *w, int32_t nticks, int32_t hash_every, uint64_t *
   FS3D_HIP(hipEventElapsedTime(&ms, w->ev0, w->ev1));
   w->last_run_ms = (double)ms / nticks;
   for (int i = 0; i < nh; i++) hashes[i] = w->h_pinned[i];
-  int fin = w->cur;
-  if (int rc = planes ? enqueue_planes(w, nticks, hash_every, nullptr, &fin, false)
-                      : enqueue_ticks(w, nticks, hash_every, nullptr, &fin, false))
-    return rc;
-  ticked(w, nticks, planes, fin);
+  if (planes) {
+    (void)plane_passes(&w->plane, item_ticks(w), w->tick, nticks, hash_every, NoLaunch());
+    ticked_planes(w, nticks);
+  } else {
+    int fin = w->cur;
+    if (int rc = enqueue_ticks(w, nticks, hash_every, nullptr, &fin, false)) return rc;
+    ticked_bytes(w, nticks, fin);
+  }
   return clear_error();
 }
 
@@ -975,7 +1002,7 @@ int fs3d_world_load(fs3d_world *w, const char *path) {
     return set_error(FS3D_ERR_INVALID, "%s holds a %dx%dx%d world, this one is %dx%dx%d", path, dims[0], dims[1],
                      dims[2], w->nx, w->ny, w->nz);
   FS3D_HIP(hipSetDevice(w->dev));
-  w->planes_valid = false;
+  w->plane.valid = false;
   // The payload goes to the idle buffer and becomes the world's state only once
   // its hash matches the stored one; on any failure the grid and tick stay as
   // they were.  Skipped segments rely on the destination buffer holding their
@@ -1007,7 +1034,7 @@ int fs3d_world_load(fs3d_world *w, const char *path) {
 int fs3d_world_fill_rain(fs3d_world *w, uint64_t seed, uint64_t thr) {
   if (int rc = check_world(w)) return rc;
   FS3D_HIP(hipSetDevice(w->dev));
-  w->planes_valid = false;
+  w->plane.valid = false;
   FS3D_HIP(launch_fill_rain(w->buf[w->cur], w->nx, w->ny, w->nz, seed, thr, w->stream));
   if (int rc = mark_all(w)) return rc;
   FS3D_HIP(hipStreamSynchronize(w->stream));
@@ -1018,7 +1045,7 @@ int fs3d_world_fill_boxes(fs3d_world *w, uint64_t seed, const fs3d_box_params *p
   if (int rc = check_world(w)) return rc;
   if (!p) return set_error(FS3D_ERR_INVALID, "params is NULL");
   FS3D_HIP(hipSetDevice(w->dev));
-  w->planes_valid = false;
+  w->plane.valid = false;
   u8 *host = nullptr;
   FS3D_HIP(hipHostMalloc(&host, w->n, hipHostMallocDefault));
   const long long nb = paint_boxes(host, w->nx, w->ny, w->nz, seed, *p);
@@ -1044,7 +1071,7 @@ int fs3d_world_fill_pillars(fs3d_world *w, uint64_t seed, const fs3d_pillar_para
   if (pillar_list(w->nx, w->ny, w->nz, seed, *p, pool, &pillars) != 0)
     return set_error(FS3D_ERR_INVALID, "pillar parameters do not fit the grid");
   FS3D_HIP(hipSetDevice(w->dev));
-  w->planes_valid = false;
+  w->plane.valid = false;
   u8 *g = w->buf[w->cur];
   const size_t layer = (size_t)w->nx * w->ny;
   if (int rc = mark_all(w)) return rc;

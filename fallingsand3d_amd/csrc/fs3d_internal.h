@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "../../include/fs3d.h"
+#include "plane_sched.h"
 
 namespace fs3d {
 
@@ -232,20 +233,18 @@ struct fs3d_world {
   fs3d::u32 *d_ctl = nullptr;         // list counts, one per tick mod 3
   fs3d::u32 list_waves = 0;           // persistent waves of the listed tick
   fs3d::u32 pack_waves = 0;           // persistent waves of the packed tick
-  // the grid as bit planes (two buffers, allocated on first use): planes[pcur]
-  // holds the current state while planes_valid; buf[cur] always does between calls
+  // the grid as bit planes (two buffers, allocated on first use): planes[plane.cur]
+  // holds the current state while plane.valid; buf[cur] always does between calls
   void *planes[2] = {nullptr, nullptr};
-  int pcur = 0;
-  bool planes_valid = false, planes_off = false;
+  fs3d::PlaneState plane;
+  bool planes_off = false;
   bool planes_tiled = false;  // the buffers' layout (its rows around the grid are zero)
   fs3d::u32 *d_reserved = nullptr;  // a byte >= 4 has been packed or set
-  // ticks of the active items only: change flags of the last pass (pflags[fcur],
-  // exact or too many while pflags_valid), items changed since the bytes were
-  // written, work list and its count
+  // ticks of the active items only: change flags of the last pass
+  // (pflags[plane.flags]), items changed since the bytes were written, work list and
+  // its counters
   fs3d::u64 *pflags[2] = {nullptr, nullptr}, *d_since = nullptr;
   fs3d::u32 *d_items = nullptr, *d_nitems = nullptr;
-  int fcur = 0;
-  bool pflags_valid = false;
   fs3d::u32 item_waves = 0;
   bool masks_stale = false;         // plane ticks have run since the change masks were last exact
   bool fuse_set = false;            // set_fuse has been called

@@ -90,7 +90,6 @@ int plane_list_blocks_per_cu();
 // this one's; since: items changed since the bytes were written; first: kAfterPack
 // for the first pass after packing (every flag set), kAfterPackTick for the first one
 // after launch_plane_pack_even.  *count is 0 before; the pass clears *next_count.
-enum { kNotFirst = 0, kAfterPack, kAfterPackTick };
 hipError_t launch_plane_list(const PlaneShape &ps, const void *src, void *dst, u64 t, const u64 *tick_dev, u32 k_off,
                              bool pair, int first, const u64 *flags_in, u64 *flags_out, u64 *since, u32 *list,
                              u32 *count, u32 *next_count, u32 nwaves, hipStream_t s);

@@ -1,0 +1,85 @@
+// The passes that a run of ticks takes on a world's bit planes, and what holds about
+// the planes between calls.  Host code without device calls: the launches are the
+// caller's (Ops), so that the bookkeeping can be checked without a device.
+#pragma once
+
+#include <cstdint>
+
+namespace fs3d {
+
+// What the first pass over the active items must know: nothing, that the grid has just
+// been packed (every flag is set), or packed and ticked once (plane.h).
+enum { kNotFirst = 0, kAfterPack, kAfterPackTick };
+
+// A world's planes between calls.
+struct PlaneState {
+  bool valid = false;        // planes[cur] holds the current state
+  int cur = 0;
+  int flags = 0;             // flag buffer and list counter of the next pass over the items
+  bool flags_valid = false;  // the flag buffer describes the last pass (exactly, or too many)
+};
+
+// A pass: one tick, or the ticks t (odd) and t + 1.
+struct PlanePass {
+  int k;       // ticks of the run before it
+  bool pair;
+  int src;     // reads planes[src], writes planes[src ^ 1]
+  int flags;   // items: reads flags[flags], writes flags[flags ^ 1], appends to counter[flags]
+               // and clears counter[flags ^ 1]
+  int first;   // items: kNotFirst, ...
+  int hash;    // everything: the hash (1, 2, ...) of planes[src] taken in the same launch, or 0
+};
+
+// nticks ticks from tick t0 with a hash every hash_every (0: none); items: passes over
+// the active items only.  *st becomes the state after them.  Ops, each returning 0 or
+// an error:
+//   packed(items)            the grid is about to be packed; items: clears both counters
+//   pack(src)                bytes to planes[src]
+//   pack_tick(src, flags)    the same and tick t0 (even); flags: -1 or the flag buffer to write
+//   all_flags(flags)         every flag set
+//   zero_hashes(n)
+//   hash(src, i)             hash i of planes[src]
+//   pass(p), item_pass(p)
+//   unpack(src, flags)       planes[src] to bytes; flags: -1 or the last pass's flag buffer
+template <class Ops>
+int plane_passes(PlaneState *st, bool items, uint64_t t0, int nticks, int hash_every, Ops &&ops) {
+  int src = st->valid ? st->cur : 0, f = st->flags;
+  // an even first tick is done while packing
+  const bool packs = !st->valid, ticks_too = packs && !(t0 & 1u);
+  st->valid = false;  // should a launch fail, the bytes are the state
+  int first = ticks_too ? kAfterPackTick : packs || !st->flags_valid ? kAfterPack : kNotFirst;
+  if (packs) {
+    if (int rc = ops.packed(items)) return rc;
+    if (int rc = ticks_too ? ops.pack_tick(src, items ? f : -1) : ops.pack(src)) return rc;
+  }
+  if (items && first == kAfterPack)
+    if (int rc = ops.all_flags(f)) return rc;
+  auto hashed_after = [&](int k) { return hash_every > 0 && (k + 1) % hash_every == 0; };
+  if (hash_every > 0 && nticks >= hash_every)
+    if (int rc = ops.zero_hashes(nticks / hash_every)) return rc;
+  int due = ticks_too && hashed_after(0) ? 1 : 0;  // the hash that planes[src] has yet to give
+  for (int k = ticks_too ? 1 : 0; k < nticks;) {
+    const bool pair = ((t0 + (uint64_t)k) & 1u) && k + 1 < nticks && !hashed_after(k);
+    // a single tick hashes the state that it reads
+    const bool with = due && !items && !pair;
+    if (due && !with)
+      if (int rc = ops.hash(src, due)) return rc;
+    const PlanePass p{k, pair, src, f, first, with ? due : 0};
+    if (int rc = items ? ops.item_pass(p) : ops.pass(p)) return rc;
+    src ^= 1;
+    if (items) f ^= 1;  // (a pass over everything clears no counter)
+    first = kNotFirst;
+    k += pair ? 2 : 1;
+    due = hashed_after(k - 1) ? k / hash_every : 0;
+  }
+  if (due)
+    if (int rc = ops.hash(src, due)) return rc;
+  if (int rc = ops.unpack(src, items ? f : -1)) return rc;
+  st->cur = src;
+  st->valid = true;
+  st->flags = f;
+  st->flags_valid = items;
+  return 0;
+}
+
+}  // namespace fs3d

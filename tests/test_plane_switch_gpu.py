@@ -1,0 +1,32 @@
+"""Changes between ticks of the active items and ticks of everything on one large world,
+against the byte kernels: an odd and an even number of dense passes in between, and
+runs that begin at either parity."""
+import pytest
+
+from conftest import announce
+
+pytestmark = pytest.mark.gpu
+
+SHAPE = (1024, 1031, 517)  # over 2^29 voxels
+
+
+def same(a, b, what):
+    assert a.tick_count == b.tick_count
+    assert a.hash() == b.hash(), what
+
+
+@pytest.mark.parametrize("t0", [0, 1])
+def test_runs_between_changes_of_schedule(gpu, t0):
+    announce(f"changes of schedule between runs, from tick {t0}")
+    with gpu.World(SHAPE) as a, gpu.World(SHAPE, flags=gpu.DENSE) as b:
+        b.fuse = False  # single byte ticks of every row quad
+        for w in (a, b):
+            w.fill_boxes(7, side_min=5, side_max=60)
+            w.tick_count = t0
+        for dense in (3, 4, 5):
+            for items in (3, 4):
+                for skip, n in ((gpu.SKIP_AUTO, 4), (gpu.SKIP_OFF, dense), (gpu.SKIP_AUTO, items)):
+                    a.skip = skip
+                    a.run(n, 0)
+                    b.run(n, 0)
+                    same(a, b, (dense, items, skip, a.tick_count))
