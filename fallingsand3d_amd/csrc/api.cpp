@@ -280,7 +280,7 @@ bool plane_path(const fs3d_world *w, int nticks) {
   if (w->skip != FS3D_SKIP_OFF && w->skip != FS3D_SKIP_AUTO) return false;
   if (!w->skip && w->fuse_set && !w->fuse) return false;
   if (w->nx < 16 || plane_words(shape_of(w)) > kMaxPlaneWords) return false;
-  return w->plane.valid || nticks >= kPlaneMinTicks;
+  return w->plane.ready(item_ticks(w)) || nticks >= kPlaneMinTicks;
 }
 
 // Plane buffers (and the item lists) on first use; false (and the byte kernels from
@@ -296,8 +296,8 @@ bool ensure_planes(fs3d_world *w) {
                                  may_list(w) ? plane_words(plane_shape(w->nx, w->ny, w->nz, true)) : 0);
     for (int i = 0; i < 2 && e == hipSuccess; i++) e = hipMalloc(&w->planes[i], most * 16);
   }
-  if (created || w->planes_tiled != ps.tiled) {
-    w->planes_tiled = ps.tiled;
+  if (created || w->plane.tiled != ps.tiled) {
+    w->plane.tiled = ps.tiled;
     w->plane.valid = false;
     for (int i = 0; i < 2 && e == hipSuccess; i++) e = launch_plane_pad(ps, w->planes[i], w->stream);
   }
@@ -308,6 +308,7 @@ bool ensure_planes(fs3d_world *w) {
     w->item_waves = (u32)(std::max(cus, 1) * plane_list_blocks_per_cu() * 4);
     for (int i = 0; i < 2 && e == hipSuccess; i++) e = hipMalloc(&w->pflags[i], c.flag_words * sizeof(u64));
     if (e == hipSuccess) e = hipMalloc(&w->d_since, c.since_words * sizeof(u64));
+    if (e == hipSuccess) e = launch_fill_u64(w->d_since, c.since_words, 0, w->stream);
     if (e == hipSuccess) e = hipMalloc(&w->d_nitems, 2 * sizeof(u32));
     if (e == hipSuccess) e = launch_fill_u32(w->d_nitems, 2, 0, w->stream);
     if (e == hipSuccess) e = hipMalloc(&w->d_items, c.list_words * sizeof(u32));
@@ -428,7 +429,7 @@ int choose_path(fs3d_world *w, int nticks, bool *planes) {
 void ticked_planes(fs3d_world *w, int nticks) {
   w->masks_stale = true;
   // the items' unpacking has marked the bricks it wrote
-  w->occ_valid = w->occ_valid && w->plane.flags_valid && w->occ_track;
+  w->occ_valid = w->occ_valid && item_ticks(w) && w->occ_track;
   w->tick += (u64)nticks;
 }
 void ticked_bytes(fs3d_world *w, int nticks, int fin) {
@@ -520,7 +521,7 @@ int world_graph(fs3d_world *w, int nticks, int hash_every, bool planes, hipGraph
   // a plane graph pairs its ticks by the start tick's parity
   const int state = !planes ? w->cur
                             : 64 | w->cur | (w->plane.valid ? 8 | w->plane.cur << 1 : 0) | (int)(w->tick & 1u) << 2 |
-                                  (item_ticks(w) ? w->plane.flags << 4 | (w->plane.flags_valid ? 32 : 0) : 0);
+                                  (item_ticks(w) ? w->plane.flags << 4 | w->plane.first << 7 : 0);
   const auto key = std::make_tuple(nticks, hash_every, state);
   auto it = w->graphs.find(key);
   if (it == w->graphs.end()) {
@@ -684,12 +685,12 @@ int fs3d_world_set_voxel(fs3d_world *w, int32_t x, int32_t y, int32_t z, uint8_t
   if (seg + 1 < lr) e.bits |= 1ull << (seg + 1);
   e.edge_off = w->mask_words;
   if (w->plane.valid) {
-    const PlaneShape ps = plane_shape(w->nx, w->ny, w->nz, w->planes_tiled);
+    const PlaneShape ps = plane_shape(w->nx, w->ny, w->nz, w->plane.tiled);
     e.planes = static_cast<u32 *>(w->planes[w->plane.cur]);
     e.reserved = w->d_reserved;
     e.word = plane_word(ps, x, y, z);
     e.x = x;
-    if (w->plane.flags_valid) e.flags = w->pflags[w->plane.flags] + plane_cell_flags(ps, y, z, &e.nflags, &e.flag_stride);
+    if (w->plane.first != kAfterPack) e.flags = w->pflags[w->plane.flags] + plane_cell_flags(ps, y, z, &e.nflags, &e.flag_stride);
   }
   w->occ_valid = false;
   FS3D_HIP(launch_set_cell(e, next_note(w), w->stream));

@@ -238,7 +238,6 @@ struct fs3d_world {
   void *planes[2] = {nullptr, nullptr};
   fs3d::PlaneState plane;
   bool planes_off = false;
-  bool planes_tiled = false;  // the buffers' layout (its rows around the grid are zero)
   fs3d::u32 *d_reserved = nullptr;  // a byte >= 4 has been packed or set
   // ticks of the active items only: change flags of the last pass
   // (pflags[plane.flags]), items changed since the bytes were written, work list and

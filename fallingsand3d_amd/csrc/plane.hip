@@ -19,6 +19,7 @@
 // Single ticks are bound by memory (2048^3: 4.3 GB in 770 us, 5.6 TB/s), pairs by
 // their instructions (1.3 evaluations per row quad and tick with the halo).
 #include "plane_quad.h"
+#include "plane_plan.h"
 
 namespace fs3d {
 namespace {
@@ -275,16 +276,13 @@ __global__ __launch_bounds__(256) void plane_pair_kernel(PlaneArgs a) {
 // since does not change.  The destination then already holds the item: it is the
 // state of two passes ago.
 //
-// Flags are u64 masks over the words of a strip (bit = word), kFlags per cell, each flag
-// of all cells in a row (so that the plan's lanes read neighbouring words): any
-// change; a change of a block at the item's first or last word bit, row, layer; any
-// change in the last pass alone.  A flag may be set without need, never missing.
+// The flags are plane_plan.h's, each flag of all cells in a row, so that the plan's lanes
+// read neighbouring words.  A flag may be set without need, never missing.
 //
 // Sand columns over a pool at 2048^3, where 12 % of the items have work: 145 us per
 // pair of ticks (123 us of it instructions).  With planes kept as rows, where the line
 // around a word holds 512 cells of one row, the same pass took 280 us; a pass over
 // everything takes 820, the byte kernels' packed schedule 2 x 360.
-enum { kAny = 0, kXFirst, kXLast, kYFirst, kYLast, kZFirst, kZLast, kNow, kFlags };
 
 // One thread per cell: which items have work, appended to the list in word order;
 // clears the flags the pass will write (or, before a single tick, carries the old
@@ -304,34 +302,8 @@ __global__ __launch_bounds__(256) void plane_plan_kernel(const u64 *__restrict__
   if (c < ncell) {
     zr = c / strips;
     st = c - zr * strips;
-#pragma unroll
-    for (int dz = -1; dz <= 1; dz++)
-#pragma unroll
-      for (int dy = -1; dy <= 1; dy++) {
-        const int y = st + dy, z = zr + dz;
-        if (y < 0 || y >= strips || z < 0 || z >= zcells) continue;
-        const u64 *f = in + (z * strips + y);
-        u64 m = f[kAny];
-        if (m == 0) continue;
-        if (first == kAfterPackTick) {  // what can move in an item may touch all its sides
-          act |= m | (m >> 1) | (m << 1);
-          continue;
-        }
-        if (dy) m &= f[(size_t)(dy > 0 ? kYFirst : kYLast) * ncell];
-        if (dz) m &= f[(size_t)(dz > 0 ? kZFirst : kZLast) * ncell];
-        act |= m | ((m & f[(size_t)kXFirst * ncell]) >> 1) | ((m & f[(size_t)kXLast * ncell]) << 1);
-      }
-    act &= bits;
-    const u64 *f = in + c;
-    const u64 now = first == kAfterPack ? 0ull : f[(size_t)kNow * ncell];
-    if (first != kNotFirst)
-      since[c] = now;
-    else if (now)
-      since[c] |= now;
-#pragma unroll
-    for (int i = 0; i < kFlags; i++)
-      out[(size_t)i * ncell + c] =
-          carry && i != kNow ? f[(size_t)(first == kAfterPackTick ? kAny : i) * ncell] : 0ull;
+    act = plan_words(in, strips, zcells, st, zr, first) & bits;
+    plan_flags(in, out, since, (size_t)c, (size_t)ncell, carry != 0, first);
   }
   const int n = __builtin_popcountll(act) + (virt && ((act >> (lr - 1)) & 1u) ? 1 : 0);
   int incl = n;

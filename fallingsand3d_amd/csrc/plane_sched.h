@@ -7,16 +7,20 @@
 
 namespace fs3d {
 
-// What the first pass over the active items must know: nothing, that the grid has just
-// been packed (every flag is set), or packed and ticked once (plane.h).
+// What a pass over the active items must know of the flags before it: those of a pass
+// like it, none (the grid has just been packed: every flag is set), or those of packing
+// and ticking in one pass (plane.h).
 enum { kNotFirst = 0, kAfterPack, kAfterPackTick };
 
 // A world's planes between calls.
 struct PlaneState {
-  bool valid = false;        // planes[cur] holds the current state
+  bool valid = false;  // planes[cur] holds the current state
+  bool tiled = false;  // the layout of the buffers
   int cur = 0;
-  int flags = 0;             // flag buffer and list counter of the next pass over the items
-  bool flags_valid = false;  // the flag buffer describes the last pass (exactly, or too many)
+  int flags = 0;           // flag buffer and list counter of the next pass over the items
+  int first = kAfterPack;  // and what that pass must know of the flags: one that has only
+                           // packed and ticked leaves others than a pass over the items
+  bool ready(bool want_tiled) const { return valid && tiled == want_tiled; }
 };
 
 // A pass: one tick, or the ticks t (odd) and t + 1.
@@ -47,7 +51,7 @@ int plane_passes(PlaneState *st, bool items, uint64_t t0, int nticks, int hash_e
   // an even first tick is done while packing
   const bool packs = !st->valid, ticks_too = packs && !(t0 & 1u);
   st->valid = false;  // should a launch fail, the bytes are the state
-  int first = ticks_too ? kAfterPackTick : packs || !st->flags_valid ? kAfterPack : kNotFirst;
+  int first = ticks_too ? kAfterPackTick : packs ? kAfterPack : st->first;
   if (packs) {
     if (int rc = ops.packed(items)) return rc;
     if (int rc = ticks_too ? ops.pack_tick(src, items ? f : -1) : ops.pack(src)) return rc;
@@ -78,7 +82,7 @@ int plane_passes(PlaneState *st, bool items, uint64_t t0, int nticks, int hash_e
   st->cur = src;
   st->valid = true;
   st->flags = f;
-  st->flags_valid = items;
+  st->first = items ? first : (int)kAfterPack;
   return 0;
 }
 

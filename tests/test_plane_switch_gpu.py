@@ -30,3 +30,21 @@ def test_runs_between_changes_of_schedule(gpu, t0):
                     a.run(n, 0)
                     b.run(n, 0)
                     same(a, b, (dense, items, skip, a.tick_count))
+
+
+@pytest.mark.parametrize("t0", [0, 1])
+@pytest.mark.parametrize("n", [1, 2, 3])
+def test_short_runs_after_a_change_of_schedule(gpu, n, t0):
+    announce(f"runs of {n} after a change of schedule, from tick {t0}")
+    with gpu.World(SHAPE, flags=gpu.DENSE) as a, gpu.World(SHAPE, flags=gpu.DENSE) as b:
+        b.fuse = False
+        for w in (a, b):
+            w.fill_boxes(8, side_min=5, side_max=60)
+            w.tick_count = t0
+            w.run(10, 0)
+        for skip, first in ((gpu.SKIP_AUTO, n), (gpu.SKIP_OFF, n), (gpu.SKIP_AUTO, n), (gpu.SKIP_OFF, 4), (gpu.SKIP_AUTO, n)):
+            a.skip = skip
+            for k in (first, n, 1, 1, n):
+                a.step(k)
+                b.step(k)
+            same(a, b, (skip, a.tick_count))
