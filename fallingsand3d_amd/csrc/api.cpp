@@ -114,8 +114,8 @@ void release(fs3d_world *w) {
   for (int i = 0; i < 2; i++)
     if (w->planes[i]) (void)hipFree(w->planes[i]);
   if (w->d_reserved) (void)hipFree(w->d_reserved);
-  for (int i = 0; i < 2; i++)
-    if (w->pflags[i]) (void)hipFree(w->pflags[i]);
+  for (u64 *f : w->pflags)
+    if (f) (void)hipFree(f);
   if (w->d_since) (void)hipFree(w->d_since);
   if (w->d_items) (void)hipFree(w->d_items);
   if (w->d_nitems) (void)hipFree(w->d_nitems);
@@ -306,11 +306,11 @@ bool ensure_planes(fs3d_world *w) {
     int cus = 0;
     e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, w->dev);
     w->item_waves = (u32)(std::max(cus, 1) * plane_list_blocks_per_cu() * 4);
-    for (int i = 0; i < 2 && e == hipSuccess; i++) e = hipMalloc(&w->pflags[i], c.flag_words * sizeof(u64));
+    for (int i = 0; i < kFlagBufs && e == hipSuccess; i++) e = hipMalloc(&w->pflags[i], c.flag_words * sizeof(u64));
     if (e == hipSuccess) e = hipMalloc(&w->d_since, c.since_words * sizeof(u64));
     if (e == hipSuccess) e = launch_fill_u64(w->d_since, c.since_words, 0, w->stream);
-    if (e == hipSuccess) e = hipMalloc(&w->d_nitems, 2 * sizeof(u32));
-    if (e == hipSuccess) e = launch_fill_u32(w->d_nitems, 2, 0, w->stream);
+    if (e == hipSuccess) e = hipMalloc(&w->d_nitems, kFlagBufs * sizeof(u32));
+    if (e == hipSuccess) e = launch_fill_u32(w->d_nitems, kFlagBufs, 0, w->stream);
     if (e == hipSuccess) e = hipMalloc(&w->d_items, c.list_words * sizeof(u32));
   }
   if (e == hipSuccess) return true;
@@ -322,8 +322,8 @@ bool ensure_planes(fs3d_world *w) {
   for (int i = 0; i < 2; i++) {
     if (w->planes[i]) (void)hipFree(w->planes[i]);
     w->planes[i] = nullptr;
-    drop(w->pflags[i]);
   }
+  for (u64 *&f : w->pflags) drop(f);
   drop(w->d_reserved);
   drop(w->d_since);
   drop(w->d_nitems);
@@ -346,7 +346,7 @@ struct PlaneLaunch {
   }
   int packed(bool items) const {
     FS3D_HIP(launch_fill_u32(w->d_reserved, 1, 0, w->stream));
-    if (items) FS3D_HIP(launch_fill_u32(w->d_nitems, 2, 0, w->stream));
+    if (items) FS3D_HIP(launch_fill_u32(w->d_nitems, kFlagBufs, 0, w->stream));
     return FS3D_OK;
   }
   int pack(int src) const {
@@ -381,9 +381,11 @@ struct PlaneLaunch {
     return p.hash ? finalize(p.hash) : FS3D_OK;
   }
   int item_pass(const PlanePass &p) const {
+    const int next = next_flags(p.flags), before = next_flags(next);
     FS3D_HIP(launch_plane_list(ps, w->planes[p.src], w->planes[p.src ^ 1], w->tick + (u64)p.k, tick_dev, (u32)p.k,
-                               p.pair, p.first, w->pflags[p.flags], w->pflags[p.flags ^ 1], w->d_since, w->d_items,
-                               w->d_nitems + p.flags, w->d_nitems + (p.flags ^ 1), w->item_waves, w->stream));
+                               p.pair, p.first, w->pflags[p.flags], p.older,
+                               p.older == kNoFlags ? nullptr : w->pflags[before], w->pflags[next], w->d_since,
+                               w->d_items, w->d_nitems + p.flags, w->d_nitems + next, w->item_waves, w->stream));
     return FS3D_OK;
   }
   int unpack(int src, int f) const {
@@ -521,7 +523,7 @@ int world_graph(fs3d_world *w, int nticks, int hash_every, bool planes, hipGraph
   // a plane graph pairs its ticks by the start tick's parity
   const int state = !planes ? w->cur
                             : 64 | w->cur | (w->plane.valid ? 8 | w->plane.cur << 1 : 0) | (int)(w->tick & 1u) << 2 |
-                                  (item_ticks(w) ? w->plane.flags << 4 | w->plane.first << 7 : 0);
+                                  (item_ticks(w) ? w->plane.flags << 4 | w->plane.first << 7 | w->plane.older << 9 : 0);
   const auto key = std::make_tuple(nticks, hash_every, state);
   auto it = w->graphs.find(key);
   if (it == w->graphs.end()) {
@@ -741,6 +743,7 @@ int fs3d_world_set_tick(fs3d_world *w, uint64_t tick) {
   if (int rc = check_world(w)) return rc;
   FS3D_HIP(hipSetDevice(w->dev));
   if (int rc = mark_all(w)) return rc;
+  if ((tick ^ w->tick) & 1u) w->plane.parity_repeats();
   w->tick = tick;
   return clear_error();
 }

@@ -239,10 +239,10 @@ struct fs3d_world {
   fs3d::PlaneState plane;
   bool planes_off = false;
   fs3d::u32 *d_reserved = nullptr;  // a byte >= 4 has been packed or set
-  // ticks of the active items only: change flags of the last pass
-  // (pflags[plane.flags]), items changed since the bytes were written, work list and
+  // ticks of the active items only: change flags of the last passes (plane_sched.h),
+  // items changed since the bytes were written, work list and
   // its counters
-  fs3d::u64 *pflags[2] = {nullptr, nullptr}, *d_since = nullptr;
+  fs3d::u64 *pflags[fs3d::kFlagBufs] = {}, *d_since = nullptr;
   fs3d::u32 *d_items = nullptr, *d_nitems = nullptr;
   fs3d::u32 item_waves = 0;
   bool masks_stale = false;         // plane ticks have run since the change masks were last exact

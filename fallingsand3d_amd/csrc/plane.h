@@ -86,13 +86,15 @@ PlaneCells plane_cells(const PlaneShape &ps);
 size_t plane_cell_flags(const PlaneShape &ps, int y, int z, int *n, size_t *stride);
 int plane_list_blocks_per_cu();
 // A pass over the active items: ticks t and t + 1 (pair, t odd) or tick t (of
-// either parity; *tick_dev + k_off has t's).  flags_in: the pass before; flags_out:
-// this one's; since: items changed since the bytes were written; first: kAfterPack
-// for the first pass after packing (every flag set), kAfterPackTick for the first one
-// after launch_plane_pack_even.  *count is 0 before; the pass clears *next_count.
+// either parity; *tick_dev + k_off has t's).  flags_in: the pass before, older: the one
+// before that, where the pass before ran one tick (else nullptr); flags_out: this one's;
+// since: items changed since the bytes were written; first and older_first: kAfterPack
+// for the flags after packing (every one set), kAfterPackTick for those of
+// launch_plane_pack_even.  *count is 0 before; the pass clears *next_count.
 hipError_t launch_plane_list(const PlaneShape &ps, const void *src, void *dst, u64 t, const u64 *tick_dev, u32 k_off,
-                             bool pair, int first, const u64 *flags_in, u64 *flags_out, u64 *since, u32 *list,
-                             u32 *count, u32 *next_count, u32 nwaves, hipStream_t s);
+                             bool pair, int first, const u64 *flags_in, int older_first, const u64 *older,
+                             u64 *flags_out, u64 *since, u32 *list, u32 *count, u32 *next_count, u32 nwaves,
+                             hipStream_t s);
 // Writes the bytes of the items in since or flags (the last pass's) and clears since;
 // dirty (or nullptr): a bit per 8^3 brick, set for those that hold a written item.
 hipError_t launch_plane_unpack_cells(const PlaneShape &ps, const void *planes, u8 *g, const u64 *flags, u64 *since,

@@ -290,9 +290,10 @@ __global__ __launch_bounds__(256) void plane_pair_kernel(PlaneArgs a) {
 // the first pass over a grid just packed, whose flags are all set).
 // A full last word (nx a multiple of 64) has a virtual neighbour, word lr, whose
 // lane evaluates the half blocks at the row's end.
-__global__ __launch_bounds__(256) void plane_plan_kernel(const u64 *__restrict__ in, u64 *__restrict__ out,
-                                                         u64 *__restrict__ since, int strips, int zcells, int lr,
-                                                         int virt, int carry, int first, u32 *list, u32 *count) {
+__global__ __launch_bounds__(256) void plane_plan_kernel(const u64 *__restrict__ in, const u64 *__restrict__ older,
+                                                         u64 *__restrict__ out, u64 *__restrict__ since, int strips,
+                                                         int zcells, int lr, int virt, int first, int older_first,
+                                                         u32 *list, u32 *count) {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int ncell = strips * zcells;
   const int c = (int)blockIdx.x * 256 + (int)threadIdx.x;
@@ -302,8 +303,10 @@ __global__ __launch_bounds__(256) void plane_plan_kernel(const u64 *__restrict__
   if (c < ncell) {
     zr = c / strips;
     st = c - zr * strips;
-    act = plan_words(in, strips, zcells, st, zr, first) & bits;
-    plan_flags(in, out, since, (size_t)c, (size_t)ncell, carry != 0, first);
+    act = plan_words(in, strips, zcells, st, zr, first);
+    if (older) act |= plan_words(older, strips, zcells, st, zr, older_first);
+    act &= bits;
+    plan_flags(in, out, since, (size_t)c, (size_t)ncell, first);
   }
   const int n = __builtin_popcountll(act) + (virt && ((act >> (lr - 1)) & 1u) ? 1 : 0);
   int incl = n;
@@ -823,8 +826,9 @@ int plane_list_blocks_per_cu() {
 }
 
 hipError_t launch_plane_list(const PlaneShape &ps, const void *src, void *dst, u64 t, const u64 *tick_dev, u32 k_off,
-                             bool pair, int first, const u64 *flags_in, u64 *flags_out, u64 *since, u32 *list,
-                             u32 *count, u32 *next_count, u32 nwaves, hipStream_t s) {
+                             bool pair, int first, const u64 *flags_in, int older_first, const u64 *older,
+                             u64 *flags_out, u64 *since, u32 *list, u32 *count, u32 *next_count, u32 nwaves,
+                             hipStream_t s) {
   PlaneArgs a{};
   fill_args(a, ps);
   a.src = static_cast<const u32x4 *>(src);
@@ -835,8 +839,8 @@ hipError_t launch_plane_list(const PlaneShape &ps, const void *src, void *dst, u
   a.zlen = kItemLayers;
   const PlaneCells c = plane_cells(ps);
   const unsigned plan = (unsigned)((c.since_words + 255) / 256);
-  hipLaunchKernelGGL(plane_plan_kernel, dim3(plan), dim3(256), 0, s, flags_in, flags_out, since, c.strips, c.zcells,
-                     ps.lr, c.virt, pair ? 0 : 1, first, list, count);
+  hipLaunchKernelGGL(plane_plan_kernel, dim3(plan), dim3(256), 0, s, flags_in, older, flags_out, since, c.strips,
+                     c.zcells, ps.lr, c.virt, first, older_first, list, count);
   const dim3 grid(nwaves / 4);
   // the caller's t has the tick's parity, on replays too
   if (pair)

@@ -49,16 +49,13 @@ FS3D_HD u64 plan_words(const u64 *in, int strips, int zcells, int st, int zr, in
 
 // The flags of cell c before the pass adds to them, and the items changed since the bytes
 // were written, to which the pass before adds its changes.
-FS3D_HD void plan_flags(const u64 *in, u64 *out, u64 *since, size_t c, size_t ncell, bool carry, int first) {
-  const u64 *f = in + c;
-  const u64 now = first == kAfterPack ? 0 : f[(size_t)kNow * ncell];
+FS3D_HD void plan_flags(const u64 *in, u64 *out, u64 *since, size_t c, size_t ncell, int first) {
+  const u64 now = first == kAfterPack ? 0 : in[(size_t)kNow * ncell + c];
   if (first != kNotFirst)
     since[c] = now;
   else if (now)
     since[c] |= now;
-  for (int i = 0; i < kFlags; i++)
-    out[(size_t)i * ncell + c] =
-        carry && i != kNow ? f[(size_t)(first == kAfterPackTick ? (int)kAny : i) * ncell] : 0;
+  for (int i = 0; i < kFlags; i++) out[(size_t)i * ncell + c] = 0;
 }
 
 }  // namespace plane

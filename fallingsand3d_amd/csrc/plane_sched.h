@@ -9,18 +9,29 @@ namespace fs3d {
 
 // What a pass over the active items must know of the flags before it: those of a pass
 // like it, none (the grid has just been packed: every flag is set), or those of packing
-// and ticking in one pass (plane.h).
-enum { kNotFirst = 0, kAfterPack, kAfterPackTick };
+// and ticking in one pass (plane.h).  kNoFlags: there is nothing to read.
+enum { kNotFirst = 0, kAfterPack, kAfterPackTick, kNoFlags };
+constexpr int kFlagBufs = 3;  // the last pass's, the one before's, and the next one's
+inline int next_flags(int f) { return f + 1 < kFlagBufs ? f + 1 : 0; }
 
 // A world's planes between calls.
 struct PlaneState {
   bool valid = false;  // planes[cur] holds the current state
   bool tiled = false;  // the layout of the buffers
   int cur = 0;
-  int flags = 0;           // flag buffer and list counter of the next pass over the items
-  int first = kAfterPack;  // and what that pass must know of the flags: one that has only
-                           // packed and ticked leaves others than a pass over the items
+  int flags = 0;           // the last pass's flag buffer and the next one's list counter,
+  int first = kAfterPack;  // and what the next pass must know of those flags: a pass that has
+                           // only packed and ticked leaves others than one over the items
+  int older = kNoFlags;    // the same for the flags of the pass before it.  A block rests when
+                           // neither parity's last tick changed it or a cell of it, so
+                           // behind a pass of one tick the one before counts too.
   bool ready(bool want_tiled) const { return valid && tiled == want_tiled; }
+  // The next tick has the parity of the last one: the other parity's last tick is not
+  // among the flags.
+  void parity_repeats() {
+    first = kAfterPack;
+    older = kNoFlags;
+  }
 };
 
 // A pass: one tick, or the ticks t (odd) and t + 1.
@@ -28,16 +39,16 @@ struct PlanePass {
   int k;       // ticks of the run before it
   bool pair;
   int src;     // reads planes[src], writes planes[src ^ 1]
-  int flags;   // items: reads flags[flags], writes flags[flags ^ 1], appends to counter[flags]
-               // and clears counter[flags ^ 1]
-  int first;   // items: kNotFirst, ...
+  int flags;   // items: reads flag buffer `flags` (and the one before it), writes the next one,
+               // appends to counter `flags` and clears the next one
+  int first, older;  // items: kNotFirst, ...
   int hash;    // everything: the hash (1, 2, ...) of planes[src] taken in the same launch, or 0
 };
 
 // nticks ticks from tick t0 with a hash every hash_every (0: none); items: passes over
 // the active items only.  *st becomes the state after them.  Ops, each returning 0 or
 // an error:
-//   packed(items)            the grid is about to be packed; items: clears both counters
+//   packed(items)            the grid is about to be packed; items: clears the counters
 //   pack(src)                bytes to planes[src]
 //   pack_tick(src, flags)    the same and tick t0 (even); flags: -1 or the flag buffer to write
 //   all_flags(flags)         every flag set
@@ -52,6 +63,7 @@ int plane_passes(PlaneState *st, bool items, uint64_t t0, int nticks, int hash_e
   const bool packs = !st->valid, ticks_too = packs && !(t0 & 1u);
   st->valid = false;  // should a launch fail, the bytes are the state
   int first = ticks_too ? kAfterPackTick : packs ? kAfterPack : st->first;
+  int older = packs ? kNoFlags : st->older;
   if (packs) {
     if (int rc = ops.packed(items)) return rc;
     if (int rc = ticks_too ? ops.pack_tick(src, items ? f : -1) : ops.pack(src)) return rc;
@@ -68,10 +80,11 @@ int plane_passes(PlaneState *st, bool items, uint64_t t0, int nticks, int hash_e
     const bool with = due && !items && !pair;
     if (due && !with)
       if (int rc = ops.hash(src, due)) return rc;
-    const PlanePass p{k, pair, src, f, first, with ? due : 0};
+    const PlanePass p{k, pair, src, f, first, older, with ? due : 0};
     if (int rc = items ? ops.item_pass(p) : ops.pass(p)) return rc;
     src ^= 1;
-    if (items) f ^= 1;  // (a pass over everything clears no counter)
+    if (items) f = next_flags(f);  // (a pass over everything clears no counter)
+    older = pair ? (int)kNoFlags : first == kAfterPackTick ? (int)kAfterPackTick : (int)kNotFirst;
     first = kNotFirst;
     k += pair ? 2 : 1;
     due = hashed_after(k - 1) ? k / hash_every : 0;
@@ -83,6 +96,7 @@ int plane_passes(PlaneState *st, bool items, uint64_t t0, int nticks, int hash_e
   st->valid = true;
   st->flags = f;
   st->first = items ? first : (int)kAfterPack;
+  st->older = items ? older : (int)kNoFlags;
   return 0;
 }
 

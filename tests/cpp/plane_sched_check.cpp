@@ -22,12 +22,13 @@ typedef unsigned char u8;
   } while (0)
 
 // ---- list counters ----
-// The plan appends to the pass's counter, the pass reads it and clears the other one.
+// The plan appends to the pass's counter, the pass reads it and clears the next one.
 struct Counters {
-  unsigned n[2] = {0, 0};
+  unsigned n[kFlagBufs] = {};
   unsigned items = 100;
   int packed(bool with_items) {
-    if (with_items) n[0] = n[1] = 0;
+    if (with_items)
+      for (unsigned &c : n) c = 0;
     return 0;
   }
   int pack(int) { return 0; }
@@ -39,7 +40,7 @@ struct Counters {
   int item_pass(const PlanePass &p) {
     CHECK(n[p.flags] == 0);
     n[p.flags] += items;
-    n[p.flags ^ 1] = 0;
+    n[next_flags(p.flags)] = 0;
     return 0;
   }
   int unpack(int, int) { return 0; }
@@ -78,7 +79,7 @@ struct Model {
   int nx, ny, nz, lr, strips, zcells;
   size_t ncell;
   std::vector<u8> bytes, buf[2];
-  std::vector<u64> flags[2], since;
+  std::vector<u64> flags[kFlagBufs], since;
   PlaneState st;
   bool items = true;
   u64 t = 0;
@@ -90,10 +91,8 @@ struct Model {
     zcells = ((nz + 1) / 2 + 7) / 8;
     ncell = (size_t)strips * zcells;
     bytes.assign((size_t)nx * ny * nz, 0);
-    for (int i = 0; i < 2; i++) {
-      buf[i].assign(bytes.size(), 9);
-      flags[i].assign(ncell * plane::kFlags, 0x5555);
-    }
+    for (auto &b : buf) b.assign(bytes.size(), 9);
+    for (auto &f : flags) f.assign(ncell * plane::kFlags, 0x5555);
     since.assign(ncell, 0);
   }
   size_t at(int x, int y, int z) const { return ((size_t)z * ny + y) * nx + x; }
@@ -188,17 +187,20 @@ struct Model {
     return 0;
   }
   int item_pass(const PlanePass &p) {
-    std::vector<u64> act(ncell, 0), *out = &flags[p.flags ^ 1];
+    const std::vector<u64> &in = flags[p.flags], &older = flags[next_flags(next_flags(p.flags))];
+    std::vector<u64> act(ncell, 0), *out = &flags[next_flags(p.flags)];
     const u64 words = (1ull << lr) - 1;
     listed = 0;
     for (int z = 0; z < zcells; z++)
       for (int y = 0; y < strips; y++) {
         const size_t c = (size_t)z * strips + y;
-        act[c] = plane::plan_words(flags[p.flags].data(), strips, zcells, y, z, p.first) & words;
+        act[c] = plane::plan_words(in.data(), strips, zcells, y, z, p.first);
+        if (p.older != kNoFlags) act[c] |= plane::plan_words(older.data(), strips, zcells, y, z, p.older);
+        act[c] &= words;
         listed += __builtin_popcountll(act[c]);
       }
     for (size_t c = 0; c < ncell; c++)
-      plane::plan_flags(flags[p.flags].data(), out->data(), since.data(), c, ncell, !p.pair, p.first);
+      plane::plan_flags(in.data(), out->data(), since.data(), c, ncell, p.first);
     std::vector<u8> s1, s2;
     tick(buf[p.src], s1, t + (u64)p.k, out, &act);
     if (p.pair)
@@ -245,6 +247,10 @@ struct Model {
     CHECK(bytes == want);
     return 0;
   }
+  void set_tick(u64 tick) {
+    if ((tick ^ t) & 1) st.parity_repeats();
+    t = tick;
+  }
   void poke(int x, int y, int z, u8 v) {
     bytes[at(x, y, z)] = v;
     if (!st.valid) return;
@@ -274,7 +280,7 @@ static int worlds() {
     w.t = seed % 2;
     w.fill(rng);
     for (int k = 0; k < 25; k++) {
-      switch (rng() % 8) {
+      switch (rng() % 10) {
         case 0: w.items = !w.items; break;
         case 1:
           for (int i = 0; i < 5; i++)
@@ -283,6 +289,7 @@ static int worlds() {
         case 2:
           if (rng() % 3 == 0) w.fill(rng);
           break;
+        case 3: w.set_tick(w.t + rng() % 3); break;
         default: CHECK(w.run(1 + (int)(rng() % 6), (int)(rng() % 3)) == 0);
       }
     }
@@ -310,13 +317,30 @@ static int switches() {
   return 0;
 }
 
+// What has come to rest is left alone, however the ticks are taken.
+static int rest() {
+  for (int every = 0; every < 2; every++)
+    for (int n : {1, 2, 5}) {
+      std::mt19937 rng(5);
+      Model w(192, 9, 38);
+      w.fill(rng);
+      for (u8 &c : w.bytes) c = c == 3 ? 0 : c;  // sand comes to rest
+      for (int k = 0; k < 150; k += n) CHECK(w.run(k < 3 ? 3 : n, every) == 0);
+      CHECK(w.listed == 0);
+      w.poke(100, 4, 30, 2);
+      for (int k = 0; k < 4; k++) CHECK(w.run(n, every) == 0);
+      CHECK(w.listed > 0 && w.listed < 30);
+    }
+  return 0;
+}
+
 int main(int argc, char **argv) {
   if (argc < 2) return 2;
   lut.resize(4 * 65536);
   FILE *f = std::fopen(argv[1], "rb");
   if (!f || std::fread(lut.data(), 2, lut.size(), f) != lut.size()) return 2;
   std::fclose(f);
-  if (counters() || switches() || worlds()) return 1;
+  if (counters() || switches() || rest() || worlds()) return 1;
   std::printf("plane schedule checks passed\n");
   return 0;
 }
