@@ -268,19 +268,15 @@ PlaneShape shape_of(const fs3d_world *w) { return plane_shape(w->nx, w->ny, w->n
 // Runs of ticks go through the bit planes: packed once, ticked in pairs at a
 // quarter of the bytes and without table lookups, unpacked once.  The byte
 // kernels keep what asks for them (an explicit segment or schedule, sweep
-// counters, fusion switched off), runs of at most kPlaneMinTicks - 1 ticks on a
-// grid that is not in planes yet (packing and unpacking cost about a byte tick
-// each: 512^3 24 + 42 us against 42 us per tick), rows under 16 cells (a row
-// takes whole 16-byte words, so planes would outgrow the bytes) and plane grids
+// counters, fusion switched off), short runs (planes_suit), rows under 16 cells (a
+// row takes whole 16-byte words, so planes would outgrow the bytes) and plane grids
 // of 4 GiB and more (buffer addressing).
-constexpr int kPlaneMinTicks = 3;
-
-bool plane_path(const fs3d_world *w, int nticks) {
+bool plane_path(const fs3d_world *w, int nticks, int hash_every) {
   if (w->planes_off || w->seg_req != 0 || w->d_stats || nticks < 1) return false;
   if (w->skip != FS3D_SKIP_OFF && w->skip != FS3D_SKIP_AUTO) return false;
   if (!w->skip && w->fuse_set && !w->fuse) return false;
   if (w->nx < 16 || plane_words(shape_of(w)) > kMaxPlaneWords) return false;
-  return w->plane.ready(item_ticks(w)) || nticks >= kPlaneMinTicks;
+  return planes_suit(w->plane, item_ticks(w), nticks, hash_every);
 }
 
 // Plane buffers (and the item lists) on first use; false (and the byte kernels from
@@ -419,8 +415,8 @@ int enqueue_planes(fs3d_world *w, int nticks, int hash_every, const u64 *tick_de
 
 // Which path the next nticks ticks take: decided once per call, with what that
 // path needs in place.
-int choose_path(fs3d_world *w, int nticks, bool *planes) {
-  *planes = plane_path(w, nticks) && ensure_planes(w);
+int choose_path(fs3d_world *w, int nticks, int hash_every, bool *planes) {
+  *planes = plane_path(w, nticks, hash_every) && ensure_planes(w);
   if (!*planes && nticks > 0 && w->skip && w->masks_stale)
     if (int rc = mark_all(w)) return rc;
   return FS3D_OK;
@@ -849,7 +845,7 @@ int fs3d_world_step(fs3d_world *w, int32_t nticks) {
   if (nticks < 0) return set_error(FS3D_ERR_INVALID, "nticks < 0");
   FS3D_HIP(hipSetDevice(w->dev));
   bool planes = false;
-  if (int rc = choose_path(w, nticks, &planes)) return rc;
+  if (int rc = choose_path(w, nticks, 0, &planes)) return rc;
   if (int rc = run_ticks(w, nticks, 0, planes)) return rc;
   return clear_error();
 }
@@ -859,7 +855,7 @@ int fs3d_world_tick(fs3d_world *w, uint64_t *hash) {
   if (!hash) return set_error(FS3D_ERR_INVALID, "hash is NULL");
   FS3D_HIP(hipSetDevice(w->dev));
   bool planes = false;
-  if (int rc = choose_path(w, 1, &planes)) return rc;
+  if (int rc = choose_path(w, 1, 1, &planes)) return rc;
   if (w->n <= kHashPostMax && !w->d_stats) {
     if (int rc = run_ticks(w, 1, 0, planes)) return rc;
     FS3D_HIP(launch_hash_post(w->buf[w->cur], w->n, w->d_parts, next_note(w), w->stream));
@@ -898,7 +894,7 @@ int fs3d_world_prepare_run(fs3d_world *w, int32_t nticks, int32_t hash_every) {
   const int nh = hash_every > 0 ? nticks / hash_every : 0;
   if (int rc = ensure_small(w, nh + 1)) return rc;
   bool planes = false;
-  if (int rc = choose_path(w, nticks, &planes)) return rc;
+  if (int rc = choose_path(w, nticks, hash_every, &planes)) return rc;
   hipGraphExec_t exec = nullptr;
   if (int rc = world_graph(w, nticks, hash_every, planes, &exec)) return rc;
   return clear_error();
@@ -913,7 +909,7 @@ int fs3d_world_run(fs3d_world *w, int32_t nticks, int32_t hash_every, uint64_t *
   FS3D_HIP(hipSetDevice(w->dev));
   if (int rc = ensure_small(w, nh + 1)) return rc;
   bool planes = false;
-  if (int rc = choose_path(w, nticks, &planes)) return rc;
+  if (int rc = choose_path(w, nticks, hash_every, &planes)) return rc;
   hipGraphExec_t exec = nullptr;
   if (int rc = world_graph(w, nticks, hash_every, planes, &exec)) return rc;
   FS3D_HIP(launch_set_u64(w->d_small, w->tick, w->stream));

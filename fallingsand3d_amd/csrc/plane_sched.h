@@ -25,6 +25,7 @@ struct PlaneState {
   int older = kNoFlags;    // the same for the flags of the pass before it.  A block rests when
                            // neither parity's last tick changed it or a cell of it, so
                            // behind a pass of one tick the one before counts too.
+  int shorts = 0;          // runs under kPlaneMinTicks ticks since the last longer one
   bool ready(bool want_tiled) const { return valid && tiled == want_tiled; }
   // The next tick has the parity of the last one: the other parity's last tick is not
   // among the flags.
@@ -33,6 +34,26 @@ struct PlaneState {
     older = kNoFlags;
   }
 };
+
+// Whether a run takes the planes (a grid that can be in planes; items: passes over the
+// active items only) or stays on bytes.
+//
+// Packing and unpacking everything cost about a byte tick each (512^3: 24 + 42 us), so
+// runs under three ticks do not pay for them, nor for the unpacking alone: one tick of a
+// grid in planes takes 193 us at 800^3, on bytes 57 with columns falling and 24 at rest
+// (512^3: 37 against 27 and 11; 64^3: 16 against 7).
+//
+// With items, only what moved is unpacked, but a single tick still takes more than on
+// bytes (1024^3, columns: 103 against 72 us; at rest 50 against 27), while going to bytes
+// and back takes two ticks of everything and a packing, 0.8 ms.  So such a run stays in
+// planes until it has been followed by that much waste.  (A hash per tick is cheaper on
+// planes: 320 against 407 us.)
+constexpr int kPlaneMinTicks = 3, kPlaneShortRuns = 24;
+inline bool planes_suit(const PlaneState &st, bool items, int nticks, int hash_every) {
+  if (nticks >= kPlaneMinTicks) return true;
+  const bool hashed = hash_every > 0 && hash_every <= nticks;
+  return items && st.ready(true) && (hashed || st.shorts < kPlaneShortRuns);
+}
 
 // A pass: one tick, or the ticks t (odd) and t + 1.
 struct PlanePass {
@@ -94,6 +115,7 @@ int plane_passes(PlaneState *st, bool items, uint64_t t0, int nticks, int hash_e
   if (int rc = ops.unpack(src, items ? f : -1)) return rc;
   st->cur = src;
   st->valid = true;
+  st->shorts = nticks >= kPlaneMinTicks ? 0 : st->shorts + 1;
   st->flags = f;
   st->first = items ? first : (int)kAfterPack;
   st->older = items ? older : (int)kNoFlags;

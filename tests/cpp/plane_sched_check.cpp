@@ -83,7 +83,8 @@ struct Model {
   PlaneState st;
   bool items = true;
   u64 t = 0;
-  long listed = 0;  // words of the last pass over the items
+  bool any_path = false;  // in planes whenever the grid is there, as a long run would
+  long listed = 0;        // words of the last pass over the items
 
   Model(int x, int y, int z) : nx(x), ny(y), nz(z) {
     lr = (nx + 63) / 64;
@@ -226,8 +227,7 @@ struct Model {
   // a world's calls
   int run(int n, int every) {
     const std::vector<u8> before = bytes;
-    const int min_ticks = 3;  // fewer on a grid that is not in planes stay on bytes
-    if (st.ready(items) || n >= min_ticks) {
+    if (any_path ? st.ready(items) || n >= kPlaneMinTicks : planes_suit(st, items, n, every)) {
       if (st.tiled != items) {
         st.tiled = items;
         st.valid = false;
@@ -277,6 +277,7 @@ static int worlds() {
   for (unsigned seed = 1; seed <= 40; seed++) {
     std::mt19937 rng(seed);
     Model w(seed & 1 ? 150 : 192, 9, 37 + (int)(seed % 3));
+    w.any_path = seed % 4 < 2;
     w.t = seed % 2;
     w.fill(rng);
     for (int k = 0; k < 25; k++) {
@@ -304,6 +305,7 @@ static int switches() {
       std::mt19937 rng(t0 + 7);
       Model w(192, 9, 38);
       w.t = t0;
+      w.any_path = true;
       w.fill(rng);
       w.items = false;
       CHECK(w.run(10, 0) == 0);
@@ -323,6 +325,7 @@ static int rest() {
     for (int n : {1, 2, 5}) {
       std::mt19937 rng(5);
       Model w(192, 9, 38);
+      w.any_path = true;
       w.fill(rng);
       for (u8 &c : w.bytes) c = c == 3 ? 0 : c;  // sand comes to rest
       for (int k = 0; k < 150; k += n) CHECK(w.run(k < 3 ? 3 : n, every) == 0);
@@ -334,13 +337,33 @@ static int rest() {
   return 0;
 }
 
+// Which runs take the planes.
+static int paths() {
+  PlaneState dense, items;
+  for (int n : {1, 2}) {
+    CHECK(!planes_suit(dense, false, n, 0) && !planes_suit(items, true, n, 0));
+    dense.valid = true;  // in planes, which are as good as bytes for them
+    CHECK(!planes_suit(dense, false, n, 0) && !planes_suit(dense, false, n, 1));
+    dense.valid = false;
+  }
+  CHECK(planes_suit(dense, false, 3, 0) && planes_suit(items, true, 3, 0));
+  Counters ops;
+  items.tiled = true;
+  CHECK(plane_passes(&items, true, 0, 4, 0, ops) == 0);
+  int k = 0;  // single ticks on planes before they go to bytes
+  for (; k < 1000 && planes_suit(items, true, 1, 0); k++) CHECK(plane_passes(&items, true, (u64)k, 1, 0, ops) == 0);
+  CHECK(k == kPlaneShortRuns && planes_suit(items, true, 1, 1) && planes_suit(items, true, 3, 0));
+  CHECK(plane_passes(&items, true, (u64)k, 3, 0, ops) == 0 && planes_suit(items, true, 1, 0));
+  return 0;
+}
+
 int main(int argc, char **argv) {
   if (argc < 2) return 2;
   lut.resize(4 * 65536);
   FILE *f = std::fopen(argv[1], "rb");
   if (!f || std::fread(lut.data(), 2, lut.size(), f) != lut.size()) return 2;
   std::fclose(f);
-  if (counters() || switches() || rest() || worlds()) return 1;
+  if (counters() || paths() || switches() || rest() || worlds()) return 1;
   std::printf("plane schedule checks passed\n");
   return 0;
 }
