@@ -251,10 +251,17 @@ int dense_chunk_seg(const fs3d_world *w) { return w->seg_req == 0 && w->nx > 102
 // the destination already holding its bytes.
 constexpr size_t kInPlaceMaxBytes = size_t(1) << 27;
 
-// Whether the plane ticks of a skipping world visit only its active items.  Below
-// this size a pass over everything is as fast as listing what moves.  (Thin grids'
-// tiles would outgrow the addressing.)
-constexpr u64 kItemsMinVoxels = 1ull << 29;
+// Whether the plane ticks of a skipping world visit only its active items.  (Thin grids'
+// tiles would outgrow the addressing.)  us per tick of runs of 4 and 30, everything /
+// items / the skipping byte ticks:
+//             columns falling                at rest                        boxes falling
+//   640^3     41, 17 / 40, 20 / 64, 49       40, 17 / 29, 17 / 33, 28       42, 18 / 75, 27 / 133, 108
+//   740^3     66, 26 / 40, 20 / 57, 46       67, 26 / 30, 17 / 30, 25       67, 27 / 110, 40 / 257, 215
+//   800^3     82, 35 / 41, 20 / 60, 49       83, 35 / 31, 17 / 29, 24       85, 36 / 129, 48 / 288, 239
+// (512^3: 20, 10 / 31, 19 / 31, 21; 21, 10 / 25, 16 / 17, 11; 22, 11 / 39, 20 / 50, 39.)
+// From 2^28 voxels on unpacking everything makes a short run of a world that mostly rests
+// slower than on bytes; with items it is not, and what moves a lot still gains.
+constexpr u64 kItemsMinVoxels = 1ull << 28;
 constexpr size_t kMaxPlaneWords = (1ull << 28) - 1;
 bool may_list(const fs3d_world *w) {
   return (u64)w->n > kItemsMinVoxels && plane_words(plane_shape(w->nx, w->ny, w->nz, true)) <= kMaxPlaneWords;

@@ -121,7 +121,7 @@ int fs3d_world_get_segment(const fs3d_world *w, int32_t *seg_bytes);
  * one); WAVES launches one wave per row-quad group that skips on its own (lower
  * per-tick overhead; best for small grids).  AUTO runs three and more ticks
  * on two bit planes (rows of 16 cells and more, planes under 4 GiB): every voxel
- * of grids up to 2^29, above that the 64 x 2 x 16 cell items in which something
+ * of grids up to 2^28, above that the 64 x 2 x 16 cell items in which something
  * moves; other ticks take SEGS above 2^17 waves of work per tick, else WAVES.
  * Hash ticks read settled segments in all three.  Worlds of up to 2^27 voxels tick in place with WAVES and LISTED (and
  * dense single ticks of rows up to 1024 bytes); the grid stays where

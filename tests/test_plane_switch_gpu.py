@@ -7,7 +7,8 @@ from conftest import announce
 
 pytestmark = pytest.mark.gpu
 
-SHAPE = (1024, 1031, 517)  # over 2^29 voxels
+SHAPE = (1024, 1031, 517)
+NEAR = (704, 640, 600)  # the fewest voxels, 2^28, whose items are listed
 
 
 def same(a, b, what):
@@ -15,10 +16,11 @@ def same(a, b, what):
     assert a.hash() == b.hash(), what
 
 
+@pytest.mark.parametrize("shape", [SHAPE, NEAR], ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("t0", [0, 1])
-def test_runs_between_changes_of_schedule(gpu, t0):
-    announce(f"changes of schedule between runs, from tick {t0}")
-    with gpu.World(SHAPE) as a, gpu.World(SHAPE, flags=gpu.DENSE) as b:
+def test_runs_between_changes_of_schedule(gpu, shape, t0):
+    announce(f"changes of schedule between runs of {shape}, from tick {t0}")
+    with gpu.World(shape) as a, gpu.World(shape, flags=gpu.DENSE) as b:
         b.fuse = False  # single byte ticks of every row quad
         for w in (a, b):
             w.fill_boxes(7, side_min=5, side_max=60)
