@@ -275,7 +275,7 @@ PlaneShape shape_of(const fs3d_world *w) { return plane_shape(w->nx, w->ny, w->n
 // Runs of ticks go through the bit planes: packed once, ticked in pairs at a
 // quarter of the bytes and without table lookups, unpacked once.  The byte
 // kernels keep what asks for them (an explicit segment or schedule, sweep
-// counters, fusion switched off), short runs (planes_suit), rows under 16 cells (a
+// counters, fusion switched off), what planes do not suit (planes_suit), rows under 16 cells (a
 // row takes whole 16-byte words, so planes would outgrow the bytes) and plane grids
 // of 4 GiB and more (buffer addressing).
 bool plane_path(const fs3d_world *w, int nticks, int hash_every) {
@@ -283,7 +283,7 @@ bool plane_path(const fs3d_world *w, int nticks, int hash_every) {
   if (w->skip != FS3D_SKIP_OFF && w->skip != FS3D_SKIP_AUTO) return false;
   if (!w->skip && w->fuse_set && !w->fuse) return false;
   if (w->nx < 16 || plane_words(shape_of(w)) > kMaxPlaneWords) return false;
-  return planes_suit(w->plane, item_ticks(w), nticks, hash_every);
+  return planes_suit(w->plane, {w->n, w->nx, w->skip != FS3D_SKIP_OFF, item_ticks(w), nticks, hash_every});
 }
 
 // Plane buffers (and the item lists) on first use; false (and the byte kernels from

@@ -46,13 +46,34 @@ struct PlaneState {
 // With items, only what moved is unpacked, but a single tick still takes more than on
 // bytes (1024^3, columns: 103 against 72 us; at rest 50 against 27), while going to bytes
 // and back takes two ticks of everything and a packing, 0.8 ms.  So such a run stays in
-// planes until it has been followed by that much waste.  (A hash per tick is cheaper on
+// planes until 24 of them in a row have wasted that much.  (A hash per tick is cheaper on
 // planes: 320 against 407 us.)
 constexpr int kPlaneMinTicks = 3, kPlaneShortRuns = 24;
-inline bool planes_suit(const PlaneState &st, bool items, int nticks, int hash_every) {
-  if (nticks >= kPlaneMinTicks) return true;
-  const bool hashed = hash_every > 0 && hash_every <= nticks;
-  return items && st.ready(true) && (hashed || st.shorts < kPlaneShortRuns);
+
+// The hash of planes takes longer than the one a byte tick takes as it writes, which tells
+// where the byte ticks run in place and in the last-level cache (512^3 boxes: 117 against
+// 72 us).  us per tick with a hash after every one, bytes / planes, boxes and rain:
+//   256^3 26, 13 / 25, 15     320^3 37, 19 / 40, 23     512^3 101, 52 / 127, 55
+//   560^3 216, 110 / 160, 71  (200^3 20, 13 / 18, 12)
+// and after every second one, where a skipping world's byte ticks are cheap: 320^3 rain
+// 12 / 15, 512^3 30 / 32.  A word of a row under 24 cells is mostly padding, which the hash
+// walks too: 16 x 1024 x 1024, hash after every tick / sixth tick / none, 26, 12, 8 on
+// bytes, 67, 17, 8 on planes.
+constexpr uint64_t kHashedBytesMin = 3ull << 22, kHashedBytesMax = 1ull << 27, kNarrowMin = 1ull << 21;
+constexpr int kNarrowRow = 24;
+
+struct PlaneRun {
+  uint64_t n;  // voxels
+  int nx;
+  bool skip, items;
+  int nticks, hash_every;
+};
+inline bool planes_suit(const PlaneState &st, const PlaneRun &r) {
+  const int64_t hashes = r.hash_every > 0 ? r.nticks / r.hash_every : 0;
+  if (r.nticks < kPlaneMinTicks) return r.items && st.ready(true) && (hashes || st.shorts < kPlaneShortRuns);
+  if (r.nx < kNarrowRow && r.n > kNarrowMin && 6 * hashes >= r.nticks) return false;
+  const bool often = r.skip ? 2 * hashes >= r.nticks : 2 * hashes > r.nticks;
+  return !(often && r.n > kHashedBytesMin && r.n <= kHashedBytesMax);
 }
 
 // A pass: one tick, or the ticks t (odd) and t + 1.

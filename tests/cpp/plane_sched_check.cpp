@@ -227,7 +227,7 @@ struct Model {
   // a world's calls
   int run(int n, int every) {
     const std::vector<u8> before = bytes;
-    if (any_path ? st.ready(items) || n >= kPlaneMinTicks : planes_suit(st, items, n, every)) {
+    if (any_path ? st.ready(items) || n >= kPlaneMinTicks : planes_suit(st, {bytes.size(), nx, items, items, n, every})) {
       if (st.tiled != items) {
         st.tiled = items;
         st.valid = false;
@@ -339,21 +339,38 @@ static int rest() {
 
 // Which runs take the planes.
 static int paths() {
+  auto suits = [](const PlaneState &st, u64 n, int nx, bool skip, int ticks, int every) {
+    return planes_suit(st, {n, nx, skip, skip && n > 1ull << 28, ticks, every});
+  };
+  const u64 big = 1ull << 29, mid = 1ull << 26;
   PlaneState dense, items;
-  for (int n : {1, 2}) {
-    CHECK(!planes_suit(dense, false, n, 0) && !planes_suit(items, true, n, 0));
-    dense.valid = true;  // in planes, which are as good as bytes for them
-    CHECK(!planes_suit(dense, false, n, 0) && !planes_suit(dense, false, n, 1));
-    dense.valid = false;
-  }
-  CHECK(planes_suit(dense, false, 3, 0) && planes_suit(items, true, 3, 0));
+  for (bool skip : {false, true})
+    for (int n : {1, 2}) {
+      CHECK(!suits(dense, mid, 500, skip, n, 0) && !suits(items, big, 500, true, n, 0));
+      dense.valid = true;  // in planes, which are no better for them
+      CHECK(!suits(dense, mid, 500, skip, n, 0) && !suits(dense, 4000, 500, skip, n, 1));
+      dense.valid = false;
+    }
+  CHECK(suits(dense, mid, 500, true, 3, 0) && suits(items, big, 500, true, 3, 0));
   Counters ops;
   items.tiled = true;
   CHECK(plane_passes(&items, true, 0, 4, 0, ops) == 0);
   int k = 0;  // single ticks on planes before they go to bytes
-  for (; k < 1000 && planes_suit(items, true, 1, 0); k++) CHECK(plane_passes(&items, true, (u64)k, 1, 0, ops) == 0);
-  CHECK(k == kPlaneShortRuns && planes_suit(items, true, 1, 1) && planes_suit(items, true, 3, 0));
-  CHECK(plane_passes(&items, true, (u64)k, 3, 0, ops) == 0 && planes_suit(items, true, 1, 0));
+  for (; k < 1000 && suits(items, big, 500, true, 1, 0); k++) CHECK(plane_passes(&items, true, (u64)k, 1, 0, ops) == 0);
+  CHECK(k == kPlaneShortRuns && suits(items, big, 500, true, 1, 1) && suits(items, big, 500, true, 3, 0));
+  CHECK(plane_passes(&items, true, (u64)k, 3, 0, ops) == 0 && suits(items, big, 500, true, 1, 0));
+  // hashed often: on bytes where those run in the last-level cache
+  for (bool skip : {false, true}) {
+    CHECK(!suits(dense, mid, 500, skip, 30, 1) && !suits(dense, 1ull << 27, 500, skip, 30, 1));
+    CHECK(!suits(dense, (3ull << 22) + 1, 500, skip, 30, 1) && suits(dense, 3ull << 22, 500, skip, 30, 1));
+    CHECK(suits(dense, (1ull << 27) + 1, 500, skip, 30, 1));
+    CHECK(suits(dense, mid, 500, skip, 30, 2) == !skip && suits(dense, mid, 500, skip, 30, 3));
+    CHECK(suits(dense, mid, 500, skip, 30, 30));
+    // rows that are mostly padding
+    CHECK(!suits(dense, 1ull << 22, 16, skip, 30, 6) && !suits(dense, big, 23, skip, 30, 1));
+    CHECK(suits(dense, 1ull << 21, 16, skip, 30, 6) && suits(dense, 1ull << 22, 16, skip, 30, 7));
+    CHECK(suits(dense, 1ull << 22, 24, skip, 30, 1) && suits(dense, 1ull << 22, 16, skip, 30, 0));
+  }
   return 0;
 }
 
