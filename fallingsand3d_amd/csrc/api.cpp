@@ -276,13 +276,14 @@ PlaneShape shape_of(const fs3d_world *w) { return plane_shape(w->nx, w->ny, w->n
 // quarter of the bytes and without table lookups, unpacked once.  The byte
 // kernels keep what asks for them (an explicit segment or schedule, sweep
 // counters, fusion switched off), what planes do not suit (planes_suit), rows under 16 cells (a
-// row takes whole 16-byte words, so planes would outgrow the bytes) and plane grids
-// of 4 GiB and more (buffer addressing).
+// row takes whole 16-byte words, so planes would outgrow the bytes), plane grids of
+// 4 GiB and more (buffer addressing) and layers beyond number (a tick's launch).
 bool plane_path(const fs3d_world *w, int nticks, int hash_every) {
   if (w->planes_off || w->seg_req != 0 || w->d_stats || nticks < 1) return false;
   if (w->skip != FS3D_SKIP_OFF && w->skip != FS3D_SKIP_AUTO) return false;
   if (!w->skip && w->fuse_set && !w->fuse) return false;
-  if (w->nx < 16 || plane_words(shape_of(w)) > kMaxPlaneWords) return false;
+  const PlaneShape ps = shape_of(w);
+  if (w->nx < 16 || plane_words(ps) > kMaxPlaneWords || plane_tick_blocks(ps) > kMaxTickBlocks) return false;
   return planes_suit(w->plane, {w->n, w->nx, w->skip != FS3D_SKIP_OFF, item_ticks(w), nticks, hash_every});
 }
 

@@ -29,6 +29,16 @@ inline size_t plane_words(const PlaneShape &p) {
   return (size_t)p.lr * ((size_t)(p.ny + 1) * (size_t)(p.nz + 2) + 1);
 }
 
+// Workgroups of a single tick (one at least for every two layers, however thin they are).
+// A launch takes fewer than 2^32 threads; half of that is the tick's, the rest room for
+// the hash in the same launch.
+inline u64 plane_tick_rows(const PlaneShape &p) {  // workgroups along y
+  const u64 per = 4 * (64 / (u64)p.lr), nyq = ((u64)p.ny + 2) >> 1;
+  return (nyq + per - 1) / per;
+}
+inline u64 plane_tick_blocks(const PlaneShape &p) { return plane_tick_rows(p) * (((u64)p.nz + 2) >> 1); }
+constexpr u64 kMaxTickBlocks = 1ull << 23;
+
 struct PlaneArgs {
   const plane_u32x4 *src;
   plane_u32x4 *dst;

@@ -721,15 +721,14 @@ hipError_t launch_plane_tick(const PlaneShape &ps, const void *src, void *dst, u
   a.t = t;
   a.tick_dev = tick_dev;
   a.k_off = k_off;
-  const int nyq = (ps.ny + 2) >> 1, nzq = (ps.nz + 2) >> 1, per = 4 * a.upw;
-  const u32 tx = (u32)((nyq + per - 1) / per);
+  const u32 tx = (u32)plane_tick_rows(ps);
   HashArgs h{};
   u32 hb = 0;
   if (hash) {
     h = hash_args(ps, *hash, src);
     hb = h.gx * h.gy;
   }
-  const dim3 grid(hb + tx * (u32)nzq);
+  const dim3 grid(hb + (u32)plane_tick_blocks(ps));
   if (ps.nx % 64 == 0)
     hipLaunchKernelGGL(plane_tick_kernel<true>, grid, dim3(256), 0, s, a, h, hb, tx);
   else
