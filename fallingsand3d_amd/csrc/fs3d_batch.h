@@ -79,6 +79,7 @@ struct FillEntry {
   u64 seed, thr;
   unsigned first;  // first workgroup of the entry
 };
+constexpr unsigned kMaxFillBlocks = (1u << 24) - 1u;  // of a launch, which takes fewer than 2^32 threads
 hipError_t launch_wide_fill(const FillEntry *ents, int n, unsigned blocks, u64 *hashes, u32 *chg, hipStream_t s);
 hipError_t launch_gather_hashes(const u64 *hashes, const int *slots, int n, u64 *out, hipStream_t s);
 hipError_t launch_expand(const long long *bpre, int n, int *blk2ent, hipStream_t s);

@@ -266,7 +266,7 @@ int admit(fs3d_server *s) {
     if (s->free_slots.empty()) break;
     const size_t fill_blocks =
         planes_fit(r) ? ((size_t)((r.nx + 63) / 64) * (size_t)r.ny * (size_t)r.nz + 255) / 256 : 0;
-    if (blocks + fill_blocks > 0x7FFFFFFFu) break;  // the next pass admits
+    if (blocks + fill_blocks > kMaxFillBlocks) break;  // the next pass admits
     u8 *g = nullptr;
     const GridArena::Result res = s->arena.alloc(need, &g);
     if (res != GridArena::kOk) {

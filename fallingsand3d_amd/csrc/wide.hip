@@ -126,12 +126,14 @@ __global__ __launch_bounds__(256) void wide_plane_kernel(const BWorld *__restric
 // 1500 requests, 37.2 with this: 24 us a round).  A workgroup adds to the entry's hash
 // once: an addition to one word takes it 13 ns.
 constexpr u32 kHashThreads = 1024, kHashWords = 2 * kHashThreads / 4;  // words of a workgroup
-__global__ __launch_bounds__(1024) void wide_hash_kernel(const HashEntry *__restrict__ ents, int n, u64 *hashes) {
+__global__ __launch_bounds__(1024) void wide_hash_kernel(const HashEntry *__restrict__ ents, int n, unsigned block0,
+                                                         u64 *hashes) {
   using namespace planedev;
+  const unsigned block = block0 + blockIdx.x;
   int lo = 0, hi = n;  // first of entry lo <= block < first of entry hi
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
-    if (ents[mid].first <= blockIdx.x) lo = mid; else hi = mid;
+    if (ents[mid].first <= block) lo = mid; else hi = mid;
   }
   const HashEntry f = ents[__builtin_amdgcn_readfirstlane(lo)];
   const u32 lr = (u32)((f.nx + 63) >> 6), words = lr * (u32)f.ny * (u32)f.nz;
@@ -139,7 +141,7 @@ __global__ __launch_bounds__(1024) void wide_hash_kernel(const HashEntry *__rest
   u64 acc = 0;
 #pragma unroll
   for (u32 k = 0; k < 2; k++) {
-    const u32 i = (blockIdx.x - f.first) * kHashWords + k * (kHashThreads / 4) + (threadIdx.x >> 2);
+    const u32 i = (block - f.first) * kHashWords + k * (kHashThreads / 4) + (threadIdx.x >> 2);
     if (i < words) {
       const u32 row = i / lr, c = 4u * (i - row * lr) + (threadIdx.x & 3u);
       const u64 i0 = (u64)row * (u64)f.nx + (u64)(16u * c);
@@ -270,8 +272,13 @@ unsigned hash_blocks(size_t words) { return (unsigned)((words + kHashWords - 1) 
 
 hipError_t launch_wide_hash(const HashEntry *ents, int n, unsigned blocks, u64 *hashes, hipStream_t s) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(wide_hash_kernel, dim3(blocks), dim3(kHashThreads), 0, s, ents, n, hashes);
-  return hipGetLastError();
+  constexpr unsigned kMax = (1u << 22) - 1u;  // a launch takes fewer than 2^32 threads
+  for (unsigned b = 0; b < blocks; b += kMax) {
+    hipLaunchKernelGGL(wide_hash_kernel, dim3(blocks - b < kMax ? blocks - b : kMax), dim3(kHashThreads), 0, s, ents, n,
+                       b, hashes);
+    if (const hipError_t e = hipGetLastError()) return e;
+  }
+  return hipSuccess;
 }
 
 hipError_t launch_wide_fill(const FillEntry *ents, int n, unsigned blocks, u64 *hashes, u32 *chg, hipStream_t s) {
