@@ -15,7 +15,8 @@
 // does not fit waits at the head of the queue until finished grids come back.
 //
 // Latency accounting: every launch is bracketed by HIP events, so each launch
-// duration is one tick-latency sample for the worlds in it; request latency is
+// duration is one tick-latency sample for the worlds in it (a round's last one ends
+// with the hashes of the requests that finish in it); request latency is
 // host time from submission to the poll that observes its final round done.
 //
 // The reference has no serving of any kind (one interactive window,
@@ -397,11 +398,12 @@ int launch_round(fs3d_server *s) {
     FS3D_HIP(launch_wide_planes(d_ents, pk, rd.d_blk + boff, 0, bp, k, s->s_tick, s->d_chg));
     FS3D_HIP(launch_wide(s->seg, d_ents, pk, rd.d_blk + boff, bp, tot[k] - bp, k, rule, s->d_hashes, s->s_tick,
                          s->d_chg));
-    FS3D_HIP(hipEventRecord(rd.ev[k + 1], s->s_tick));
+    if (k + 1 < K) FS3D_HIP(hipEventRecord(rd.ev[k + 1], s->s_tick));
     boff += (size_t)tot[k];
   }
   FS3D_HIP(launch_wide_hash((const HashEntry *)(rd.d_buf + ent_bytes + pre_bytes + koff_bytes), n_hash, hash_blk,
                             s->d_hashes, s->s_tick));
+  FS3D_HIP(hipEventRecord(rd.ev[K], s->s_tick));  // the finished requests' hash is part of the last tick
   FS3D_HIP(launch_gather_hashes(s->d_hashes, (const int *)(rd.d_buf + ent_bytes + pre_bytes + koff_bytes + hash_bytes),
                                 (int)fin.size(), rd.h_hash, s->s_tick));
   FS3D_HIP(hipEventRecord(rd.done, s->s_tick));
