@@ -599,7 +599,6 @@ int fs3d_world_create(const int32_t dims[3], uint32_t flags, fs3d_world **out) {
   int rc = ensure_device(dev);
   if (rc) return rc;
   fs3d_world *w = new fs3d_world();
-  hostcopy_world(1);
   w->dev = dev;
   w->nx = dims[0];
   w->ny = dims[1];
@@ -614,6 +613,7 @@ int fs3d_world_create(const int32_t dims[3], uint32_t flags, fs3d_world **out) {
     delete w;
     return rc;
   }
+  hostcopy_world(1);  // (release takes it back)
   hipError_t e = hipStreamCreateWithFlags(&w->stream, hipStreamNonBlocking);
   for (int i = 0; i < 2 && e == hipSuccess; i++) e = hipMalloc(&w->buf[i], w->alloc);
   for (int i = 0; i < 2 && e == hipSuccess; i++) e = hipMalloc(&w->d_masks[i], 2 * w->mask_words * sizeof(u64));

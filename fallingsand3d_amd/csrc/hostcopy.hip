@@ -4,7 +4,8 @@
 // buffer: 18 GB/s into pages that exist and 11 GB/s into fresh ones, which that
 // thread also has to fault in, where the link carries 56 GB/s.  Here a kernel writes
 // the bytes to pinned slots, a launch to as many as are free, and up to four threads
-// copy out of the slots, so that the link, the copying and the page faults overlap.
+// copy out of the slots (copy_job.h), so that the link, the copying and the page faults
+// overlap.
 // A piece reports itself by a flag in pinned memory: a copy command per piece takes
 // 10 us more than its bytes, an event 5.  Only the calling thread talks to the
 // runtime, whose first call in a new thread costs 100 us and more.
@@ -13,19 +14,18 @@
 #include "hostcopy.h"
 
 #include <algorithm>
-#include <atomic>
 #include <cstring>
 #include <memory>
 #include <mutex>
-#include <thread>
+
+#include "copy_job.h"
 
 namespace fs3d {
 namespace {
 
 typedef u32 u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kHelpers = 3;  // (11 were no faster)
-constexpr size_t kSlots = 12;
+constexpr size_t kSlots = kCopySlots;
 constexpr size_t kSlotBytes = 1u << 20;
 constexpr size_t kAloneMax = 512u << 10;  // up to here the calling thread copies alone
 constexpr size_t kDirectMax = 64u << 10;  // below, the runtime's copy is as fast
@@ -107,128 +107,48 @@ void give_back(Staging *g) {
   destroy(g);
 }
 
-struct Piece {
-  u8 *host;
-  size_t off, n;  // in its span
-  size_t span;
-};
 // Launches the kernel for bytes [off, off + out.n) of a span.
 typedef std::function<hipError_t(size_t span, size_t off, const PieceOut &out, hipStream_t)> Issue;
 
-// Piece c goes through slot c % slots; the slot's flag becomes c + 1.  Helpers share the
-// job: a thread that gets to run only after the copy is over finds nothing to claim and
-// touches nothing else, so that nobody has to wait for it.  (Joined, threads that were
-// not scheduled for a while made a copy of 0.3 ms take 4.)
-struct Job {
-  std::vector<Piece> pieces;
-  const Staging *g;
-  size_t piece, slots;                    // bytes of a slot, slots in use
-  std::atomic<size_t> taken{0};           // pieces claimed
-  std::atomic<size_t> copied{0};          // pieces copied out
-  std::atomic<int> busy{0};               // helpers between a claim and its end
-  std::atomic<size_t> done[kSlots] = {};  // of a slot: the last piece copied out of it, plus 1
-  std::atomic<bool> stop{false};
+CopyHelpers g_helpers;
+
+// The launches of a copy through g's slots.
+struct Slots {
+  Staging *g;
+  size_t piece;
+  hipStream_t s;
+  const Issue &make;
+  int issue(const CopyPiece &p, size_t slot, size_t bytes, u32 value) const {
+    return make(p.span, p.off,
+                PieceOut{g->slots() + slot * piece, (u32)bytes, (u32)piece, g->counters + slot, g->flag(slot), value},
+                s);
+  }
+  int wait() const { return hipStreamSynchronize(s); }
+  int lost() const { return hipErrorUnknown; }
 };
 
-bool arrived(const Job *j, size_t c) {
-  return __atomic_load_n(j->g->flag(c % j->slots), __ATOMIC_ACQUIRE) == (u32)c + 1u;
-}
-
-void copy_out(Job *j, size_t c) {
-  const Piece &p = j->pieces[c];
-  std::memcpy(p.host, j->g->slots() + (c % j->slots) * j->piece, p.n);
-  j->done[c % j->slots].store(c + 1, std::memory_order_release);
-  j->copied.fetch_add(1);
-}
-
-void help(std::shared_ptr<Job> job) {
-  Job *j = job.get();
-  for (;;) {
-    j->busy.fetch_add(1);
-    const size_t c = j->stop.load() ? j->pieces.size() : j->taken.fetch_add(1);
-    bool mine = c < j->pieces.size();
-    while (mine && !arrived(j, c)) {
-      if (j->stop.load()) mine = false;
-      std::this_thread::yield();
-    }
-    if (mine) copy_out(j, c);
-    j->busy.fetch_sub(1);
-    if (!mine) return;
-  }
-}
-
 // Runs the pieces through g; the stream is idle when it returns.
-hipError_t run(Staging *g, std::vector<Piece> all, size_t piece, size_t total, hipStream_t s, const Issue &issue) {
-  const std::shared_ptr<Job> job = std::make_shared<Job>();
-  Job &j = *job;
-  j.pieces = std::move(all);
-  const std::vector<Piece> &pieces = j.pieces;
-  j.g = g;
-  j.piece = piece;
-  const size_t slots = j.slots = std::min(kSlots, g->bytes / piece);
+hipError_t run(Staging *g, std::vector<CopyPiece> pieces, size_t piece, size_t total, hipStream_t s,
+               const Issue &issue) {
+  const std::shared_ptr<CopyJob> job = std::make_shared<CopyJob>();
+  job->pieces = std::move(pieces);
+  job->mem = g->slots();
+  job->flags = g->flag(0);
+  job->flag_stride = kFlagStride;
+  job->piece = piece;
+  job->slots = std::min(kSlots, g->bytes / piece);
   for (size_t k = 0; k < kSlots; k++) *g->flag(k) = 0;
-  const size_t n = pieces.size();
-  hipError_t e = g->cleared ? hipSuccess : launch_fill_u32(g->counters, kSlots, 0, s);
-  g->cleared = g->cleared || e == hipSuccess;
-  size_t issued = 0;
-  // Launches what follows in free neighbouring slots (once a few are free).
-  auto issue_free = [&] {
-    while (issued < n && e == hipSuccess) {
-      const Piece &p = pieces[issued];
-      size_t m = 0, bytes = 0;
-      while (issued + m < n && pieces[issued + m].span == p.span && issued % slots + m < slots &&
-             (issued + m < slots || j.done[issued % slots + m].load(std::memory_order_acquire) ==
-                                         issued + m - slots + 1)) {
-        bytes += pieces[issued + m].n;
-        m++;
-      }
-      const bool all = issued + m == n || issued % slots + m == slots || pieces[issued + m].span != p.span;
-      if (m == 0 || (m < slots / 4 && !all)) return;
-      const size_t k = issued % slots;
-      e = issue(p.span, p.off,
-                PieceOut{g->slots() + k * piece, (u32)bytes, (u32)piece, g->counters + k, g->flag(k), (u32)issued + 1u}, s);
-      issued += m;
-    }
-  };
-  issue_free();
-  if (total > kAloneMax)
-    for (int i = 0; i < (int)std::min<size_t>(kHelpers, n - 1); i++) {
-      try {
-        std::thread(help, job).detach();
-      } catch (...) {
-        break;  // fewer threads do the same work
-      }
-    }
-  // The calling thread issues the pieces and copies too.  What it waits for ends with
-  // its kernel: a stream that has stopped without the flag is an error.
-  while (e == hipSuccess) {
-    const size_t c = j.taken.fetch_add(1);
-    if (c >= n && issued == n) break;
-    for (u32 spins = 1; e == hipSuccess; spins++) {
-      issue_free();
-      if (c >= n ? issued == n : c < issued && arrived(&j, c)) break;
-      if (spins % 4096 == 0) {
-        const hipError_t q = hipStreamQuery(s);
-        if (q == hipErrorNotReady)
-          (void)hipGetLastError();
-        else if (q != hipSuccess)
-          e = q;
-        else if (c < issued && !arrived(&j, c))
-          e = hipErrorUnknown;
-      }
-      std::this_thread::yield();
-    }
-    if (e == hipSuccess && c < n) copy_out(&j, c);
-  }
-  if (e != hipSuccess) j.stop.store(true);
-  while (e == hipSuccess ? j.copied.load() < n : j.busy.load() != 0) std::this_thread::yield();
-  const hipError_t last = hipStreamSynchronize(s);  // no slot is in use any more
-  return e != hipSuccess ? e : last;
+  if (!g->cleared)
+    if (const hipError_t e = launch_fill_u32(g->counters, kSlots, 0, s)) return e;
+  const int helpers = total > kAloneMax ? (int)std::min<size_t>(CopyHelpers::kMost, job->pieces.size() - 1) : 0;
+  const hipError_t e = (hipError_t)copy_run(job, &g_helpers, helpers, Slots{g, piece, s, issue});
+  g->cleared = e == hipSuccess;  // (a launch that failed may have left counts)
+  return e;
 }
 
-void split(std::vector<Piece> *pieces, void *host, size_t n, size_t span, size_t piece) {
+void split(std::vector<CopyPiece> *pieces, void *host, size_t n, size_t span, size_t piece) {
   for (size_t off = 0; off < n; off += piece)
-    pieces->push_back(Piece{(u8 *)host + off, off, std::min(piece, n - off), span});
+    pieces->push_back(CopyPiece{(u8 *)host + off, off, std::min(piece, n - off), span});
 }
 
 // The first piece of a small copy is there soon, and no helper is left without one.
@@ -263,7 +183,7 @@ hipError_t copy_to_host(const std::vector<HostSpan> &spans, int dev, hipStream_t
   }
   hipError_t e = hipErrorOutOfMemory;
   try {
-    std::vector<Piece> pieces;
+    std::vector<CopyPiece> pieces;
     for (size_t i = 0; i < spans.size(); i++) split(&pieces, spans[i].host, spans[i].n, i, piece_of(total));
     e = run(g, pieces, piece_of(total), total, s, [&](size_t i, size_t off, const PieceOut &out, hipStream_t st) {
       hipLaunchKernelGGL(piece_kernel, dim3(piece_blocks(out)), dim3(256), 0, st, (const u8 *)spans[i].dev + off, out);
@@ -284,7 +204,7 @@ hipError_t make_on_host(void *host, size_t n, int dev,
   try {
     std::vector<u8> between;  // the threads write ordinary memory only
     if (!pageable(host)) between.resize(n);
-    std::vector<Piece> pieces;
+    std::vector<CopyPiece> pieces;
     split(&pieces, between.empty() ? host : between.data(), n, 0, piece_of(n));
     e = g->stream ? hipSuccess : hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking);
     if (e == hipSuccess)
