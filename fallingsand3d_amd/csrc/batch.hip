@@ -63,6 +63,11 @@ __device__ __forceinline__ BWorld world_at(const BWorld *worlds, int wi) {
   return w;
 }
 
+// Orders a wave's accesses for its own lanes, which pass planes to each other through LDS
+// from packing to the ticks and to unpacking: no instruction, since the LDS answers a wave
+// in order, but the compiler keeps to it.
+__device__ __forceinline__ void wave_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
+
 struct Geo {
   int nx, ny, nz, lr, upw;
   int ul, seg, prev, next;  // the lane's row quad of a group, word, ring neighbours
@@ -237,11 +242,13 @@ __global__ __launch_bounds__(NT, 4) void batch_kernel(BWorld *worlds, const int 
     const Geo g = geo_of(w, lane);
     u8 *const bytes = grid_of(w);
     const bool keep = __any(batch_pack(mem, bytes, g, words, lane, 64));
+    wave_fence();
     int quiet = 0;
     for (int k = 0; k < nticks; k++) {
       if (settle && quiet >= 2) break;
       const u32 t = (u32)(w.tick + (u64)k);
       const bool ch = (t & 1u) ? batch_tick<1>(mem, g, t, 0, 1) : batch_tick<0>(mem, g, t, 0, 1);
+      wave_fence();
       quiet = __any(ch) ? 0 : quiet + 1;
     }
     const u64 acc = wave_sum_u64(batch_unpack(mem, bytes, g, words, lane, 64, keep, want_hash));
