@@ -19,6 +19,7 @@ struct fs3d_batch {
   int n = 0;
   std::vector<int> nx, ny, nz;
   std::vector<size_t> off, cells;
+  size_t total_cells = 0;
   std::vector<TickShape> plain_shape;  // single-world launch shape per world (plain loop)
   u8 *arena = nullptr;
   size_t arena_bytes = 0;  // of the grids
@@ -209,6 +210,17 @@ int run_wide(fs3d_batch *b, int nticks, int want_hash) {
   return FS3D_OK;
 }
 
+// Whether a persistent run takes the wide kernel instead: without plane scratch, and for
+// one or two ticks, which packing and unpacking every world cost more than they gain
+// (us of a run of one tick, persistent on planes / wide / persistent on bytes, as it was:
+// 4096 worlds of 16-128 cells a side 1202 / 854 / 911; 256 of them 653 / 114 / 380; 300 of
+// 8 x 128 x 128 431 / 135 / 145; 24 of 8-16 cells a side 68 / 74 / 57; of two ticks 621 /
+// 680 / 1652, 687 / 153 / 594, 458 / 191 / 232, 64 / 76 / 58).
+bool goes_wide(const fs3d_batch *b, int nticks) {
+  constexpr size_t kMinCells = 1u << 17;
+  return b->planes_off || (nticks <= 2 && b->total_cells > kMinCells);
+}
+
 int run_plain(fs3d_batch *b, int nticks, int want_hash) {
   const u64 *rule = device_rule_table(b->dev);
   FS3D_HIP(hipEventRecord(b->ev0, b->stream));
@@ -248,6 +260,7 @@ int fs3d_batch_create(int32_t n, const int32_t *dims, fs3d_batch **out) {
     b->nz.push_back(z);
     const size_t c = (size_t)x * y * z;
     b->cells.push_back(c);
+    b->total_cells += c;
     b->off.push_back(total);
     total += (c + kGuardBytes + 255) & ~(size_t)255;
     TickShape sh;
@@ -429,7 +442,7 @@ int fs3d_batch_run(fs3d_batch *b, int32_t nticks, int32_t mode, uint64_t *hashes
     b->last_ms = 0.0;
     return clear_error();
   }
-  if (mode == FS3D_BATCH_PERSISTENT && b->planes_off) mode = FS3D_BATCH_WIDE;
+  if (mode == FS3D_BATCH_PERSISTENT && goes_wide(b, nticks)) mode = FS3D_BATCH_WIDE;
   int rc = mode == FS3D_BATCH_PERSISTENT ? run_persistent(b, nticks, want_hash)
            : mode == FS3D_BATCH_WIDE     ? run_wide(b, nticks, want_hash)
                                          : run_plain(b, nticks, want_hash);

@@ -184,7 +184,9 @@ int fs3d_threshold(uint64_t num, uint64_t den, uint64_t *thr);
  * counterpart: the reference runs one scene in one process (src/main.cpp:6-16).
  * FS3D_BATCH_PERSISTENT steps every world for nticks ticks in one persistent
  * kernel launch (captured in a HIP graph): workgroups pull worlds from an atomic
- * queue, largest first, and run all ticks of a world in place.
+ * queue, largest first, and run all ticks of a world in place.  (Runs of one or
+ * two ticks, but for a handful of small worlds, take FS3D_BATCH_WIDE's kernel,
+ * which is faster for them.)
  * FS3D_BATCH_PLAIN launches the single-world tick kernel once per world per
  * tick (the baseline).  Both give bit-identical grids.  Worlds share the tick
  * counter; nx <= 2048. */
