@@ -111,8 +111,7 @@ void release(fs3d_world *w) {
   w->graphs.clear();
   for (int i = 0; i < 2; i++)
     if (w->buf[i]) (void)hipFree(w->buf[i]);
-  for (int i = 0; i < 2; i++)
-    if (w->planes[i]) (void)hipFree(w->planes[i]);
+  if (w->plane_mem) (void)hipFree(w->plane_mem);
   if (w->d_reserved) (void)hipFree(w->d_reserved);
   for (u64 *f : w->pflags)
     if (f) (void)hipFree(f);
@@ -287,23 +286,43 @@ bool plane_path(const fs3d_world *w, int nticks, int hash_every) {
   return planes_suit(w->plane, {w->n, w->nx, w->skip != FS3D_SKIP_OFF, item_ticks(w), nticks, hash_every});
 }
 
+// Bytes of a plane buffer, where the two of them are (an index of `padded`) and one's
+// address.  In the byte buffer that is not current they cost a world no memory: its
+// bytes count only for ticks on bytes, which find every change bit set after planes.
+size_t plane_bytes(const PlaneShape &ps) {
+  const size_t b = plane_words(ps) * 16, align = b < ((size_t)32 << 20) ? 256 : (size_t)2 << 20;
+  return (b + align - 1) / align * align;
+}
+int plane_region(const fs3d_world *w, const PlaneShape &ps) {
+  return 2 * plane_bytes(ps) <= w->n ? w->cur ^ 1 : 2;
+}
+void *plane_buf(const fs3d_world *w, const PlaneShape &ps, int i) {
+  const int r = plane_region(w, ps);
+  return (r < 2 ? w->buf[r] : static_cast<u8 *>(w->plane_mem)) + (size_t)i * plane_bytes(ps);
+}
+
 // Plane buffers (and the item lists) on first use; false (and the byte kernels from
 // then on) when the device has no room for them.
 bool ensure_planes(fs3d_world *w) {
   const PlaneShape ps = shape_of(w);
   hipError_t e = hipSuccess;
-  const bool created = !w->planes[0];
-  if (created) {
-    e = hipMalloc((void **)&w->d_reserved, sizeof(u32));
+  if (!w->d_reserved) e = hipMalloc((void **)&w->d_reserved, sizeof(u32));
+  const int r = plane_region(w, ps);
+  if (r == 2 && !w->plane_mem && e == hipSuccess) {
     // room for either layout: the schedule may change
-    const size_t most = std::max(plane_words(plane_shape(w->nx, w->ny, w->nz)),
-                                 may_list(w) ? plane_words(plane_shape(w->nx, w->ny, w->nz, true)) : 0);
-    for (int i = 0; i < 2 && e == hipSuccess; i++) e = hipMalloc(&w->planes[i], most * 16);
+    const size_t most = std::max(plane_bytes(plane_shape(w->nx, w->ny, w->nz)),
+                                 may_list(w) ? plane_bytes(plane_shape(w->nx, w->ny, w->nz, true)) : 0);
+    e = hipMalloc(&w->plane_mem, 2 * most);
   }
-  if (created || w->plane.tiled != ps.tiled) {
+  if (w->plane.tiled != ps.tiled) {
     w->plane.tiled = ps.tiled;
     w->plane.valid = false;
-    for (int i = 0; i < 2 && e == hipSuccess; i++) e = launch_plane_pad(ps, w->planes[i], w->stream);
+  }
+  if (w->padded[r] != (signed char)ps.tiled && e == hipSuccess) {
+    for (int i = 0; i < 2 && e == hipSuccess; i++) e = launch_plane_pad(ps, plane_buf(w, ps, i), w->stream);
+    w->padded[r] = (signed char)ps.tiled;
+    w->plane.valid = false;
+    w->masks_stale = true;  // the byte buffer that is not current has been written to
   }
   if (item_ticks(w) && !w->d_items && e == hipSuccess) {
     const PlaneCells c = plane_cells(ps);
@@ -320,13 +339,10 @@ bool ensure_planes(fs3d_world *w) {
   if (e == hipSuccess) return true;
   (void)hipGetLastError();
   auto drop = [](auto *&p) {
-    if (p) (void)hipFree(p);
+    if (p) (void)hipFree((void *)p);
     p = nullptr;
   };
-  for (int i = 0; i < 2; i++) {
-    if (w->planes[i]) (void)hipFree(w->planes[i]);
-    w->planes[i] = nullptr;
-  }
+  drop(w->plane_mem);
   for (u64 *&f : w->pflags) drop(f);
   drop(w->d_reserved);
   drop(w->d_since);
@@ -343,6 +359,7 @@ struct PlaneLaunch {
   PlaneShape ps;
   const u64 *tick_dev;
 
+  void *at(int i) const { return plane_buf(w, ps, i); }
   PlaneHash hash_to(int i) const { return PlaneHash{w->buf[w->cur], w->d_reserved, w->d_parts, w->d_small + i}; }
   int finalize(int i) const {
     if (!plane_hash_direct(ps)) FS3D_HIP(launch_hash_finalize(w->d_parts, w->d_small + i, w->stream));
@@ -354,12 +371,12 @@ struct PlaneLaunch {
     return FS3D_OK;
   }
   int pack(int src) const {
-    FS3D_HIP(launch_plane_pack(ps, w->buf[w->cur], w->planes[src], w->d_reserved, w->stream));
+    FS3D_HIP(launch_plane_pack(ps, w->buf[w->cur], at(src), w->d_reserved, w->stream));
     return FS3D_OK;
   }
   int pack_tick(int src, int f) const {
-    FS3D_HIP(launch_plane_pack_even(ps, w->buf[w->cur], w->planes[src], w->d_reserved, w->tick, tick_dev, 0,
-                                    f < 0 ? nullptr : w->pflags[f], w->planes[src ^ 1], w->stream));
+    FS3D_HIP(launch_plane_pack_even(ps, w->buf[w->cur], at(src), w->d_reserved, w->tick, tick_dev, 0,
+                                    f < 0 ? nullptr : w->pflags[f], at(src ^ 1), w->stream));
     return FS3D_OK;
   }
   int all_flags(int f) const {
@@ -371,22 +388,22 @@ struct PlaneLaunch {
     return FS3D_OK;
   }
   int hash(int src, int i) const {
-    FS3D_HIP(launch_plane_hash(ps, w->planes[src], hash_to(i), w->stream));
+    FS3D_HIP(launch_plane_hash(ps, at(src), hash_to(i), w->stream));
     return finalize(i);
   }
   int pass(const PlanePass &p) const {
     const u64 t = w->tick + (u64)p.k;
     const PlaneHash h = hash_to(p.hash);
     if (p.pair)
-      FS3D_HIP(launch_plane_pair(ps, w->planes[p.src], w->planes[p.src ^ 1], t, tick_dev, (u32)p.k, w->stream));
+      FS3D_HIP(launch_plane_pair(ps, at(p.src), at(p.src ^ 1), t, tick_dev, (u32)p.k, w->stream));
     else
-      FS3D_HIP(launch_plane_tick(ps, w->planes[p.src], w->planes[p.src ^ 1], t, tick_dev, (u32)p.k,
+      FS3D_HIP(launch_plane_tick(ps, at(p.src), at(p.src ^ 1), t, tick_dev, (u32)p.k,
                                  p.hash ? &h : nullptr, w->stream));
     return p.hash ? finalize(p.hash) : FS3D_OK;
   }
   int item_pass(const PlanePass &p) const {
     const int next = next_flags(p.flags), before = next_flags(next);
-    FS3D_HIP(launch_plane_list(ps, w->planes[p.src], w->planes[p.src ^ 1], w->tick + (u64)p.k, tick_dev, (u32)p.k,
+    FS3D_HIP(launch_plane_list(ps, at(p.src), at(p.src ^ 1), w->tick + (u64)p.k, tick_dev, (u32)p.k,
                                p.pair, p.first, w->pflags[p.flags], p.older,
                                p.older == kNoFlags ? nullptr : w->pflags[before], w->pflags[next], w->d_since,
                                w->d_items, w->d_nitems + p.flags, w->d_nitems + next, w->item_waves, w->stream));
@@ -394,10 +411,10 @@ struct PlaneLaunch {
   }
   int unpack(int src, int f) const {
     if (f >= 0)
-      FS3D_HIP(launch_plane_unpack_cells(ps, w->planes[src], w->buf[w->cur], w->pflags[f], w->d_since, w->d_reserved,
+      FS3D_HIP(launch_plane_unpack_cells(ps, at(src), w->buf[w->cur], w->pflags[f], w->d_since, w->d_reserved,
                                          w->occ_track ? w->d_dirty : nullptr, w->stream));
     else
-      FS3D_HIP(launch_plane_unpack(ps, w->planes[src], w->buf[w->cur], w->d_reserved, w->stream));
+      FS3D_HIP(launch_plane_unpack(ps, at(src), w->buf[w->cur], w->d_reserved, w->stream));
     return FS3D_OK;
   }
 };
@@ -477,6 +494,7 @@ int enqueue_ticks(fs3d_world *w, int nticks, int hash_every, const u64 *tick_dev
         FS3D_HIP(launch_tick2(w->shape2, w->buf[src], w->buf[src ^ 1], w->nx, w->ny, w->nz, w->tick + (u64)k,
                               tick_dev, (u32)k, rule, tick2_zlen(w), w->stream));
       src ^= 1;
+      w->padded[src] = -1;
       k += 2;
       continue;
     }
@@ -484,6 +502,7 @@ int enqueue_ticks(fs3d_world *w, int nticks, int hash_every, const u64 *tick_dev
     const bool chunked = !masks && dense_chunk_seg(w);
     const bool packed = masks && sched == FS3D_SKIP_SEGS && !hashed;
     const int dst = inplace && !chunked && !packed ? src : src ^ 1;
+    if (dst != src) w->padded[dst] = -1;
     if (launch) {
       if (masks && sched == FS3D_SKIP_LISTED && !hashed) {
         // settled row quads are listed out; hash ticks read every segment anyway
@@ -692,7 +711,7 @@ int fs3d_world_set_voxel(fs3d_world *w, int32_t x, int32_t y, int32_t z, uint8_t
   e.edge_off = w->mask_words;
   if (w->plane.valid) {
     const PlaneShape ps = plane_shape(w->nx, w->ny, w->nz, w->plane.tiled);
-    e.planes = static_cast<u32 *>(w->planes[w->plane.cur]);
+    e.planes = static_cast<u32 *>(plane_buf(w, ps, w->plane.cur));
     e.reserved = w->d_reserved;
     e.word = plane_word(ps, x, y, z);
     e.x = x;
@@ -1011,6 +1030,7 @@ int fs3d_world_load(fs3d_world *w, const char *path) {
                      dims[2], w->nx, w->ny, w->nz);
   FS3D_HIP(hipSetDevice(w->dev));
   w->plane.valid = false;
+  w->padded[w->cur ^ 1] = -1;
   // The payload goes to the idle buffer and becomes the world's state only once
   // its hash matches the stored one; on any failure the grid and tick stay as
   // they were.  Skipped segments rely on the destination buffer holding their

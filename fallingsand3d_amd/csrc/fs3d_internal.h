@@ -233,11 +233,15 @@ struct fs3d_world {
   fs3d::u32 *d_ctl = nullptr;         // list counts, one per tick mod 3
   fs3d::u32 list_waves = 0;           // persistent waves of the listed tick
   fs3d::u32 pack_waves = 0;           // persistent waves of the packed tick
-  // the grid as bit planes (two buffers, allocated on first use): planes[plane.cur]
-  // holds the current state while plane.valid; buf[cur] always does between calls
-  void *planes[2] = {nullptr, nullptr};
+  // the grid as two buffers of bit planes, of which plane.cur holds the current state
+  // while plane.valid; buf[cur] always does between calls.  They lie in the byte buffer
+  // that is not current, or in plane_mem (allocated on first use) where rows of few cells
+  // make them larger than that.
+  void *plane_mem = nullptr;
   fs3d::PlaneState plane;
   bool planes_off = false;
+  // layout whose rows around the grid are zero in buf[0], buf[1], plane_mem: 0 rows, 1 tiles
+  signed char padded[3] = {-1, -1, -1};
   fs3d::u32 *d_reserved = nullptr;  // a byte >= 4 has been packed or set
   // ticks of the active items only: change flags of the last passes (plane_sched.h),
   // items changed since the bytes were written, work list and

@@ -68,7 +68,7 @@ hipError_t launch_plane_tick(const PlaneShape &ps, const void *src, void *dst, u
 // Ticks t and t + 1, t odd.
 hipError_t launch_plane_pair(const PlaneShape &ps, const void *src, void *dst, u64 t, const u64 *tick_dev, u32 k_off,
                              hipStream_t s);
-// Zeroes the rows around the grid (once per buffer and layout: no kernel writes them).
+// Zeroes the rows around the grid (no kernel here writes them).
 hipError_t launch_plane_pad(const PlaneShape &ps, void *planes, hipStream_t s);
 // Bytes (values >= 4 as STATIC, *reserved set) to planes and back (with *reserved,
 // bytes >= 4 already in g stay).

@@ -603,7 +603,7 @@ __global__ __launch_bounds__(256) void plane_unpack_kernel(const u32x4 *in, u8 *
 }
 
 // The rows around the grid: the layers before the first and after the last, and the
-// row between every two layers.
+// row between every two layers; in tiles, the first and what is behind the last row.
 __global__ __launch_bounds__(256) void plane_pad_kernel(u32x4 *p, int ny, int nz, int lr) {
   const size_t end = (size_t)(ny + 1) * (u32)lr, mid = (size_t)nz * (u32)lr, n = 2 * end + mid + (u32)lr;
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
@@ -615,6 +615,24 @@ __global__ __launch_bounds__(256) void plane_pad_kernel(u32x4 *p, int ny, int nz
       w = (z + 1) * end + (k - z * (u32)lr);
     } else {
       w = (size_t)(nz + 1) * end + (i - end - mid);
+    }
+    p[w] = u32x4{0u, 0u, 0u, 0u};
+  }
+}
+
+__global__ __launch_bounds__(256) void plane_pad_tiles_kernel(u32x4 *p, int ny, int nz, int lr, int tiles) {
+  const u32 tile = 8u * (u32)lr, layer = tile * (u32)tiles, last = (u32)(ny + 8) / 8u;  // the tile of row ny
+  const u32 mid = tile * (1u + (u32)tiles - last);  // words of a layer of the grid that may be outside it
+  const u64 n = 2 * (u64)layer + (u64)mid * (u32)nz;
+  for (u64 i = (u64)blockIdx.x * 256 + threadIdx.x; i < n; i += (u64)gridDim.x * 256) {
+    u64 w = i;
+    if (i >= layer && i < layer + (u64)mid * (u32)nz) {
+      const u32 z = (u32)((i - layer) / mid), k = (u32)((i - layer) - (u64)z * mid);
+      const u32 t = k < tile ? 0u : last - 1u + k / tile;
+      if (t >= last && t * 8u + (k & 7u) < (u32)(ny + 8)) continue;  // (a tile's words: word, row)
+      w = (u64)(z + 1u) * layer + (u64)t * tile + k % tile;
+    } else if (i >= layer) {
+      w = (u64)(nz + 1) * layer + (i - layer - (u64)mid * (u32)nz);
     }
     p[w] = u32x4{0u, 0u, 0u, 0u};
   }
@@ -866,7 +884,11 @@ hipError_t launch_plane_unpack_cells(const PlaneShape &ps, const void *planes, u
 }
 
 hipError_t launch_plane_pad(const PlaneShape &ps, void *planes, hipStream_t s) {
-  if (ps.tiled) return launch_fill_u64(static_cast<u64 *>(planes), 2 * plane_words(ps), 0, s);
+  if (ps.tiled) {
+    hipLaunchKernelGGL(plane_pad_tiles_kernel, dim3(2048), dim3(256), 0, s, static_cast<u32x4 *>(planes), ps.ny, ps.nz,
+                       ps.lr, plane_tiles(ps));
+    return hipGetLastError();
+  }
   const size_t n = ((size_t)2 * (u32)(ps.ny + 1) + (u32)ps.nz + 1) * (u32)ps.lr;
   hipLaunchKernelGGL(plane_pad_kernel, dim3((unsigned)std::min<size_t>((n + 255) / 256, 4096)), dim3(256), 0, s,
                      static_cast<u32x4 *>(planes), ps.ny, ps.nz, ps.lr);
