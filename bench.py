@@ -19,8 +19,9 @@ Default run (one JSON line on stdout):
            child processes under rocprofv3 --pmc (FETCH_SIZE, then WRITE_SIZE),
            scaled by the counters of a copy of known size in the same process.
            "dense" holds dense ticks of the same world; "hbm2048" the dense byte
-           tick of the 2048^3 pillar scene, whose buffers (2 x 8 GiB) do not fit
-           the 256 MB Infinity Cache: the HBM-bound figure.
+           tick of the 2048^3 pillar scene (fuse off; the default there are pairs on
+           planes, extra.pillars2048.fused_pairs), whose buffers (2 x 8 GiB) do not
+           fit the 256 MB Infinity Cache: the HBM-bound figure.
   extra    pillars2048: the 2048^3 pillar scene, skipping, dense and dense fused
            in pairs; pillars2048_render: that scene with a 1920x1080 voxel render
            every 10 ticks; copy: a plain device copy of the same bytes, with
@@ -115,24 +116,40 @@ def timed_boxes_window(w, warmup, steps):
     return wall, dev / steps, hashes, ticks
 
 
+def run_passes(t, nt, he):
+    """Passes over the planes in a run of nt ticks from tick t: a pair of ticks from an
+    odd one on, single ticks elsewhere and before a hash that falls between the two.  A
+    run of one or two ticks stays on bytes."""
+    n = k = 0
+    while nt > 2 and k < nt:
+        k += 2 if (t + k) & 1 and k + 1 < nt and (k + 1) % he else 1
+        n += 1
+    return n
+
+
 def plane_passes(start, steps):
-    """Passes over the planes in timed_boxes_window's runs: a pair of ticks from an
-    odd one on, single ticks elsewhere and before a hash that falls between the two."""
+    """Passes over the planes in timed_boxes_window's runs."""
     n, t = 0, start
     for nt, he in hash_segments(steps):
-        k = 0
-        while k < nt:
-            k += 2 if (t + k) & 1 and k + 1 < nt and (k + 1) % he else 1
-            n += 1
+        n += run_passes(t, nt, he)
         t += nt
     return n
 
 
 def plane_bytes(vox, start, steps):
-    """Bytes of those passes, of the hashes and of the runs' write-back as bytes."""
-    segs = hash_segments(steps)
-    hashes = sum(nt // he for nt, he in segs)
-    return vox * (0.5 * plane_passes(start, steps) + 0.25 * hashes + 1.25 * len(segs))
+    """Bytes of those passes, of the hashes, of the runs' write-back as bytes, of packing
+    a grid that is not in planes (an even first tick is part of it) and of ticks on bytes."""
+    total, planes, t = 0.0, start > 2, start
+    for nt, he in hash_segments(steps):
+        if nt > 2:
+            total += 0.5 * run_passes(t, nt, he) + 0.25 * (nt // he) + 1.25
+            if not planes:
+                total += 1.25 - (0.0 if t & 1 else 0.5)
+        else:
+            total += 2.0 * nt
+        planes = nt > 2
+        t += nt
+    return vox * total
 
 
 def bench_boxes512(F, steps, warmup, kernel_ticks=200):
@@ -794,6 +811,7 @@ def main():
         hbm = {"bound": "hbm", "achieved": round(ach2 / 1e9, 1), "peak": HBM_PEAK / 1e9, "unit": "GB/s",
                "frac": round(frac2, 4), "traffic": None,
                "kernel": DENSE2048_LABEL,
+               "note": "with fuse off; dense ticks run in pairs on planes by default (extra.pillars2048.fused_pairs)",
                "kernel_ms": round(p["dense"]["kern_ms"], 5), "alg_bytes_per_tick": 2 * p["vox"],
                "frac_of_copy": round(ach2 / 1e9 / c["GBps"], 4),
                "frac_of_streaming_copy": round(ach2 / 1e9 / c["streaming"]["GBps"], 4)}
